@@ -446,6 +446,7 @@ struct FusedArgs {
     int N0, L0;
     int p0;                // first problem of the chunk
     int c0, ccount;        // coil range of this launch
+    int gcoils;            // coils per workgroup of the forward plane kernels (group blockIdx.z)
     int accumulate;        // out += (later coil chunks)
     int coil_pstride;      // problem p uses coil-map rows coils[i] + p * coil_pstride
     const int* pcoils;     // optional [P] device: problem p uses its first pcoils[p] coils
@@ -460,6 +461,14 @@ __device__ __forceinline__ int coil_count(const FusedArgs& a, int p)
     if (!a.pcoils) return a.ccount;
     const int n = a.pcoils[p] - a.c0;
     return n < 0 ? 0 : (n < a.ccount ? n : a.ccount);
+}
+
+// The forward plane kernels' share of those coils: group blockIdx.z of gcoils coils.
+__device__ __forceinline__ int group_begin(const FusedArgs& a) { return (int)blockIdx.z * a.gcoils; }
+__device__ __forceinline__ int group_end(const FusedArgs& a, int ncl)
+{
+    const int e = group_begin(a) + a.gcoils;
+    return e < ncl ? e : ncl;
 }
 
 template <int NB> __global__ void __launch_bounds__(kXY) fwd_xy_kernel(FusedArgs a)
@@ -483,8 +492,8 @@ template <int NB> __global__ void __launch_bounds__(kXY) fwd_xy_kernel(FusedArgs
     const float2* xp = a.x + ((int64_t)p * a.N0 + z) * plane;
     lds_barrier();
 
-    const int ncl = coil_count(a, a.p0 + pl);
-    for (int ci = 0; ci < ncl; ++ci) {
+    const int cend = group_end(a, coil_count(a, a.p0 + pl));
+    for (int ci = group_begin(a); ci < cend; ++ci) {
         const int coil = a.coils[a.c0 + ci] + p * a.coil_pstride;
         const float2* sp = a.smaps + ((int64_t)coil * a.N0 + z) * plane;
         float2 v[NB][NB];
@@ -875,8 +884,8 @@ template <int NB> __global__ void __launch_bounds__(kXYW) fwd_xy_w_kernel(FusedA
     const LaneTw32 lt = lane_tw32(b, a.tw32);
     lds_barrier();
 
-    const int ncl = coil_count(a, a.p0 + pl);
-    for (int ci = 0; ci < ncl; ++ci) {
+    const int cend = group_end(a, coil_count(a, a.p0 + pl));
+    for (int ci = group_begin(a); ci < cend; ++ci) {
         const int coil = a.coils[a.c0 + ci] + p * a.coil_pstride;
         const auto sr = plane_rsrc(a.smaps + ((int64_t)coil * a.N0 + z) * plane, sizeof(float2) * N * N);
         float2 v[2 * NB][NB];
@@ -962,11 +971,12 @@ inline unsigned inv_w_grid_x(int NB, int N0)
     return inv_row_splits(NB) == 1 ? (unsigned)N0 : (unsigned)(16 * ((N0 + 7) / 8));
 }
 
-template <int NB> __global__ void __launch_bounds__(kXYW) inv_xy_w_kernel(FusedArgs a)
+template <int NB, bool SPLIT> __global__ void __launch_bounds__(kXYW) inv_xy_w_kernel(FusedArgs a)
 {
     constexpr int N = 32 * NB, L = 64 * NB, P = 2 * NB, R2 = 4 * NB, CS = cosets_per_step(NB);
     constexpr int HS = inv_row_splits(NB), KR = 2 * NB / HS;  // row halves; y2 values per thread
     constexpr int CW = L * kW;
+    static_assert(!SPLIT || HS == 1, "a coil image overwrites its T plane, which the row halves share");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     float2* buf = reinterpret_cast<float2*>(smem_raw);  // [CS][16 y1][R2 k1][32 m]
     float2* twL = buf + CS * CW;
@@ -1000,7 +1010,7 @@ template <int NB> __global__ void __launch_bounds__(kXYW) inv_xy_w_kernel(FusedA
     lds_barrier();
 
     const int ncl = coil_count(a, a.p0 + pl);
-    for (int ci = 0; ci < ncl; ++ci) {
+    for (int ci = SPLIT ? (int)blockIdx.z : 0; ci < (SPLIT ? min(ncl, (int)blockIdx.z + 1) : ncl); ++ci) {
         const int coil = a.coils[a.c0 + ci] + p * a.coil_pstride;
         const auto sr = plane_rsrc(a.smaps + ((int64_t)coil * a.N0 + z) * plane, sizeof(float2) * N * N);
         // this coil's image, summed over the cosets; times conj(S) once at the end
@@ -1059,6 +1069,14 @@ template <int NB> __global__ void __launch_bounds__(kXYW) inv_xy_w_kernel(FusedA
             }
             lds_barrier();
         }
+        if constexpr (SPLIT) {
+            // every wave is past its T loads (they fed the LDS blocks of the last barriers)
+#pragma unroll
+            for (int k = 0; k < KR; ++k)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) bstore(tr, ic[k][j], xoff, (uint32_t)(16 * k * N + 32 * j) * 8u);
+            continue;
+        }
 #pragma unroll
         for (int k = 0; k < KR; ++k)
 #pragma unroll
@@ -1066,6 +1084,7 @@ template <int NB> __global__ void __launch_bounds__(kXYW) inv_xy_w_kernel(FusedA
                 acc[k][j] = cfma_conj(acc[k][j], bload<true>(sr, xoff, (uint32_t)(16 * (y0 + k) * N + 32 * j) * 8u),
                                       ic[k][j]);
     }
+    if constexpr (SPLIT) return;
     const auto orr = plane_rsrc(a.out + ((int64_t)p * a.N0 + z) * plane, sizeof(float2) * N * N);
     const auto sbr = plane_rsrc(a.sub ? a.sub + ((int64_t)p * a.N0 + z) * plane : a.out, sizeof(float2) * N * N);
 #pragma unroll
@@ -1291,7 +1310,7 @@ __global__ void __launch_bounds__(kQT) fwd_xy_r16_kernel(FusedArgs a)
     const uint32_t toff = (uint32_t)t * 8u;
     phase_barrier();
 
-    const int ncl = coil_count(a, p);
+    const int cbeg = group_begin(a), cend = group_end(a, coil_count(a, p));
     auto smap_rsrc = [&](int ci) {
         const int coil = a.coils[a.c0 + ci] + p * a.coil_pstride;
         return plane_rsrc(a.smaps + ((int64_t)coil * a.N0 + z) * plane, sizeof(float2) * N * N);
@@ -1307,8 +1326,8 @@ __global__ void __launch_bounds__(kQT) fwd_xy_r16_kernel(FusedArgs a)
             ns[x2] = bload<true>(sr, xoff, so);
         }
     };
-    if (ncl > 0) load_row(smap_rsrc(0), 0);
-    for (int ci = 0; ci < ncl; ++ci) {
+    if (cbeg < cend) load_row(smap_rsrc(cbeg), 0);
+    for (int ci = cbeg; ci < cend; ++ci) {
         const auto sr = smap_rsrc(ci);
         const auto tr = plane_rsrc(a.T + (((int64_t)pl * a.ccount + ci) * a.N0 + z) * (int64_t)L * L,
                                    sizeof(float2) * L * L);
@@ -1351,7 +1370,7 @@ __global__ void __launch_bounds__(kQT) fwd_xy_r16_kernel(FusedArgs a)
                 __builtin_amdgcn_sched_barrier(0);
             }
             phase_barrier();
-            if (h == 3 && ci + 1 < ncl) load_row(smap_rsrc(ci + 1), 0);
+            if (h == 3 && ci + 1 < cend) load_row(smap_rsrc(ci + 1), 0);
             {
                 const int col = t & 63, ka = t >> 6;
                 float2 u[32];
@@ -1366,7 +1385,7 @@ __global__ void __launch_bounds__(kQT) fwd_xy_r16_kernel(FusedArgs a)
     }
 }
 
-__global__ void __launch_bounds__(kQT) inv_xy_r16_kernel(FusedArgs a)
+template <bool SPLIT> __global__ void __launch_bounds__(kQT) inv_xy_r16_kernel(FusedArgs a)
 {
     constexpr int N = 128, L = 256;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1394,7 +1413,7 @@ __global__ void __launch_bounds__(kQT) inv_xy_r16_kernel(FusedArgs a)
     const uint32_t xoff = (uint32_t)(g * N + q) * 8u;
     const uint32_t toff = (uint32_t)t * 8u;
     const int ncl = coil_count(a, p);
-    for (int ci = 0; ci < ncl; ++ci) {
+    for (int ci = SPLIT ? (int)blockIdx.z : 0; ci < (SPLIT ? min(ncl, (int)blockIdx.z + 1) : ncl); ++ci) {
         const int coil = a.coils[a.c0 + ci] + p * a.coil_pstride;
         const auto sr = plane_rsrc(a.smaps + ((int64_t)coil * a.N0 + z) * plane, sizeof(float2) * N * N);
         const auto tr = plane_rsrc(a.T + (((int64_t)pl * a.ccount + ci) * a.N0 + z) * (int64_t)L * L,
@@ -1434,7 +1453,7 @@ __global__ void __launch_bounds__(kQT) inv_xy_r16_kernel(FusedArgs a)
                 }
             }
             phase_barrier();
-            if (h == 3) load_srow(sv, 0);
+            if (!SPLIT && h == 3) load_srow(sv, 0);
             // twiddle w256^{-g ka}, inverse DFT over ka -> i, rows i < 4 kept
             const float sg = g < 16 ? 1.f : -1.f;
             const int gp = g & 15;
@@ -1472,14 +1491,21 @@ __global__ void __launch_bounds__(kQT) inv_xy_r16_kernel(FusedArgs a)
 #pragma unroll
             for (int k1 = 1; k1 < 16; ++k1) u[k1] = cmulc(tq[qo + k1], yb[xo + qo + k1]);
             dft16<1>(u);
+            if constexpr (SPLIT) {
+                // every wave is past its T loads (they fed the LDS exchange of the last barriers)
 #pragma unroll
-            for (int x2 = 0; x2 < 8; ++x2) acc[i][x2] = cfma_conj(acc[i][x2], sv[x2], u[x2]);
-            // the next row's maps load during that row's transforms
-            if (i < 3) load_srow(sv, i + 1);
+                for (int x2 = 0; x2 < 8; ++x2) bstore(tr, u[x2], xoff, (uint32_t)(i * 32 * N + 16 * x2) * 8u);
+            } else {
+#pragma unroll
+                for (int x2 = 0; x2 < 8; ++x2) acc[i][x2] = cfma_conj(acc[i][x2], sv[x2], u[x2]);
+                // the next row's maps load during that row's transforms
+                if (i < 3) load_srow(sv, i + 1);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
         phase_barrier();
     }
+    if constexpr (SPLIT) return;
     float2* op = a.out + ((int64_t)p * a.N0 + z) * plane;
     const float2* sb = a.sub ? a.sub + ((int64_t)p * a.N0 + z) * plane : nullptr;
 #pragma unroll
@@ -1492,6 +1518,35 @@ __global__ void __launch_bounds__(kQT) inv_xy_r16_kernel(FusedArgs a)
             else if (sb) rr = csub(rr, sb[idx]);
             op[idx] = rr;
         }
+}
+
+// Coil sum of the split inverse plane kernels: each coil's image lies in the first N1 N2
+// elements of its T planes. The same multiply-adds in the same coil order as the unsplit
+// kernels, so a problem's result does not depend on how its launch was split. The split
+// writes and re-reads every coil image (16 N^3 bytes per coil next to the 96 N^3 of the
+// grid), so it serves launches whose (z-plane, problem) pairs leave the GPU idle: one 64^3
+// x 8 coil problem (64 pairs) went 85 -> 20 + 7.5 us (inverse, sum; forward 73 -> 21 us).
+__global__ void __launch_bounds__(256) coil_sum_kernel(FusedArgs a, int plane, int LL)
+{
+    const int pl = blockIdx.y;
+    const int p = a.p0 + pl;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.N0 * plane) return;
+    const int z = i / plane;
+    const float2* ic = a.T + ((int64_t)pl * a.ccount * a.N0 + z) * LL + (i - z * plane);
+    const int64_t cstep = (int64_t)a.N0 * LL;
+    const int64_t vox = (int64_t)a.N0 * plane;
+    const int ncl = coil_count(a, p);
+    float2 acc = float2{0.f, 0.f};
+#pragma unroll 4
+    for (int ci = 0; ci < ncl; ++ci) {
+        const int coil = a.coils[a.c0 + ci] + p * a.coil_pstride;
+        acc = cfma_conj(acc, a.smaps[coil * vox + i], ic[ci * cstep]);
+    }
+    const int64_t o = (int64_t)p * vox + i;
+    if (a.accumulate) acc = cadd(acc, a.out[o]);
+    else if (a.sub) acc = csub(acc, a.sub[o]);
+    a.out[o] = acc;
 }
 
 // z-axis pass for L0 = 256 (N0 = 128) as a 16 x 16 four-step FFT with the data in
@@ -1808,6 +1863,20 @@ size_t sense_fused_workspace_bytes(const int64_t* n3, int pchunk, int ccount)
     return sizeof(float2) * (size_t)pchunk * ccount * n3[0] * L * L;
 }
 
+// Coil groups of a forward plane launch of `wgs` (z-plane, problem) pairs: one workgroup
+// per pair and group, so the fewest groups (a power of two, at most the coils) whose last
+// round over the GPU's `slots` is at least 90 % full (a group re-reads the image plane and
+// loses the prefetch across its border). Together with the split inverse: 32^3 x 8 coils
+// 84 -> 49 us per apply, a 64^3 x 8 CG of 10 iterations 2.38 -> 1.26 ms, 160^3 x 20 coils x
+// 2 problems (320 pairs, 1.25 rounds) 8.06 -> 7.56 ms.
+static int coil_groups(int64_t wgs, int coils, int64_t slots)
+{
+    int g = 1;
+    for (; 2 * g <= coils; g *= 2)
+        if (wgs * g * 10 >= 9 * slots * ceil_div(wgs * g, slots)) break;
+    return g;
+}
+
 // kernels: permuted layout (sense_fused_permute_kernel with r16); kidx: host int [P].
 void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const int* coils_dev, int ncoil,
                        const float* kernels, bool r16, const int* kidx, const float2* sub, int P, const int64_t* n3,
@@ -1850,6 +1919,7 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
     if (zct) allow_lds(zct, smem_zct);
     auto fwd = NB == 1 ? fwd_xy_kernel<1> : NB == 2 ? fwd_xy_kernel<2> : NB == 3 ? fwd_xy_kernel<3> : fwd_xy_kernel<4>;
     auto inv = NB == 1 ? inv_xy_kernel<1> : NB == 2 ? inv_xy_kernel<2> : NB == 3 ? inv_xy_kernel<3> : inv_xy_kernel<4>;
+    decltype(inv) inv_split = nullptr;  // one coil per workgroup; null where there is none
     int nxy = kXY;
     const int variant = g_xy_variant.load();
     // at N = 160 only the coset kernels (one coset per step) fit in LDS
@@ -1859,26 +1929,37 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
               : NB == 3 ? fwd_xy_w_kernel<3>
               : NB == 4 ? fwd_xy_w_kernel<4>
                         : fwd_xy_w_kernel<5>;
-        inv = NB == 1   ? inv_xy_w_kernel<1>
-              : NB == 2 ? inv_xy_w_kernel<2>
-              : NB == 3 ? inv_xy_w_kernel<3>
-              : NB == 4 ? inv_xy_w_kernel<4>
-                        : inv_xy_w_kernel<5>;
+        inv = NB == 1   ? inv_xy_w_kernel<1, false>
+              : NB == 2 ? inv_xy_w_kernel<2, false>
+              : NB == 3 ? inv_xy_w_kernel<3, false>
+              : NB == 4 ? inv_xy_w_kernel<4, false>
+                        : inv_xy_w_kernel<5, false>;
+        inv_split = NB == 1   ? inv_xy_w_kernel<1, true>
+                    : NB == 2 ? inv_xy_w_kernel<2, true>
+                    : NB == 3 ? inv_xy_w_kernel<3, true>
+                    : NB == 4 ? inv_xy_w_kernel<4, true>
+                              : nullptr;
         nxy = kXYW;
         smem_xy = coset_kernel_lds(NB);
     }
-    if (variant == 3 && NB <= 4)  // stage + transform buffers: the LDS of two coset blocks
+    if (variant == 3 && NB <= 4) {  // stage + transform buffers: the LDS of two coset blocks
+        inv_split = nullptr;
         inv = NB == 1 ? inv_xy_d_kernel<1> : NB == 2 ? inv_xy_d_kernel<2> : NB == 3 ? inv_xy_d_kernel<3> : inv_xy_d_kernel<4>;
+    }
     HASTY_REQUIRE(!r16 || N == 128, "the register-kernel layout needs N1 = N2 = 128");
     if (r16) {
         fwd = fwd_xy_r16_kernel;
-        inv = inv_xy_r16_kernel;
+        inv = inv_xy_r16_kernel<false>;
+        inv_split = inv_xy_r16_kernel<true>;
         nxy = kQT;
         smem_xy = kQLds;
     }
     allow_lds(fwd, smem_xy);
     allow_lds(inv, smem_xy);
+    if (inv_split) allow_lds(inv_split, smem_xy);
     if (!zct && L0 != 256) allow_lds(z_conv_kernel, smem_z);
+    // workgroups of a plane kernel the GPU runs at once: one or two per CU, by LDS
+    const int64_t slots = NB <= 2 ? 512 : 256;
     // at N = 160 (always the coset kernels) the inverse runs two workgroups per z-plane
     const unsigned inv_grid_x = inv_w_grid_x(NB, N0);
     for (int p0 = 0; p0 < P; p0 += pchunk) {
@@ -1889,8 +1970,10 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
             a.ccount = std::min(cchunk, ncoil - c0);
             a.accumulate = c0 > 0 ? 1 : 0;
             {
+                const int groups = coil_groups((int64_t)N0 * np, a.ccount, slots);
+                a.gcoils = (a.ccount + groups - 1) / groups;
                 KernelTimer t("sense_fwd_xy", s);
-                hipLaunchKernelGGL(fwd, dim3(N0, np), dim3(nxy), smem_xy, s, a);
+                hipLaunchKernelGGL(fwd, dim3(N0, np, (a.ccount + a.gcoils - 1) / a.gcoils), dim3(nxy), smem_xy, s, a);
                 check_launch("fwd_xy_kernel");
             }
             const int zvar = g_zconv_variant.load();
@@ -1928,6 +2011,18 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
                                        K);
                 }
                 check_launch("z_conv_kernel");
+            }
+            if (inv_split && a.ccount > 1 && (int64_t)N0 * np < slots) {
+                {
+                    KernelTimer t("sense_inv_xy", s);
+                    hipLaunchKernelGGL(inv_split, dim3(N0, np, a.ccount), dim3(nxy), smem_xy, s, a);
+                    check_launch("inv_xy_kernel");
+                }
+                KernelTimer t("sense_coil_sum", s);
+                hipLaunchKernelGGL(coil_sum_kernel, dim3((unsigned)ceil_div((int64_t)N0 * N * N, 256), np), dim3(256), 0, s,
+                                   a, N * N, L * L);
+                check_launch("coil_sum_kernel");
+                continue;
             }
             KernelTimer t("sense_inv_xy", s);
             hipLaunchKernelGGL(inv, dim3(inv_grid_x, np), dim3(nxy), smem_xy, s, a);

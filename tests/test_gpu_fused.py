@@ -196,3 +196,35 @@ def test_zconv_variants_vs_oracle(N, variant, N0):
         e = O.rel_l2(out[p:p + 1], O.sense_normal_toeplitz(diags[kidx[p]], x[p:p + 1], S, [0, 1, 2]))
         print(f"z-conv variant {variant} problem {p}: {e:.2e}", flush=True)
         assert e < 1e-5
+
+
+@pytest.mark.parametrize("n", [32, 64, 96, 128])
+@pytest.mark.parametrize("coil_batch", [2, 5])
+def test_split_launches_equal_whole_launches(N, n, coil_batch):
+    """A few problems split the plane kernels by coils (coil images, then a coil sum), many
+    do not; a problem's result is the same to the bit either way, with coil chunks that
+    accumulate, uneven coil counts and a subtracted term."""
+    C, P = 5, {32: 16, 64: 8, 96: 3, 128: 2}[n]  # P problems fill the GPU, one does not
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(n + coil_batch)
+    smaps = torch.randn((C, n, n, n), dtype=torch.complex64, device="cuda:0", generator=gen)
+    kern = torch.rand((2 * n, 2 * n, 2 * n), dtype=torch.float32, device="cuda:0", generator=gen)
+    x = torch.randn((P, n, n, n), dtype=torch.complex64, device="cuda:0", generator=gen)
+    sub = torch.randn((P, n, n, n), dtype=torch.complex64, device="cuda:0", generator=gen)
+    op = N.SenseNormalToeplitz(smaps, kern, coil_batch=coil_batch, problem_batch=P)
+    counts = [C - p % 4 for p in range(P)]
+    whole = op.apply(x, sub=sub)
+    uneven = op.apply(x, sub=sub, problem_ncoil=counts)
+    for p in (0, 1, P - 1):
+        xp, sp = x[p:p + 1].contiguous(), sub[p:p + 1].contiguous()
+        assert torch.equal(op.apply(xp, sub=sp)[0], whole[p])
+        assert torch.equal(op.apply(xp, sub=sp, problem_ncoil=counts[p:p + 1])[0], uneven[p])
+    # the split result against the same convolution in FP64
+    ref = torch.zeros((n, n, n), dtype=torch.complex128, device="cuda:0")
+    kd = kern.double()
+    for s in smaps.to(torch.complex128):
+        y = torch.fft.ifftn(torch.fft.fftn(s * x[0], s=[2 * n] * 3) * kd) * float((2 * n) ** 3)
+        ref += s.conj() * y[:n, :n, :n]
+    ref -= sub[0]
+    err = float(torch.linalg.vector_norm(whole[0] - ref) / torch.linalg.vector_norm(ref))
+    assert err < 1e-6, err

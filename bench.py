@@ -60,7 +60,7 @@ def parse():
     ap.add_argument("--xy-variant", type=int, default=None,
                     help="plane kernels of the fused path (library option sense_xy_variant)")
     ap.add_argument("--zconv-variant", type=int, default=None,
-                    help="z-convolution kernel at N0 = 128 (library option sense_zconv_variant, 0..3)")
+                    help="z-convolution bundles at N0 = 128 and 160 (library option sense_zconv_variant, 0..3)")
     ap.add_argument("--zconv-batch", type=int, default=None,
                     help="problems per z-convolution launch at N0 = 128 (library option sense_zconv_batch, 1..16)")
     ap.add_argument("--cg-iters", type=int, default=15)

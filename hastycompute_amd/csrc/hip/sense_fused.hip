@@ -14,7 +14,7 @@
 //              after the twiddle exp(-2 pi i s n / L) (one wavefront shuffle FFT per
 //              row), followed by the L-point y FFT of the 32 columns in LDS. Writes
 //              T[p][c][z][s][ky][m] (N0 planes of L*L, i.e. half the oversampled grid).
-//  B  z_conv   one workgroup per bundle of 32 (ky, kx) columns: loads the kernel
+//  B  z_conv   one workgroup per bundle of 8 to 32 (ky, kx) columns: loads the kernel
 //              column bundle once, then for each coil: z FFT (N0 -> L0 padded), times
 //              the real kernel, inverse z FFT, crop to N0, in place in T.
 //  C  inv_xy   one workgroup per (problem, z-plane): for each coil and coset, the
@@ -363,47 +363,6 @@ __device__ __forceinline__ void col_pass_ct(const float2* __restrict__ src, floa
     }
 }
 
-// Same pass in place: every thread first gathers all its butterflies into registers,
-// the workgroup synchronises, then the results are written back (one LDS buffer).
-template <int RAD, int S, int NCOL, int NT, int L, int NS>
-__device__ __forceinline__ void col_pass_ip(float2* __restrict__ buf, const float2* __restrict__ twL, int zero_from)
-{
-    constexpr int nbf = L / RAD;
-    constexpr int twstep = L / (NS * RAD);
-    constexpr int total = nbf * NCOL;
-    constexpr int BPT = (total + NT - 1) / NT;
-    float2 v[BPT][RAD];
-#pragma unroll
-    for (int q = 0; q < BPT; ++q) {
-        const int bf = threadIdx.x + q * NT;
-        if (total % NT != 0 && bf >= total) break;
-        const int c = bf % NCOL;
-        const int j = bf / NCOL;
-        const int k = j % NS;
-#pragma unroll
-        for (int r = 0; r < RAD; ++r) {
-            const int row = j + r * nbf;
-            float2 x = row < zero_from ? buf[row * NCOL + c] : float2{0.f, 0.f};
-            if (r > 0 && NS > 1) x = cmul(x, twid<S>(twL, r * k * twstep));
-            v[q][r] = x;
-        }
-        dftR<RAD, S>(v[q]);
-    }
-    lds_barrier();
-#pragma unroll
-    for (int q = 0; q < BPT; ++q) {
-        const int bf = threadIdx.x + q * NT;
-        if (total % NT != 0 && bf >= total) break;
-        const int c = bf % NCOL;
-        const int j = bf / NCOL;
-        const int k = j % NS;
-        const int o = (j / NS) * NS * RAD + k;
-#pragma unroll
-        for (int r = 0; r < RAD; ++r) buf[(o + r * NS) * NCOL + c] = v[q][r];
-    }
-    lds_barrier();
-}
-
 // L = 64 * NB as radix 8 x 8 (x NB): ping-pong form, returns the result buffer.
 template <int S, int NCOL, int NT, int NB>
 __device__ __forceinline__ float2* col_fft_ct(float2* a, float2* b, const float2* twL, int zero_from)
@@ -420,16 +379,6 @@ __device__ __forceinline__ float2* col_fft_ct(float2* a, float2* b, const float2
         lds_barrier();
         return b;
     }
-}
-
-// In-place form (result in buf).
-template <int S, int NCOL, int NT, int NB>
-__device__ __forceinline__ void col_fft_ip(float2* buf, const float2* twL, int zero_from)
-{
-    constexpr int L = 64 * NB;
-    col_pass_ip<8, S, NCOL, NT, L, 1>(buf, twL, zero_from);
-    col_pass_ip<8, S, NCOL, NT, L, 8>(buf, twL, L);
-    if constexpr (NB > 1) col_pass_ip<NB, S, NCOL, NT, L, 64>(buf, twL, L);
 }
 
 struct FusedArgs {
@@ -640,76 +589,6 @@ __global__ void __launch_bounds__(kZ) z_conv_kernel(FusedArgs a, int LL, int pl,
     }
 }
 
-// z-axis pass for L0 = 64 * NB0: 16-column bundles, 512 threads, one in-place LDS buffer
-// (L0 * 16 complex), so several workgroups share a CU and overlap loads with FFT work.
-constexpr int kZC = 16;
-constexpr int kZT = 512;
-
-template <int NB0>
-__global__ void __launch_bounds__(kZT) z_conv_ct_kernel(FusedArgs a, int LL, int pl, const float* __restrict__ K)
-{
-    constexpr int L0 = 64 * NB0;
-    constexpr int N0 = L0 / 2;
-    constexpr int NEL = L0 * kZC;
-    constexpr int PER = (NEL + kZT - 1) / kZT;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    float2* buf = reinterpret_cast<float2*>(smem_raw);
-    float2* twz = buf + NEL;
-    const int t = threadIdx.x;
-    const int pos0 = blockIdx.x * kZC;
-    for (int i = t; i < L0; i += kZT) twz[i] = a.twL0[i];
-    float kv[PER];
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int e = t + kZT * i;
-        kv[i] = e < NEL ? K[(int64_t)(e / kZC) * LL + pos0 + (e % kZC)] : 0.f;
-    }
-    lds_barrier();
-    // the next coil's bundle is prefetched into registers during the current transform
-    constexpr int PFZ = (N0 * kZC + kZT - 1) / kZT;
-    float2 pf[PFZ];
-    {
-        const float2* T0 = a.T + (int64_t)pl * a.ccount * N0 * (int64_t)LL + pos0;
-#pragma unroll
-        for (int i = 0; i < PFZ; ++i) {
-            const int e = t + kZT * i;
-            if (e < N0 * kZC) pf[i] = T0[(int64_t)(e / kZC) * LL + (e % kZC)];
-        }
-    }
-    const int ncl = coil_count(a, a.p0 + pl);
-    for (int ci = 0; ci < ncl; ++ci) {
-        float2* Tc = a.T + ((int64_t)pl * a.ccount + ci) * N0 * (int64_t)LL + pos0;
-#pragma unroll
-        for (int i = 0; i < PFZ; ++i) {
-            const int e = t + kZT * i;
-            if (e < N0 * kZC) buf[e] = pf[i];
-        }
-        lds_barrier();
-        if (ci + 1 < ncl) {
-            const float2* Tn = Tc + (int64_t)N0 * LL;
-#pragma unroll
-            for (int i = 0; i < PFZ; ++i) {
-                const int e = t + kZT * i;
-                if (e < N0 * kZC) pf[i] = Tn[(int64_t)(e / kZC) * LL + (e % kZC)];
-            }
-        }
-        col_fft_ip<-1, kZC, kZT, NB0>(buf, twz, N0);
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int e = t + kZT * i;
-            if (e < NEL) buf[e] = cscale(buf[e], kv[i]);
-        }
-        lds_barrier();
-        col_fft_ip<1, kZC, kZT, NB0>(buf, twz, L0);
-#pragma unroll
-        for (int i = 0; i < (N0 * kZC + kZT - 1) / kZT; ++i) {
-            const int e = t + kZT * i;
-            if (e < N0 * kZC) Tc[(int64_t)(e / kZC) * LL + (e % kZC)] = buf[e];
-        }
-        lds_barrier();
-    }
-}
-
 // 16-point DFT in registers: n = 4a + b, k = c + 4d,
 // X[c + 4d] = sum_b w16^{bc} w4^{bd} sum_a v[4a + b] w4^{ac}.
 template <int S, bool HALF = false> __device__ __forceinline__ void dft16(float2* v)
@@ -800,18 +679,17 @@ template <int S, bool HALF = false> __device__ __forceinline__ void dft20_dr(flo
 }
 
 // Register DFTs of length R: natural order for R in {4, 8, 12, 16}; for R = 20 the
-// in-place form above, with output k in slot dft_slot<R>(k). With HALF (R = 20 only)
-// the upper half of the inputs is zero and is not read.
+// in-place form above, with output k in slot dft_slot<R>(k). With HALF the upper half of
+// the inputs is zero (and not read for R = 8, 16, 20).
 template <int R> __host__ __device__ constexpr int dft_slot(int k) { return R == 20 ? 5 * (k % 4) + k / 4 : k; }
 
 template <int R, int S, bool HALF = false> __device__ __forceinline__ void dftn(float2* v)
 {
     static_assert(R == 4 || R == 8 || R == 12 || R == 16 || R == 20, "unsupported register DFT length");
-    static_assert(!HALF || R == 20, "HALF is implemented for R = 20");
     if constexpr (R == 4) dft4<S>(v);
-    else if constexpr (R == 8) dft8<S>(v);
+    else if constexpr (R == 8) dft8<S, HALF>(v);
     else if constexpr (R == 12) dft12<S>(v);
-    else if constexpr (R == 16) dft16<S>(v);
+    else if constexpr (R == 16) dft16<S, HALF>(v);
     else dft20_dr<S, HALF>(v);
 }
 
@@ -1549,16 +1427,40 @@ __global__ void __launch_bounds__(256) coil_sum_kernel(FusedArgs a, int plane, i
     a.out[o] = acc;
 }
 
-// z-axis pass for L0 = 256 (N0 = 128) as a 16 x 16 four-step FFT with the data in
-// registers: each thread owns one (column, group) pair of a COLS-column bundle, does
-// 16-point DFTs in registers and meets the others through one LDS transpose per
-// direction; loads and stores go straight between HBM and registers. DB: two transpose
-// buffers (forward and inverse), so a coil needs two workgroup barriers instead of four.
-template <int COLS> struct ZConvShape {
-    static constexpr int T = 16 * COLS;                  // threads
-    static constexpr int S1 = COLS + 1;                  // LDS stride of the inner index (padded)
-    static constexpr int S2 = COLS == 16 ? 280 : 152;    // LDS stride of the outer index (padded)
-    static constexpr size_t lds_bytes(bool db) { return sizeof(float2) * (db ? 2 : 1) * 16 * S2; }
+// Coil groups of a forward plane launch of `wgs` (z-plane, problem) pairs: one workgroup
+// per pair and group, so the fewest groups (a power of two, at most the coils) whose last
+// round over the GPU's `slots` is at least 90 % full (a group re-reads the image plane and
+// loses the prefetch across its border). Together with the split inverse: 32^3 x 8 coils
+// 84 -> 49 us per apply, a 64^3 x 8 CG of 10 iterations 2.38 -> 1.26 ms, 160^3 x 20 coils x
+// 2 problems (320 pairs, 1.25 rounds) 8.06 -> 7.56 ms.
+int coil_groups(int64_t wgs, int coils, int64_t slots)
+{
+    int g = 1;
+    for (; 2 * g <= coils; g *= 2)
+        if (wgs * g * 10 >= 9 * slots * ceil_div(wgs * g, slots)) break;
+    return g;
+}
+
+// z-axis pass for L0 = 2 N0 = R1 R2 as a four-step FFT with the data in registers:
+// z = R2 n1 + n2 (n1 < R1 / 2 nonzero) and k = k1 + R1 k2. In steps A and A' (the R1-point
+// DFTs) thread g of a column owns n2 = g, in step B (the R2-point DFTs, the kernel and
+// back) it owns k1 = g; the threads g >= R1 (whole waves) only meet the others at the
+// barriers there. Loads and stores go straight between HBM and registers, the next coil's
+// column loads during the current one's transforms.
+//
+// One LDS buffer and two barriers per coil: element (k1, n2) has one place, step B writes
+// its results where it read its inputs, and step A of the next coil writes where step A'
+// of this one read, each thread its own places. With separate buffers for the two
+// transposes a 320-point workgroup took 89 KB, one per CU: 3.20 ms per 160^3 x 20 coils x
+// 2 problems, 2.34 ms here (5.2 TB/s of grid and kernel traffic). 256-point lines are at
+// the rate of a 1:1 stream either way (2.15 and 2.07 ms at 128^3 x 16 coils x 5).
+template <int R1, int R2, int COLS> struct ZConvShape {
+    static constexpr int T = R2 * COLS;                      // threads
+    // LDS stride of k1 (float2): columns are contiguous, and below 32 columns the next
+    // thread group's rows start that many banks further on
+    static constexpr int SF = R2 * COLS + (COLS < 32 ? (COLS + 32 - (R2 * COLS) % 32) % 32 : 0);
+    static constexpr size_t lds_bytes() { return sizeof(float2) * R1 * SF; }
+    static_assert(R1 <= R2 && (R1 * COLS) % 64 == 0, "one k1 per thread; idle threads of step B fill whole waves");
 };
 
 // Toeplitz kernels of the problems of one launch (problem pl0 + blockIdx.y uses k[blockIdx.y])
@@ -1567,208 +1469,269 @@ struct ZKernels {
     const float* k[kZMaxProblems];
 };
 
-template <int COLS, bool DB>
-__global__ void __launch_bounds__(ZConvShape<COLS>::T) z_conv_r16_kernel(FusedArgs a, int LL, int pl0, ZKernels zk)
+template <int R1, int R2, int COLS>
+__global__ void __launch_bounds__(R2 * COLS) z_conv_reg_kernel(FusedArgs a, int LL, int pl0, ZKernels zk, int gcoils)
 {
-    using Sh = ZConvShape<COLS>;
-    constexpr int S1 = Sh::S1, S2 = Sh::S2;
+    using Sh = ZConvShape<R1, R2, COLS>;
+    constexpr int SF = Sh::SF, L0 = R1 * R2, N0 = L0 / 2, NH = R1 / 2;
     const int pl = pl0 + (int)blockIdx.y;
     const float* __restrict__ K = zk.k[blockIdx.y];
-    extern __shared__ float2 lds_all[];  // ZConvShape<COLS>::lds_bytes(DB)
-    float2* ldsf = lds_all;
-    float2* ldsi = lds_all + (DB ? 16 * S2 : 0);
+    extern __shared__ float2 lds_all[];  // ZConvShape::lds_bytes()
     const int t = threadIdx.x;
     const int c = t % COLS;
     const int g = t / COLS;
     const int pos0 = blockIdx.x * COLS;
-    float2 tw[16];  // w256^{g m}, forward sign
+    float2 tw[R1];  // wL0^{n2 k1} of n2 = g, forward sign
 #pragma unroll
-    for (int m = 0; m < 16; ++m) tw[m] = a.twL0[(g * m) & 255];
-    float kv[16];   // kernel at k = g + 16 k2 of this column
+    for (int k1 = 1; k1 < R1; ++k1) tw[k1] = a.twL0[(g * k1) % L0];
+    const bool active = R1 == R2 || g < R1;
+    float kv[R2];  // kernel at k = g + R1 k2 of this column
 #pragma unroll
-    for (int k2 = 0; k2 < 16; ++k2) kv[k2] = K[(int64_t)(g + 16 * k2) * LL + pos0 + c];
-    // one coil's half grid [128 z][LL] as a buffer: element (z, pos0 + c) of z = 16 n1 + g
-    // at byte voff + n1 * 16 * LL * 8
+    for (int k2 = 0; k2 < R2; ++k2) kv[k2] = active ? K[(int64_t)(g + R1 * k2) * LL + pos0 + c] : 0.f;
+    // one coil's half grid [N0][LL] as a buffer: element (z, pos0 + c) of z = R2 n1 + g
+    // at byte voff + n1 * R2 * LL * 8
     auto grid_rsrc = [&](int ci) {
-        return plane_rsrc(a.T + ((int64_t)pl * a.ccount + ci) * 128 * (int64_t)LL, (uint32_t)(128 * 8 * (int64_t)LL));
+        return plane_rsrc(a.T + ((int64_t)pl * a.ccount + ci) * N0 * (int64_t)LL, (uint32_t)(N0 * 8 * (int64_t)LL));
     };
     const uint32_t voff = (uint32_t)(((int64_t)g * LL + pos0 + c) * 8);
-    const uint32_t zstep = (uint32_t)(16 * 8 * (int64_t)LL);
-    float2 pf[8];
-    {
-        const auto r0 = grid_rsrc(0);
-#pragma unroll
-        for (int n1 = 0; n1 < 8; ++n1) pf[n1] = bload<true>(r0, voff, n1 * zstep);
-    }
-
+    const uint32_t zstep = (uint32_t)(R2 * 8 * (int64_t)LL);
+    float2* const colA = lds_all + g * COLS + c;  // (k1, n2 = g) at colA[k1 * SF]
+    float2* const colB = lds_all + g * SF + c;    // (k1 = g, n2) at colB[n2 * COLS]
     const int ncl = coil_count(a, a.p0 + pl);
-    for (int ci = 0; ci < ncl; ++ci) {
+    const int cbeg = (int)blockIdx.z * gcoils, cend = min(ncl, cbeg + gcoils);
+    float2 pf[NH];
+    if (cbeg < cend) {
+        const auto r0 = grid_rsrc(cbeg);
+#pragma unroll
+        for (int n1 = 0; n1 < NH; ++n1) pf[n1] = bload<true>(r0, voff, n1 * zstep);
+    }
+    for (int ci = cbeg; ci < cend; ++ci) {
         const auto rc = grid_rsrc(ci);
-        float2 v[16];
+        {
+            float2 v[R1];
 #pragma unroll
-        for (int n1 = 0; n1 < 8; ++n1) v[n1] = pf[n1];
+            for (int n1 = 0; n1 < NH; ++n1) v[n1] = pf[n1];
 #pragma unroll
-        for (int n1 = 8; n1 < 16; ++n1) v[n1] = float2{0.f, 0.f};
-        if (ci + 1 < ncl) {
-            const auto rn = grid_rsrc(ci + 1);
+            for (int n1 = NH; n1 < R1; ++n1) v[n1] = float2{0.f, 0.f};
+            if (ci + 1 < cend) {
+                const auto rn = grid_rsrc(ci + 1);
 #pragma unroll
-            for (int n1 = 0; n1 < 8; ++n1) pf[n1] = bload<true>(rn, voff, n1 * zstep);
+                for (int n1 = 0; n1 < NH; ++n1) pf[n1] = bload<true>(rn, voff, n1 * zstep);
+            }
+            // step A: DFT over n1, twiddle, (k1, n2 = g) to LDS
+            dftn<R1, -1, true>(v);
+            colA[0] = v[0];
+#pragma unroll
+            for (int k1 = 1; k1 < R1; ++k1) colA[k1 * SF] = cmul(v[k1], tw[k1]);
         }
-        // forward, step A (n2 = g): DFT over n1 (n1 < 8 nonzero), twiddle w256^{g k1}, transpose
-        dft16<-1, true>(v);
-#pragma unroll
-        for (int k1 = 1; k1 < 16; ++k1) v[k1] = cmul(v[k1], tw[k1]);
-#pragma unroll
-        for (int k1 = 0; k1 < 16; ++k1) ldsf[k1 * S2 + g * S1 + c] = v[k1];
         lds_barrier();
-        // forward, step B (k1 = g): DFT over n2 -> X[g + 16 k2]; times the kernel
+        // step B: DFT over n2 -> X[k1 + R1 k2], times the kernel, inverse DFT over k2 -> n2
+        if (active) {
+            float2 v[R2], w[R2];
 #pragma unroll
-        for (int n2 = 0; n2 < 16; ++n2) v[n2] = ldsf[g * S2 + n2 * S1 + c];
-        dft16<-1>(v);
+            for (int n2 = 0; n2 < R2; ++n2) v[n2] = colB[n2 * COLS];
+            dftn<R2, -1>(v);
 #pragma unroll
-        for (int k2 = 0; k2 < 16; ++k2) v[k2] = cscale(v[k2], kv[k2]);
-        // inverse, step B' (k1 = g): IDFT over k2 -> n1, twiddle w256^{-g n1}
-        dft16<1>(v);
+            for (int k2 = 0; k2 < R2; ++k2) w[k2] = cscale(v[dft_slot<R2>(k2)], kv[k2]);
+            dftn<R2, 1>(w);
 #pragma unroll
-        for (int n1 = 1; n1 < 16; ++n1) v[n1] = cmulc(tw[n1], v[n1]);
-        // one buffer: all step-B reads are done before the transpose is overwritten.
-        // Two buffers: the next coil's forward writes come after this coil's second
-        // barrier, which every thread passes only after its step-B reads, and the next
-        // inverse writes after the next first barrier, past this coil's step-A' reads.
-        if (!DB) lds_barrier();
-#pragma unroll
-        for (int n1 = 0; n1 < 16; ++n1) ldsi[n1 * S2 + g * S1 + c] = v[n1];
+            for (int n2 = 0; n2 < R2; ++n2) colB[n2 * COLS] = w[dft_slot<R2>(n2)];
+        }
         lds_barrier();
-        // inverse, step A' (n1 = g): IDFT over k1 -> out[g + 16 n2], keep rows < 128
+        // step A': twiddle, inverse DFT over k1 -> out[R2 n1 + g], n1 < R1 / 2 kept
+        float2 v[R1];
+        v[0] = colA[0];
 #pragma unroll
-        for (int k1 = 0; k1 < 16; ++k1) v[k1] = ldsi[g * S2 + k1 * S1 + c];
-        dft16<1>(v);
+        for (int k1 = 1; k1 < R1; ++k1) v[k1] = cmul(colA[k1 * SF], float2{tw[k1].x, -tw[k1].y});
+        dftn<R1, 1>(v);
 #pragma unroll
-        for (int n2 = 0; n2 < 8; ++n2) bstore<true>(rc, v[n2], voff, n2 * zstep);
-        if (!DB) lds_barrier();
+        for (int n1 = 0; n1 < NH; ++n1) bstore<true>(rc, v[n1], voff, n1 * zstep);
     }
 }
 
-template <int COLS, bool DB> void launch_zconv(const FusedArgs& a, int LL, int q0, int nq, const ZKernels& zk, hipStream_t s)
+// The value as a store to LDS would leave it: the compiler may not contract the product
+// it comes from into a later sum, nor (volatile: it counts as used) contract differently
+// because nothing reads it.
+__device__ __forceinline__ float2 rounded(float2 v)
 {
-    const size_t smem = ZConvShape<COLS>::lds_bytes(DB);
-    allow_lds(z_conv_r16_kernel<COLS, DB>, smem);
-    hipLaunchKernelGGL((z_conv_r16_kernel<COLS, DB>), dim3((unsigned)(LL / COLS), (unsigned)nq),
-                       dim3(ZConvShape<COLS>::T), smem, s, a, LL, q0, zk);
+    asm volatile("" : "+v"(v.x), "+v"(v.y));
+    return v;
+}
+// x w and x conj(w) with the products that are rounded before the sum spelled out (the
+// compiler picks one of two by the order of the operands' definitions). FIRST: of the
+// imaginary part of x w, x.y w.x is rounded, else x.x w.y.
+template <bool FIRST> __device__ __forceinline__ float2 cmul_fma(float2 x, float2 w)
+{
+    const float re = fmaf(x.x, w.x, -(x.y * w.y));
+    return float2{re, FIRST ? fmaf(x.x, w.y, x.y * w.x) : fmaf(x.y, w.x, x.x * w.y)};
+}
+__device__ __forceinline__ float2 cmul_conj_fma(float2 x, float2 w)
+{
+    return float2{fmaf(x.x, w.x, x.y * w.y), fmaf(x.y, w.x, -(x.x * w.y))};
 }
 
-// z-axis pass for L0 = 320 (N0 = 160) as a 20 x 16 four-step FFT in registers:
-// z = 20 n1 + n2 (n1 < 8 nonzero), k = k1 + 16 k2. 16 columns per workgroup and 20 threads
-// per column (320 threads): in the 16-point steps thread g of a column owns n2 = g, in
-// the 20-point steps (over n2 -> k2 and back) the threads g < 16 own k1 = g and the
-// other four wait at the barrier. One LDS transpose per direction; DB: separate forward
-// and inverse buffers (two barriers per coil instead of four).
-struct ZConv20 {
-    static constexpr int COLS = 16, T = 20 * COLS;
-    static constexpr int S1 = COLS + 1;  // stride of the inner index (padded)
-    static constexpr int SF = 348;       // forward buffer [k1 < 16][n2 < 20 (S1)][c]
-    static constexpr int SI = 280;       // inverse buffer [n2 < 20][k1 < 16 (S1)][c]
-    // transpose buffer(s), then the w320 table
-    static constexpr size_t lds_bytes(bool db)
-    {
-        return sizeof(float2) * ((db ? 16 * SF + 20 * SI : std::max(16 * SF, 20 * SI)) + 320);
-    }
-};
-
-template <bool DB>
-__global__ void __launch_bounds__(ZConv20::T) z_conv_r20_kernel(FusedArgs a, int LL, int pl0, ZKernels zk)
+// The same at L0 = 64 NB (NB = 1, 2) as radix 8 x 8 x NB, 8 threads per column and 8 NB
+// points per thread in every step: z = 8 NB n1 + n2 with thread g at n2 = g (and g + 8) in
+// step A, k = g + 8 m in step B, and z = g + 8 s on the way back; for NB = 2 the even and
+// the odd n2 meet in a radix-2 step in the thread that holds both. Radices, twiddles and
+// roundings are those of LDS Stockham passes of radix 8, 8, NB, so the results equal
+// theirs to the bit. One 64^3 x 8 coil problem (67 MB of grid): 52 us with such passes in
+// LDS (six barriers per transform), 30 us here.
+constexpr int kZ8Cols = 32;
+template <int NB>
+__global__ void __launch_bounds__(8 * kZ8Cols) z_conv_r8_kernel(FusedArgs a, int LL, int pl0, ZKernels zk, int gcoils)
 {
-    constexpr int S1 = ZConv20::S1, SF = ZConv20::SF, SI = ZConv20::SI, COLS = ZConv20::COLS;
+    constexpr int COLS = kZ8Cols, SF = 8 * NB * COLS, N0 = 32 * NB, NL = 4 * NB;
     const int pl = pl0 + (int)blockIdx.y;
     const float* __restrict__ K = zk.k[blockIdx.y];
-    extern __shared__ float2 lds_all[];  // ZConv20::lds_bytes(DB)
-    float2* ldsf = lds_all;
-    float2* ldsi = lds_all + (DB ? 16 * SF : 0);
-    float2* twz = lds_all + (DB ? 16 * SF + 20 * SI : std::max(16 * SF, 20 * SI));  // w320^k, forward sign
+    __shared__ float2 buf[8 * SF];  // (k1, n2) at k1 * SF + n2 * COLS + column
     const int t = threadIdx.x;
     const int c = t % COLS;
-    const int g = t / COLS;  // 0..19
+    const int g = t / COLS;
     const int pos0 = blockIdx.x * COLS;
-    for (int i = t; i < 320; i += ZConv20::T) twz[i] = a.twL0[i];
-    // the 20-point steps: kernel at k = g + 16 k2 of this column
-    float kv[20];
+    float2 tw[8], tw2[8];  // w64^{g r}; w128^{g + 8 m} of the radix-2 step
+    float kv[8 * NB];      // kernel at k = g + 8 m of this column
 #pragma unroll
-    for (int k2 = 0; k2 < 20; ++k2) kv[k2] = g < 16 ? K[(int64_t)(g + 16 * k2) * LL + pos0 + c] : 0.f;
-    // one coil's half grid [160 z][LL]: element (z, pos0 + c) of z = 20 n1 + g at byte
-    // voff + n1 * 20 * LL * 8
+    for (int r = 0; r < 8; ++r) {
+        tw[r] = a.twL0[NB * g * r];
+        if (NB == 2) tw2[r] = a.twL0[g + 8 * r];
+    }
+#pragma unroll
+    for (int m = 0; m < 8 * NB; ++m) kv[m] = K[(int64_t)(g + 8 * m) * LL + pos0 + c];
     auto grid_rsrc = [&](int ci) {
-        return plane_rsrc(a.T + ((int64_t)pl * a.ccount + ci) * 160 * (int64_t)LL, (uint32_t)(160 * 8 * (int64_t)LL));
+        return plane_rsrc(a.T + ((int64_t)pl * a.ccount + ci) * N0 * (int64_t)LL, (uint32_t)(N0 * 8 * (int64_t)LL));
     };
     const uint32_t voff = (uint32_t)(((int64_t)g * LL + pos0 + c) * 8);
-    const uint32_t zstep = (uint32_t)(20 * 8 * (int64_t)LL);
-    float2 pf[8];
-    {
-        const auto r0 = grid_rsrc(0);
-#pragma unroll
-        for (int n1 = 0; n1 < 8; ++n1) pf[n1] = bload<true>(r0, voff, n1 * zstep);
-    }
-
+    const uint32_t z8 = (uint32_t)(8 * 8 * (int64_t)LL);  // eight z-planes further
+    float2* const rowg = buf + g * SF + c;    // (k1 = g, n2) at rowg[n2 * COLS]
+    float2* const colg = buf + g * COLS + c;  // (k1, n2 = g + 8 b) at colg[k1 * SF + 8 b COLS]
     const int ncl = coil_count(a, a.p0 + pl);
-    for (int ci = 0; ci < ncl; ++ci) {
+    const int cbeg = (int)blockIdx.z * gcoils, cend = min(ncl, cbeg + gcoils);
+    float2 pf[NL];  // z = g + 8 i
+    if (cbeg < cend) {
+        const auto r0 = grid_rsrc(cbeg);
+#pragma unroll
+        for (int i = 0; i < NL; ++i) pf[i] = bload<true>(r0, voff, i * z8);
+    }
+    for (int ci = cbeg; ci < cend; ++ci) {
         const auto rc = grid_rsrc(ci);
-        float2 v[20];
+        // step A: 8-point DFTs over n1 (n1 < 4 nonzero), to LDS
+        float2 v[NB][8], w[NB][8];
 #pragma unroll
-        for (int n1 = 0; n1 < 8; ++n1) v[n1] = pf[n1];
-#pragma unroll
-        for (int n1 = 8; n1 < 16; ++n1) v[n1] = float2{0.f, 0.f};
-        if (ci + 1 < ncl) {
+        for (int i = 0; i < NL; ++i) v[i % NB][i / NB] = pf[i];
+        if (ci + 1 < cend) {
             const auto rn = grid_rsrc(ci + 1);
 #pragma unroll
-            for (int n1 = 0; n1 < 8; ++n1) pf[n1] = bload<true>(rn, voff, n1 * zstep);
+            for (int i = 0; i < NL; ++i) pf[i] = bload<true>(rn, voff, i * z8);
         }
-        // forward, step A (n2 = g): DFT over n1 (n1 < 8 nonzero), twiddle w320^{g k1}, transpose
-        dft16<-1, true>(v);
-        if (ci == 0) lds_barrier();  // the twiddle table is written
 #pragma unroll
-        for (int k1 = 1; k1 < 16; ++k1) v[k1] = cmul(v[k1], twz[(g * k1) % 320]);
+        for (int b = 0; b < NB; ++b) {
+            dft8<-1, true>(v[b]);
 #pragma unroll
-        for (int k1 = 0; k1 < 16; ++k1) ldsf[k1 * SF + g * S1 + c] = v[k1];
+            for (int k1 = 0; k1 < 8; ++k1) colg[k1 * SF + 8 * b * COLS] = v[b][k1];
+        }
         lds_barrier();
-        // forward, step B (k1 = g < 16): DFT over n2 -> X[g + 16 k2] (slot order), times
-        // the kernel; inverse, step B': IDFT over k2 -> n2 (slot order). Waves 0-3 hold
-        // g < 16 and wave 4 g >= 16, so the branches are uniform per wave; the barriers
-        // stay outside them.
-        float2 w[20];  // natural order k2 for the inverse
-        if (g < 16) {
+        // step B: twiddles, 8-point DFTs (over the even and the odd n2, then radix 2), the
+        // kernel, and the first 8-point DFTs of the way back
 #pragma unroll
-            for (int n2 = 0; n2 < 20; ++n2) v[n2] = ldsf[g * SF + n2 * S1 + c];
-            dft20_dr<-1>(v);
+        for (int b = 0; b < NB; ++b) {
 #pragma unroll
-            for (int k2 = 0; k2 < 20; ++k2) w[k2] = cscale(v[dft_slot<20>(k2)], kv[k2]);
-            dft20_dr<1>(w);
+            for (int r = 0; r < 8; ++r) {
+                const float2 x = rowg[(NB * r + b) * COLS];
+                v[b][r] = r ? cmul_fma<true>(x, tw[r]) : x;
+            }
+            dft8<-1>(v[b]);
+#pragma unroll
+            for (int m = 0; m < 8; ++m) v[b][m] = rounded(v[b][m]);
         }
-        // one buffer: all step-B reads are done before the transpose is overwritten
-        if (!DB) lds_barrier();
-        if (g < 16) {
-            // twiddle w320^{-g n2}, transpose
 #pragma unroll
-            for (int n2 = 0; n2 < 20; ++n2) {
-                const float2 f = w[dft_slot<20>(n2)];
-                ldsi[n2 * SI + g * S1 + c] = n2 == 0 ? f : cmulc(twz[(g * n2) % 320], f);
+        for (int m = 0; m < 8; ++m) {
+            if constexpr (NB == 1) {
+                w[0][m] = rounded(cscale(v[0][m], kv[m]));
+            } else {
+                const float2 o = cmul_fma<false>(v[1][m], tw2[m]);
+                w[m & 1][m >> 1] = rounded(cscale(rounded(cadd(v[0][m], o)), kv[m]));
+                w[m & 1][(m >> 1) + 4] = rounded(cscale(rounded(csub(v[0][m], o)), kv[m + 8]));
             }
         }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            dft8<1>(w[b]);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) rowg[(r + 8 * b) * COLS] = w[b][r];
+        }
         lds_barrier();
-        // inverse, step A' (n2 = g): IDFT over k1 -> out[20 n1 + g], keep n1 < 8
+        // step A': output g of the DFTs of k mod 8 NB = j (row j mod 8, place g + 8 (j / 8)):
+        // twiddles, 8-point DFTs, radix 2, z = g + 8 s < N0
 #pragma unroll
-        for (int k1 = 0; k1 < 16; ++k1) v[k1] = ldsi[g * SI + k1 * S1 + c];
-        dft16<1>(v);
+        for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int n1 = 0; n1 < 8; ++n1) bstore<true>(rc, v[n1], voff, n1 * zstep);
-        if (!DB) lds_barrier();
+            for (int r = 0; r < 8; ++r) {
+                const int j = NB * r + b;
+                const float2 x = colg[(j % 8) * SF + 8 * (j / 8) * COLS];
+                v[b][r] = r ? cmul_conj_fma(x, tw[r]) : x;
+            }
+            dft8<1>(v[b]);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) v[b][s] = rounded(v[b][s]);
+        }
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            float2 o = v[0][i];
+            if constexpr (NB == 2) o = cadd(o, cmul_conj_fma(v[1][i], tw2[i]));
+            bstore<true>(rc, o, voff, i * z8);
+        }
     }
 }
 
-template <bool DB> void launch_zconv20(const FusedArgs& a, int LL, int q0, int nq, const ZKernels& zk, hipStream_t s)
+// Coils per workgroup of a z-convolution launch of `wgs` (bundle, problem) pairs.
+int zconv_group(const FusedArgs& a, int64_t wgs)
 {
-    const size_t smem = ZConv20::lds_bytes(DB);
-    allow_lds(z_conv_r20_kernel<DB>, smem);
-    hipLaunchKernelGGL((z_conv_r20_kernel<DB>), dim3((unsigned)(LL / ZConv20::COLS), (unsigned)nq),
-                       dim3(ZConv20::T), smem, s, a, LL, q0, zk);
+    const int groups = coil_groups(wgs, a.ccount, 1024);
+    return (a.ccount + groups - 1) / groups;
+}
+
+template <int R1, int R2, int COLS>
+void launch_zconv_reg(const FusedArgs& a, int LL, int q0, int nq, const ZKernels& zk, hipStream_t s)
+{
+    using Sh = ZConvShape<R1, R2, COLS>;
+    // at most three workgroups per CU: more streams in flight ran slower at 256 (2.30 ms
+    // with four, 2.07 ms with two or three, 128^3 x 16 coils x 5 problems)
+    constexpr size_t smem = std::max(Sh::lds_bytes(), (size_t)(Sh::T >= 256 ? 53 * 1024 : 0));
+    allow_lds(z_conv_reg_kernel<R1, R2, COLS>, smem);
+    const int gcoils = zconv_group(a, (int64_t)(LL / COLS) * nq);
+    hipLaunchKernelGGL((z_conv_reg_kernel<R1, R2, COLS>),
+                       dim3((unsigned)(LL / COLS), (unsigned)nq, (unsigned)ceil_div(a.ccount, gcoils)), dim3(Sh::T), smem,
+                       s, a, LL, q0, zk, gcoils);
+}
+
+template <int NB>
+void launch_zconv_r8(const FusedArgs& a, int LL, int q0, int nq, const ZKernels& zk, hipStream_t s)
+{
+    const int gcoils = zconv_group(a, (int64_t)(LL / kZ8Cols) * nq);
+    hipLaunchKernelGGL(z_conv_r8_kernel<NB>,
+                       dim3((unsigned)(LL / kZ8Cols), (unsigned)nq, (unsigned)ceil_div(a.ccount, gcoils)),
+                       dim3(8 * kZ8Cols), 0, s, a, LL, q0, zk, gcoils);
+}
+
+// The z-convolution of problems [q0, q0 + nq) of the chunk at L0 = 64 k <= 320; false for
+// other lengths. `narrow`: 8-column bundles (64-byte row segments) at 256 and 320.
+bool launch_zconv(const FusedArgs& a, int LL, int q0, int nq, const ZKernels& zk, bool narrow, hipStream_t s)
+{
+    switch (a.L0) {
+    case 64: launch_zconv_r8<1>(a, LL, q0, nq, zk, s); return true;
+    case 128: launch_zconv_r8<2>(a, LL, q0, nq, zk, s); return true;
+    case 192: launch_zconv_reg<12, 16, 16>(a, LL, q0, nq, zk, s); return true;
+    case 256:
+        if (narrow) launch_zconv_reg<16, 16, 8>(a, LL, q0, nq, zk, s);
+        else launch_zconv_reg<16, 16, 16>(a, LL, q0, nq, zk, s);
+        return true;
+    case 320:
+        if (narrow) launch_zconv_reg<16, 20, 8>(a, LL, q0, nq, zk, s);
+        else launch_zconv_reg<16, 20, 16>(a, LL, q0, nq, zk, s);
+        return true;
+    default: return false;
+    }
 }
 
 uint32_t radix_code(int L, int* npass)
@@ -1815,10 +1778,8 @@ namespace {
 // variant, so it is set before kernels are prepared.
 std::atomic<int> g_xy_variant{2};
 std::atomic<int> g_zconv_batch{16};  // problems per z-convolution launch (N0 = 128), 1..16
-// z-convolution at N0 = 128: 0 16 columns x 256 threads, one LDS buffer (four barriers
-// per coil); 1 8 columns x 128 threads; 2 (default) 16 columns with two buffers (two
-// barriers per coil); 3 8 columns with two buffers. At 128^3 x 16 coils, 4 problems per
-// launch: 1.85, 3.58, 1.66 and 3.59 ms (8 columns leave 64-byte row segments per wave)
+// z-convolution bundles at N0 = 128 and 160: 0, 2 (default) 16 columns, 1, 3 8 columns
+// (half-used 128-byte lines: 3.6 ms where 16 take 1.66 ms, 128^3 x 16 coils x 4 problems)
 std::atomic<int> g_zconv_variant{2};
 
 bool use_r16(int N) { return g_xy_variant == 2 && N == 128; }
@@ -1831,7 +1792,7 @@ int sense_fused_get_zconv_batch() { return g_zconv_batch; }
 void sense_fused_set_zconv_variant(int v) { g_zconv_variant = v; }
 int sense_fused_get_zconv_variant() { return g_zconv_variant; }
 
-// The z-convolution has register / compact-LDS forms for 2 N0 = 64 k (k <= 5); other
+// The z-convolution has register forms for 2 N0 = 64 k (k <= 5); other
 // lengths use z_conv_kernel, which holds two 32-column blocks of the line in LDS.
 static bool zconv_fits(int64_t L0)
 {
@@ -1861,20 +1822,6 @@ size_t sense_fused_workspace_bytes(const int64_t* n3, int pchunk, int ccount)
 {
     const int64_t L = 2 * n3[1];
     return sizeof(float2) * (size_t)pchunk * ccount * n3[0] * L * L;
-}
-
-// Coil groups of a forward plane launch of `wgs` (z-plane, problem) pairs: one workgroup
-// per pair and group, so the fewest groups (a power of two, at most the coils) whose last
-// round over the GPU's `slots` is at least 90 % full (a group re-reads the image plane and
-// loses the prefetch across its border). Together with the split inverse: 32^3 x 8 coils
-// 84 -> 49 us per apply, a 64^3 x 8 CG of 10 iterations 2.38 -> 1.26 ms, 160^3 x 20 coils x
-// 2 problems (320 pairs, 1.25 rounds) 8.06 -> 7.56 ms.
-static int coil_groups(int64_t wgs, int coils, int64_t slots)
-{
-    int g = 1;
-    for (; 2 * g <= coils; g *= 2)
-        if (wgs * g * 10 >= 9 * slots * ceil_div(wgs * g, slots)) break;
-    return g;
 }
 
 // kernels: permuted layout (sense_fused_permute_kernel with r16); kidx: host int [P].
@@ -1909,14 +1856,6 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
     a.codeL0 = radix_code(L0, &a.npassL0);
     size_t smem_xy = sizeof(float2) * (2 * (size_t)L * kW + L + 32);
     const size_t smem_z = sizeof(float2) * (2 * (size_t)L0 * kW + L0);
-    const size_t smem_zct = sizeof(float2) * ((size_t)L0 * kZC + L0);
-    decltype(&z_conv_ct_kernel<1>) zct = nullptr;
-    if (L0 == 64) zct = z_conv_ct_kernel<1>;
-    else if (L0 == 128) zct = z_conv_ct_kernel<2>;
-    else if (L0 == 192) zct = z_conv_ct_kernel<3>;
-    else if (L0 == 256) zct = z_conv_ct_kernel<4>;
-    else if (L0 == 320) zct = z_conv_ct_kernel<5>;
-    if (zct) allow_lds(zct, smem_zct);
     auto fwd = NB == 1 ? fwd_xy_kernel<1> : NB == 2 ? fwd_xy_kernel<2> : NB == 3 ? fwd_xy_kernel<3> : fwd_xy_kernel<4>;
     auto inv = NB == 1 ? inv_xy_kernel<1> : NB == 2 ? inv_xy_kernel<2> : NB == 3 ? inv_xy_kernel<3> : inv_xy_kernel<4>;
     decltype(inv) inv_split = nullptr;  // one coil per workgroup; null where there is none
@@ -1957,7 +1896,8 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
     allow_lds(fwd, smem_xy);
     allow_lds(inv, smem_xy);
     if (inv_split) allow_lds(inv_split, smem_xy);
-    if (!zct && L0 != 256) allow_lds(z_conv_kernel, smem_z);
+    const bool zreg = L0 % 64 == 0 && L0 <= 320;  // register z-convolution
+    if (!zreg) allow_lds(z_conv_kernel, smem_z);
     // workgroups of a plane kernel the GPU runs at once: one or two per CU, by LDS
     const int64_t slots = NB <= 2 ? 512 : 256;
     // at N = 160 (always the coset kernels) the inverse runs two workgroups per z-plane
@@ -1976,10 +1916,9 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
                 hipLaunchKernelGGL(fwd, dim3(N0, np, (a.ccount + a.gcoils - 1) / a.gcoils), dim3(nxy), smem_xy, s, a);
                 check_launch("fwd_xy_kernel");
             }
-            const int zvar = g_zconv_variant.load();
-            const bool z20 = L0 == 320 && (zvar == 0 || zvar == 2);  // else the LDS Stockham form
-            if (L0 == 256 || z20) {
+            if (zreg) {
                 // one launch per up to g_zconv_batch problems of the chunk
+                const bool narrow = (g_zconv_variant.load() & 1) != 0;
                 const int zbatch = g_zconv_batch.load();
                 for (int q0 = 0; q0 < np; q0 += zbatch) {
                     const int nq = std::min(zbatch, np - q0);
@@ -1987,29 +1926,14 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
                     for (int j = 0; j < nq; ++j)
                         zk.k[j] = kernels + (int64_t)kidx[p0 + q0 + j] * L0 * (int64_t)L * L;
                     KernelTimer t("sense_z_conv", s);
-                    if (z20) {
-                        if (zvar == 2) launch_zconv20<true>(a, L * L, q0, nq, zk, s);
-                        else launch_zconv20<false>(a, L * L, q0, nq, zk, s);
-                    } else {
-                        switch (zvar) {
-                        case 1: launch_zconv<8, false>(a, L * L, q0, nq, zk, s); break;
-                        case 2: launch_zconv<16, true>(a, L * L, q0, nq, zk, s); break;
-                        case 3: launch_zconv<8, true>(a, L * L, q0, nq, zk, s); break;
-                        default: launch_zconv<16, false>(a, L * L, q0, nq, zk, s); break;
-                        }
-                    }
-                    check_launch("z_conv_kernel");
+                    HASTY_REQUIRE(launch_zconv(a, L * L, q0, nq, zk, narrow, s), "no register z-convolution for this length");
+                    check_launch("z_conv_reg_kernel");
                 }
             }
-            for (int pl = 0; pl < np && L0 != 256 && !z20; ++pl) {
+            for (int pl = 0; pl < np && !zreg; ++pl) {
                 const float* K = kernels + (int64_t)kidx[p0 + pl] * L0 * (int64_t)L * L;
                 KernelTimer t("sense_z_conv", s);
-                if (zct) {
-                    hipLaunchKernelGGL(zct, dim3((unsigned)(L * L / kZC)), dim3(kZT), smem_zct, s, a, L * L, pl, K);
-                } else {
-                    hipLaunchKernelGGL(z_conv_kernel, dim3((unsigned)(L * L / kW)), dim3(kZ), smem_z, s, a, L * L, pl,
-                                       K);
-                }
+                hipLaunchKernelGGL(z_conv_kernel, dim3((unsigned)(L * L / kW)), dim3(kZ), smem_z, s, a, L * L, pl, K);
                 check_launch("z_conv_kernel");
             }
             if (inv_split && a.ccount > 1 && (int64_t)N0 * np < slots) {

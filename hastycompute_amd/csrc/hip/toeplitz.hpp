@@ -64,11 +64,11 @@ void circulant_precond_apply(const float2* in, float2* out, const float2* diag, 
 bool sense_fused_supported(const int64_t* n3);
 // 1 (default): plane kernels with register four-step y transforms; 0: LDS Stockham passes.
 void sense_fused_set_xy_variant(int v);
-// problems per z-convolution launch of the fused operator at N0 = 128 (1..16)
+// problems per register z-convolution launch of the fused operator (1..16)
 void sense_fused_set_zconv_batch(int v);
 int sense_fused_get_xy_variant();
 int sense_fused_get_zconv_batch();
-// z-convolution kernel at N0 = 128 (0..3, see sense_fused.hip)
+// z-convolution bundles at N0 = 128 and 160 (0..3, see sense_fused.hip)
 void sense_fused_set_zconv_variant(int v);
 int sense_fused_get_zconv_variant();
 // true when the current sense_xy_variant gives the register kernels at this size

@@ -175,18 +175,6 @@ SenseChoice autotune_sense_normal(const int64_t* n3, int ncoil, int nproblems, b
                 }
             }
             if (2 * n3[0] == 256) {
-                // the z-convolution kernel: the two 16-column ones (8 columns halve the
-                // row segments a wave reads and run at half speed)
-                for (int zv : {2, 0}) {
-                    if (zv == best.zconv_variant) continue;
-                    sense_fused_set_zconv_variant(zv);
-                    const double t = run_with(best.coil_batch, best.problem_batch);
-                    if (t < kGain * tbest) {
-                        tbest = t;
-                        best.zconv_variant = zv;
-                    }
-                }
-                sense_fused_set_zconv_variant(best.zconv_variant);
                 // problems per z-convolution launch: values at or above the problem batch
                 // all mean one launch per chunk, so each effective value is timed once
                 std::vector<int> seen = {std::min(best.zconv_batch, best.problem_batch)};

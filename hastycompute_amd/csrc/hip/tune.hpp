@@ -10,7 +10,7 @@ namespace hasty_hip {
 struct SenseChoice {
     int xy_variant = 2;     // plane kernels of the fused operator (library option sense_xy_variant)
     int zconv_batch = 16;   // problems per z-convolution launch at N0 = 128 (sense_zconv_batch)
-    int zconv_variant = 2;  // z-convolution kernel at N0 = 128 (sense_zconv_variant)
+    int zconv_variant = 2;  // z-convolution bundles (sense_zconv_variant; not swept, 16 columns are best)
     int problem_batch = 1;  // problems per launch (workspace sized for this many)
     int coil_batch = 1;     // coils sharing one oversampled-grid workspace
     double ms_per_problem = 0.0;
@@ -18,7 +18,7 @@ struct SenseChoice {
 
 // Times the batched Toeplitz SENSE normal operator for `nproblems` problems (at most 8
 // timed) of `ncoil` coils at image size n3 over the candidate plane kernels, problem
-// batches, z-convolution kernels and batches and coil batches; sets the library options
+// batches, z-convolution batches and coil batches; sets the library options
 // sense_xy_variant / sense_zconv_variant / sense_zconv_batch to the winners (kernels
 // must be prepared after this call) and returns the choice. Cached per shape.
 SenseChoice autotune_sense_normal(const int64_t* n3, int ncoil, int nproblems, bool allow_fused, hipStream_t s);

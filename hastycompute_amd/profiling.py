@@ -24,9 +24,8 @@ import sys
 # kernel symbol -> name used by the library's event timing
 KERNEL_NAMES = {"fwd_xy_kernel": "sense_fwd_xy", "inv_xy_kernel": "sense_inv_xy", "fwd_xy_w_kernel": "sense_fwd_xy",
                 "inv_xy_w_kernel": "sense_inv_xy", "inv_xy_d_kernel": "sense_inv_xy", "fwd_xy_r16_kernel": "sense_fwd_xy",
-                "inv_xy_r16_kernel": "sense_inv_xy", "z_conv_r16_kernel": "sense_z_conv",
-                "z_conv_r20_kernel": "sense_z_conv",
-                "z_conv_ct_kernel": "sense_z_conv", "z_conv_kernel": "sense_z_conv", "spread_kernel": "nufft_spread",
+                "inv_xy_r16_kernel": "sense_inv_xy", "coil_sum_kernel": "sense_coil_sum",
+                "z_conv_reg_kernel": "sense_z_conv", "z_conv_r8_kernel": "sense_z_conv", "z_conv_kernel": "sense_z_conv", "spread_kernel": "nufft_spread",
                 "spread_rows_kernel": "nufft_spread", "spread_planes_kernel": "nufft_spread",
                 "gather_spread_kernel": "nufft_spread", "zero_kernel": "fill_zero",
                 "interp_kernel": "nufft_interp", "axis_fft_kernel": "fft_axis", "axis_fft_r16_kernel": "fft_axis",
@@ -58,9 +57,10 @@ def counter_per_kernel(path: str):
 
 # kernel symbol -> the source file it is compiled from (for the staleness stamp)
 KERNEL_SOURCES = {"fwd_xy_r16_kernel": "sense_fused.hip", "inv_xy_r16_kernel": "sense_fused.hip",
-                  "z_conv_r16_kernel": "sense_fused.hip", "fwd_xy_w_kernel": "sense_fused.hip",
+                  "z_conv_reg_kernel": "sense_fused.hip", "z_conv_r8_kernel": "sense_fused.hip",
+                  "coil_sum_kernel": "sense_fused.hip", "fwd_xy_w_kernel": "sense_fused.hip",
                   "inv_xy_w_kernel": "sense_fused.hip", "fwd_xy_kernel": "sense_fused.hip",
-                  "inv_xy_kernel": "sense_fused.hip", "z_conv_r20_kernel": "sense_fused.hip",
+                  "inv_xy_kernel": "sense_fused.hip",
                   "spread_kernel": "nufft.hip", "interp_kernel": "nufft.hip",
                   "spread_rows_kernel": "nufft.hip", "spread_planes_kernel": "nufft.hip",
                   "gather_spread_kernel": "nufft.hip", "zero_kernel": "nufft.hip",

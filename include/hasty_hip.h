@@ -126,15 +126,13 @@ int hasty_sense_normal_toeplitz_ex(const void* x, void* out, const void* smaps, 
  *     (0 LDS Stockham, 1 coset lane-DFT, 2 register radix-16 at 128 x 128 planes and
  *     coset elsewhere, 3 coset with an LDS-DMA inverse), set before preparing kernels;
  *   "sense_zconv_batch" 1..16 (default 16): problems per z-convolution launch of the fused
- *     normal operator at N0 = 128.
+ *     normal operator at 2 N0 = 64 k <= 320.
  *   "nufft_locality" 0..4 (default 4): point ordering of plans made after the call: bit 0
  *     numbers the bins by 4^3 super-tiles, bit 1 hands the spreading and interpolation
  *     workgroups to the XCDs in contiguous runs; 4 picks 3 for type-1 and 0 for type-2
  *     plans.
- *   "sense_zconv_variant" 0..3 (default 2): z-convolution kernel at N0 = 128 (0: 16
- *     columns per workgroup, one LDS transpose buffer; 1: 8 columns; 2: 16 columns, two
- *     buffers; 3: 8 columns, two buffers) and at N0 = 160 (0: 20 x 16 register FFT, one
- *     buffer; 2: the same with two buffers; 1, 3: LDS Stockham passes).
+ *   "sense_zconv_variant" 0..3 (default 2): z-convolution bundles at N0 = 128 and 160:
+ *     0 and 2 sixteen (ky, kx) columns per workgroup, 1 and 3 eight.
  *   "llr_max_sweeps" 1..15 (default 15): cap on the Jacobi sweeps of the LLR eigensolver.
  *   "llr_eig_threads" 256, 512 or 768 (default 512): the LLR eigensolver's workgroup.
  *   "nufft_spread_tile" 0 or 12..28 (default 0 = 20): 3-D spreading tile edge in fine-grid
@@ -171,7 +169,7 @@ int hasty_get_option(const char* name, int64_t* value);
  * hasty_autotune_sense_normal: the batched Toeplitz SENSE normal operator at image size
  *   nmodes3 with ncoil coils and nproblems problems (at most 8 timed), on synthetic
  *   data: plane kernels, problems per launch, problems per z-convolution launch and
- *   coils per workspace, and at N0 = 128 the z-convolution kernel. Sets
+ *   coils per workspace. Sets
  *   sense_xy_variant, sense_zconv_variant and sense_zconv_batch to the winners (prepare
  *   kernels after this call) and writes choice[5] = {sense_xy_variant,
  *   sense_zconv_batch, problem_batch, coil_batch, sense_zconv_variant} (size the

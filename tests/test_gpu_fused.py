@@ -228,3 +228,34 @@ def test_split_launches_equal_whole_launches(N, n, coil_batch):
     ref -= sub[0]
     err = float(torch.linalg.vector_norm(whole[0] - ref) / torch.linalg.vector_norm(ref))
     assert err < 1e-6, err
+
+
+@pytest.mark.parametrize("n0", [32, 64, 96, 128, 160])
+@pytest.mark.parametrize("narrow", [False, True])
+def test_z_convolution_lengths(N, n0, narrow):
+    """The register z-convolutions (2 N0 = 64 .. 320; coil groups of one and of several
+    coils, one and two problems per launch) against the same convolution in FP64. Float32
+    FFTs of 15 levels there and back stay below 15 * 2^-23 = 1.8e-6."""
+    from hastycompute_amd import _capi
+
+    C, n = 5, 32
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(n0)
+    smaps = torch.randn((C, n0, n, n), dtype=torch.complex64, device="cuda:0", generator=gen)
+    kern = torch.rand((2, 2 * n0, 2 * n, 2 * n), dtype=torch.float32, device="cuda:0", generator=gen)
+    x = torch.randn((2, n0, n, n), dtype=torch.complex64, device="cuda:0", generator=gen)
+    prev = _capi.get_option("sense_zconv_variant")
+    _capi.set_option("sense_zconv_variant", 1 if narrow else 2)
+    try:
+        outs = [N.SenseNormalToeplitz(smaps, kern, coil_batch=cb, problem_batch=pb).apply(x, kernel_index=[1, 0])
+                for cb, pb in ((5, 2), (2, 1))]
+    finally:
+        _capi.set_option("sense_zconv_variant", prev)
+    for p in range(2):
+        ref = torch.zeros((n0, n, n), dtype=torch.complex128, device="cuda:0")
+        for s in smaps.to(torch.complex128):
+            y = torch.fft.ifftn(torch.fft.fftn(s * x[p], s=[2 * n0, 2 * n, 2 * n]) * kern[1 - p].double())
+            ref += s.conj() * y[:n0, :n, :n] * float(8 * n0 * n * n)
+        for out in outs:
+            err = float(torch.linalg.vector_norm(out[p] - ref) / torch.linalg.vector_norm(ref))
+            assert err < 1.8e-6, err

@@ -36,6 +36,9 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
 ]
+# Per-file additions. nufft.hip: the spreader's MFMA sums stay in VGPRs; in AGPRs they were
+# copied there and back around every skipped tile (8 moves per 2 MFMAs).
+FILE_FLAGS = {"nufft.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _run(cmd):
@@ -59,7 +62,8 @@ def build_hip(jobs: int = 8, verbose: bool = False) -> str:
 
     def comp(pair):
         src, obj = pair
-        return _run([HIPCC, *HIP_FLAGS, "-I", HIP_SRC, "-c", src, "-o", obj])
+        extra = FILE_FLAGS.get(os.path.basename(src), [])
+        return _run([HIPCC, *HIP_FLAGS, *extra, "-I", HIP_SRC, "-c", src, "-o", obj])
 
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
         for out in ex.map(comp, zip(srcs, objs)):

@@ -635,24 +635,22 @@ __global__ void __launch_bounds__(64 * NW) spread_planes_kernel(SpreadArgs<R> a)
 // The fine grid is cut into cores of kGC^3 cells (kGC divides every fine-grid dim). A
 // window of ns <= 16 cells overlaps one or two cores per dim, so each point belongs to at
 // most 8 cores; setpts lists, per core, the points whose windows overlap it (the pairs,
-// with the window corner relative to the core). One launch gives every core with at most
-// kGatherPart such points one workgroup that spreads them into an LDS copy of the core
-// and then stores the whole core, zeros included: each of its fine-grid cells is written
-// once with plain, whole-line stores, and neither a zero pass nor global atomics are
-// needed. A crowded core (the k-space centre of a radial trajectory) is zeroed by a small
-// kernel beforehand and split into parts of kGatherPart points whose workgroups add their
-// LDS cores to the grid with atomics. The crowded cores' parts are listed first, most
-// crowded first, so the long ones start first.
+// with the window corner relative to the core). One launch gives every core a workgroup
+// that spreads its points and stores the whole core, zeros included: each fine-grid cell
+// is written once with plain, whole-line stores, and neither a zero pass nor atomics are
+// needed. A crowded core (the k-space centre of a radial trajectory) is split into parts
+// whose sums are added in a fixed order by a second kernel. The crowded cores' parts are
+// listed first, most crowded first, so the long ones start first. Results do not depend
+// on scheduling.
 constexpr int kGC = 16;
-constexpr int kGatherWaves = 4;
-// points per part (staged at once), and the core's LDS row pitch: complex64 cores take
-// 128 points and a 19-cell pitch (three workgroups per CU at 51 KB for ns = 7), complex128
-// cores 32 points and a 17-cell pitch (two workgroups per CU at 77 KB for ns = 11)
-template <typename R> constexpr int gather_part() { return sizeof(R) == 4 ? 128 : 32; }
-template <typename R> inline int gather_row_pitch(int ns)
-{
-    return sizeof(R) == 4 ? (ns < kGC ? kGC + 3 : kGC) : kGC + 1;
-}
+constexpr int kGatherThreads = 256;
+constexpr int kGatherChunk = 64;  // points staged at once
+// Pairs per part of a crowded core: from 128 up until all crowded cores together have at
+// most kGatherMaxParts parts (each part writes and re-reads its 4096 sums: on the 128^3
+// kooshball 62 us with 290 parts, 69 us with 790; on a 64^3 one, whose grid is an eighth,
+// 80 us with 290, 60 us with 570, 57 us with 1130).
+constexpr int kGatherMinPart = 128;
+constexpr int kGatherMaxParts = 768;
 
 // ES kernel for complex64 staging with the hardware exp2 and square root (about 1 ulp
 // each, far below the tolerances a complex64 plan is made for)
@@ -708,7 +706,8 @@ template <typename R> __global__ void gather_count_kernel(GatherBins<R> g, int* 
     }
 }
 
-// points in core-bin order: first window cell l0 and fine-grid position minus l0 per dim
+// first window cell l0 per dim in core-bin order (with the point's index), and the
+// fine-grid position minus l0 by point index
 template <typename R>
 __global__ void gather_scatter_kernel(GatherBins<R> g, const int* binstart, const int* rank, int* l0, R* frac, int* idx)
 {
@@ -720,7 +719,7 @@ __global__ void gather_scatter_kernel(GatherBins<R> g, const int* binstart, cons
     for (int d = 0; d < 3; ++d) {
         const double l = ceil(t[d] - 0.5 * g.ns);
         l0[d * g.M + p] = (int)l;
-        frac[d * g.M + p] = (R)(t[d] - l);
+        frac[d * g.M + j] = (R)(t[d] - l);
     }
     idx[p] = (int)j;
 }
@@ -733,7 +732,7 @@ __global__ void gather_scatter_kernel(GatherBins<R> g, const int* binstart, cons
 // are contiguous and their order is fixed by the core-bin order of the points.
 template <typename R, bool COUNT>
 __global__ void __launch_bounds__(64) gather_pairs_kernel(GatherBins<R> g, const int* binstart, const int* l0,
-                                                          int* pcount, const int* pstart, int* pairs, int* prel)
+                                                          const int* idx, int* pcount, const int* pstart, int* pairs, int* prel)
 {
     const int ci = blockIdx.x / 27, k = blockIdx.x % 27;
     const int lane = threadIdx.x;
@@ -774,7 +773,7 @@ __global__ void __launch_bounds__(64) gather_pairs_kernel(GatherBins<R> g, const
         const unsigned long long m = __ballot(acc);
         if (!COUNT && acc) {
             const int e = out + __popcll(m & ((1ull << lane) - 1ull));
-            pairs[e] = p;
+            pairs[e] = idx[p];
             prel[e] = rel;
         }
         out += __popcll(m);
@@ -790,20 +789,21 @@ __global__ void core_pairs_kernel(const int* pstart, int* cnt, int64_t ncore)
 }
 
 template <typename R> struct GatherArgs {
-    const R* frac;       // [3][M], core-bin order
-    const int* idx;      // [M]
+    const R* frac;       // [3][M]
     const int* pstart;   // 27 cores + 1: core ci's pairs are [pstart[27 ci], pstart[27 ci + 27])
-    const int* pairs;    // sorted point of each pair
+    const int* pairs;    // point of each pair
     const int* prel;     // window corner relative to the core, 8 bits per dim (+16)
-    const int* list;     // (core, part) pairs of this launch
+    const int* list;     // (core, part) pairs of this launch, the crowded cores' first
+    cplx<R>* partial;    // [ncrowded][16^3] sums of the crowded cores' parts
     const cplx<R>* c;
     cplx<R>* fine;
     int64_t M;
     int nb[3];
     int64_t nf[3];
     R beta, cfac;
-    int rp;    // LDS row pitch of the core (float2), gather_row_pitch
-    int natomic;  // list entries [0, natomic) (the crowded cores' parts) add with atomics
+    int ns;
+    int part;      // pairs per part
+    int ncrowded;  // list entries [0, ncrowded) are parts of crowded cores
 };
 
 template <typename R> __device__ __forceinline__ R gather_es(R z, R beta, R c)
@@ -814,216 +814,201 @@ template <typename R> __device__ __forceinline__ R gather_es(R z, R beta, R c)
         return es_eval<R>(z, beta, c);
 }
 
-template <typename R, int NS>
-__global__ void __launch_bounds__(64 * kGatherWaves) gather_spread_kernel(GatherArgs<R> a)
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+template <typename R> struct MfmaTile;
+template <> struct MfmaTile<float> {
+    using Acc = floatx4;
+    __device__ __forceinline__ static Acc mac(float a, float b, Acc c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ __forceinline__ static int row(int lane, int v) { return 4 * (lane >> 4) + v; }
+};
+template <> struct MfmaTile<double> {
+    using Acc = doublex4;
+    __device__ __forceinline__ static Acc mac(double a, double b, Acc c)
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    __device__ __forceinline__ static int row(int lane, int v) { return (lane >> 4) + 4 * v; }
+};
+
+// Keeps LDS accesses of one wavefront in program order (the hardware runs them so).
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Number of lanes whose 5-bit key is smaller, or equal on a lower lane: each lane's place
+// when the wave's keys are sorted.
+__device__ __forceinline__ int rank_in_wave(int key)
+{
+    const int lane = threadIdx.x & 63;
+    unsigned long long eq = ~0ull;
+    int less = 0;
+#pragma unroll
+    for (int b = 4; b >= 0; --b) {
+        const bool one = (key >> b) & 1;
+        const unsigned long long m = __ballot(one);
+        if (one) less += __popcll(eq & ~m);
+        eq &= one ? m : ~m;
+    }
+    return less + __popcll(eq & ((1ull << lane) - 1ull));
+}
+
+// One part of one core on the matrix cores: with a point's weights laid out over the
+// core's 16 cells per dim (zero outside its window), the core is
+//   G[i0][i1][i2] = sum_p (c_p w0_p[i0]) (w1_p[i1] w2_p[i2]),
+// for every i1 a 16 x 16 product over the points (a real and an imaginary one). Wave w owns
+// i1 = w, w + 4, ...; the sums stay in its registers, so nothing is read, modified and
+// written per point. Points are staged 64 at a time, one wave per factor, sorted by their
+// first cell along i1: the four points of one MFMA step then share most of their window,
+// and the i1 that none of them reaches are skipped (about 60 % of them at ns = 7). The next
+// chunk's points load during the products. Read-modify-writes of an LDS core by four waves
+// took 241 us on the 128^3 kooshball of 147 200 points (ns = 7, 430 000 pairs), 213 us on
+// a 64^3 one of 128 000 (ns = 6) and 3.44 ms for the FP64 PSF of a 96^3 kernel (480 000
+// points, ns = 9); this form 62, 58 and 530 us (the 256^3 grid's store alone is 25 us).
+// Bound by its vector instructions (weights, operand products), not by the matrix cores.
+template <typename R> __global__ void __launch_bounds__(kGatherThreads) gather_spread_kernel(GatherArgs<R> a)
 {
     using C2 = cplx<R>;
-    constexpr int kGatherPart = gather_part<R>();
-    constexpr int kGatherRest = gather_part<R>();  // points of the parts after the first
-    constexpr int NW = kGatherWaves;
-    constexpr int NT = 64 * NW;
-    constexpr int S = 3 * NS + 2;
-    constexpr int KP = (NS + NW - 1) / NW;   // owned window planes per point, at most
-    constexpr int NQ = (NS * NS + 63) / 64;  // 64-lane chunks of a plane's NS x NS cells
-    static_assert(kGatherPart <= NT, "one staging round per part");
-    static_assert((NW & (NW - 1)) == 0, "plane ownership by a mask");
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int rp = a.rp;
-    C2* core = reinterpret_cast<C2*>(smem_raw);
-    R* stage = reinterpret_cast<R*>(core + kGC * kGC * rp);
-    int* stage_p = reinterpret_cast<int*>(stage + kGatherPart * S);
+    using Mf = MfmaTile<R>;
+    constexpr int CH = kGatherChunk;
+    __shared__ __align__(16) R st[4][CH][16];  // c.x w0, w1 (i1 = 4 j + w at 4 w + j), w2, c.y w0
+    __shared__ unsigned reach[CH / 4];         // i1 reached by each step's points, bit 4 w + j
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
+    const int n = lane & 15, kg = lane >> 4;
     const int ci = a.list[2 * blockIdx.x];
     const int part = a.list[2 * blockIdx.x + 1];
-    // pairs of this part: the first part holds kGatherPart of the core's pairs, each
-    // further part kGatherRest (staged kGatherPart at a time)
     const int pbase = a.pstart[27 * ci];
     const int cnt = a.pstart[27 * ci + 27] - pbase;
-    const int lo = part == 0 ? 0 : kGatherPart + (part - 1) * kGatherRest;
-    const int hi = min(cnt, part == 0 ? kGatherPart : lo + kGatherRest);
-
-    for (int i = tid; i < kGC * kGC * rp; i += NT) core[i] = C2{(R)0, (R)0};
-    // this lane's window rows and columns: chunk u holds (ib, q) = divmod(64 u + lane, NS)
-    int cib[NQ], cq[NQ];
+    const int lo = part * a.part;
+    const int hi = min(cnt, lo + a.part);
+    typename Mf::Acc re[4], im[4];
 #pragma unroll
-    for (int u = 0; u < NQ; ++u) {
-        const int r = u * 64 + lane;
-        cib[u] = r / NS;
-        cq[u] = r - cib[u] * NS;
+    for (int j = 0; j < 4; ++j) {
+        re[j] = typename Mf::Acc{0, 0, 0, 0};
+        im[j] = typename Mf::Acc{0, 0, 0, 0};
     }
-
-    for (int r0 = lo; r0 < hi; r0 += kGatherPart) {
-        const int np = min(kGatherPart, hi - r0);
-        __syncthreads();  // the previous round is accumulated (and the core cleared)
-        if (tid < np) {
-            const int p = a.pairs[pbase + r0 + tid];
-            const int rel = a.prel[pbase + r0 + tid];
-            const C2 cj = a.c[a.idx[p]];
-            R* st = stage + tid * S;
-            st[0] = cj.x;
-            st[1] = cj.y;
+    const int dim = wave == 3 ? 0 : wave;  // the factor this wave stages
+    const R* frac = a.frac + dim * a.M;
+    // the chunk to stage next, loaded while the current one is multiplied: first the pair
+    // (lanes without one sort last), then what its point gives
+    int rel = 31 << 8, pt = -1;
+    R fr = (R)0, scale = (R)1;
+    auto load_pair = [&](int r0) {
+        rel = 31 << 8;
+        pt = -1;
+        if (r0 + lane < hi) {
+            rel = a.prel[pbase + r0 + lane];
+            pt = a.pairs[pbase + r0 + lane];
+        }
+    };
+    auto load_point = [&]() {
+        if (pt < 0) return;
+        fr = frac[pt];
+        if (dim == 0) scale = wave == 0 ? a.c[pt].x : a.c[pt].y;
+    };
+    load_pair(lo);
+    load_point();
+    for (int r0 = lo; r0 < hi; r0 += CH) {
+        if (r0 > lo) __syncthreads();  // the previous chunk has been read
+        const int slot = rank_in_wave((rel >> 8) & 31);
+        R* flat = &st[wave][0][0];
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const R fr = a.frac[d * a.M + p];
-#pragma unroll
-                for (int q = 0; q < NS; ++q) st[2 + d * NS + q] = gather_es<R>((R)q - fr, a.beta, a.cfac);
-                stage_p[3 * tid + d] = ((rel >> (8 * d)) & 255) - 16;
+        for (int i = 0; i < CH * 16 / 64; ++i) flat[64 * i + lane] = (R)0;
+        if (wave == 1 && lane < CH / 4) reach[lane] = 0;
+        wave_order();
+        if (pt >= 0) {
+            R* row = st[wave][slot];
+            const int first = ((rel >> (8 * dim)) & 255) - 16;
+            unsigned mask = 0;
+            for (int q = 0; q < a.ns; ++q) {
+                const int i = first + q;
+                if ((unsigned)i < 16u) {
+                    const int at = wave == 1 ? 4 * (i & 3) + (i >> 2) : i;
+                    row[at] = scale * gather_es<R>((R)q - fr, a.beta, a.cfac);
+                    mask |= 1u << at;
+                }
             }
+            if (wave == 1) atomicOr(&reach[slot >> 2], mask);
         }
         __syncthreads();
-        // Wave w owns the core planes i0 with i0 mod NW == w. Per point: each lane's
-        // row-column cell offset and weight (strength folded in), then per owned plane
-        // (a wave-uniform branch) the loads of its cells; while they are in flight, the
-        // next point's row-column part; then the adds and stores. One wave's LDS
-        // operations execute in order, so the next point's loads see these stores.
-        int off[NQ];
-        C2 wc[NQ];
-        int p0 = 0;
-        auto prep = [&](int e, int* o, C2* w, int& q0) {
-            const R* st = stage + e * S;
-            const int p1 = stage_p[3 * e + 1];
-            const int p2 = stage_p[3 * e + 2];
-            q0 = stage_p[3 * e];
-            const R cx = st[0], cy = st[1];
+        const int steps = (min(CH, hi - r0) + 3) >> 2;
+        load_pair(r0 + CH);
+        const unsigned masks = reach[lane & (CH / 4 - 1)] >> (4 * wave);
+        // operands of step q, one step ahead of their use
+        R ax, ay, w2, w1[4];
+        auto load_step = [&](int q) {
+            const int e = 4 * q + kg;
+            ax = st[0][e][n];
+            ay = st[3][e][n];
+            w2 = st[2][e][n];
 #pragma unroll
-            for (int u = 0; u < NQ; ++u) {
-                const int i1 = p1 + cib[u], i2 = p2 + cq[u];
-                const bool in = u * 64 + lane < NS * NS && (unsigned)i1 < (unsigned)kGC && (unsigned)i2 < (unsigned)kGC;
-                o[u] = in ? i1 * rp + i2 : -1;
-                const R w12 = in ? st[2 + NS + cib[u]] * st[2 + 2 * NS + cq[u]] : (R)0;
-                w[u] = C2{w12 * cx, w12 * cy};
-            }
+            for (int j = 0; j < 4; ++j) w1[j] = st[1][e][4 * wave + j];
         };
-        if (np > 0) prep(0, off, wc, p0);
-        for (int e = 0; e < np; ++e) {
-            const R* st = stage + e * S;
-            const int ia0 = (wave - p0) & (NW - 1);
-            C2 val[KP][NQ];
-            int cell0[KP];
-            R w0[KP];
-            bool pl[KP];
+        load_step(0);
+        for (int q = 0; q < steps; ++q) {
+            if (q == steps / 2) load_point();
+            const R bx = ax, by = ay;
+            R w12[4];
 #pragma unroll
-            for (int k = 0; k < KP; ++k) {
-                const int ia = ia0 + k * NW;
-                const int i0 = p0 + ia;
-                pl[k] = ia < NS && (unsigned)i0 < (unsigned)kGC;  // wave-uniform
-                cell0[k] = i0 * kGC * rp;
-                w0[k] = pl[k] ? st[2 + ia] : (R)0;
-                if (pl[k]) {
+            for (int j = 0; j < 4; ++j) w12[j] = w1[j] * w2;
+            if (q + 1 < steps) load_step(q + 1);
+            const unsigned m = (unsigned)__builtin_amdgcn_readlane((int)masks, q);
 #pragma unroll
-                    for (int u = 0; u < NQ; ++u)
-                        if (off[u] >= 0) val[k][u] = core[cell0[k] + off[u]];
-                }
+            for (int j = 0; j < 4; ++j) {
+                if (!(m & (1u << j))) continue;
+                re[j] = Mf::mac(bx, w12[j], re[j]);
+                im[j] = Mf::mac(by, w12[j], im[j]);
             }
-            int noff[NQ];
-            C2 nwc[NQ];
-            int np0 = 0;
-            if (e + 1 < np) {
-                prep(e + 1, noff, nwc, np0);
-            } else {
-#pragma unroll
-                for (int u = 0; u < NQ; ++u) {
-                    noff[u] = -1;
-                    nwc[u] = C2{(R)0, (R)0};
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < KP; ++k) {
-                if (pl[k]) {
-                    const R wa = w0[k];
-#pragma unroll
-                    for (int u = 0; u < NQ; ++u) {
-                        if (off[u] >= 0) {
-                            val[k][u].x += wa * wc[u].x;
-                            val[k][u].y += wa * wc[u].y;
-                            core[cell0[k] + off[u]] = val[k][u];
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < NQ; ++u) {
-                off[u] = noff[u];
-                wc[u] = nwc[u];
-            }
-            p0 = np0;
         }
     }
-    __syncthreads();
 
-    int b[3];
-    b[2] = ci % a.nb[2];
-    b[1] = (ci / a.nb[2]) % a.nb[1];
-    b[0] = ci / (a.nb[2] * a.nb[1]);
-    const int64_t o0 = (int64_t)b[0] * kGC, o1 = (int64_t)b[1] * kGC, o2 = (int64_t)b[2] * kGC;
-    for (int i = tid; i < kGC * kGC * kGC; i += NT) {
-        const int i0 = i / (kGC * kGC), i1 = (i / kGC) % kGC, i2 = i % kGC;
-        const C2 v = core[(i0 * kGC + i1) * rp + i2];
-        C2* dst = a.fine + ((o0 + i0) * a.nf[1] + (o1 + i1)) * a.nf[2] + (o2 + i2);
-        if ((int)blockIdx.x >= a.natomic) {
-            *dst = v;
-        } else if (v.x != (R)0 || v.y != (R)0) {
-            atomicAdd(&dst->x, v.x);
-            atomicAdd(&dst->y, v.y);
-        }
+    // a part of a crowded core leaves its sums for sum_parts_kernel, the others are cores
+    const bool whole = (int)blockIdx.x >= a.ncrowded;
+    C2* dst;
+    int64_t s0, s1;
+    if (whole) {
+        const int b2 = ci % a.nb[2], b1 = (ci / a.nb[2]) % a.nb[1], b0 = ci / (a.nb[2] * a.nb[1]);
+        s1 = a.nf[2];
+        s0 = a.nf[1] * s1;
+        dst = a.fine + ((int64_t)b0 * s0 + (int64_t)b1 * s1 + b2) * kGC;
+    } else {
+        s1 = kGC;
+        s0 = kGC * kGC;
+        dst = a.partial + (int64_t)blockIdx.x * (kGC * kGC * kGC);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        C2* row = dst + Mf::row(lane, v) * s0 + wave * s1 + n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) row[4 * j * s1] = C2{re[j][v], im[j][v]};
     }
 }
 
-// zeros the cores whose parts all add with atomics (before the spreading launch)
-template <typename R> __global__ void zero_cores_kernel(cplx<R>* fine, const int* cores, int nb1, int nb2, int64_t nf1,
-                                                        int64_t nf2)
+// The crowded cores: the sums of a core's parts, in their order, stored to the grid. One
+// thread per cell; cores[3 k] is the core, then its first part and how many it has.
+template <typename R>
+__global__ void __launch_bounds__(kThreads) sum_parts_kernel(const cplx<R>* partial, const int* cores, cplx<R>* fine,
+                                                             int nb1, int nb2, int64_t nf1, int64_t nf2)
 {
-    const int ci = cores[blockIdx.x];
-    const int64_t o0 = (int64_t)(ci / (nb2 * nb1)) * kGC, o1 = (int64_t)((ci / nb2) % nb1) * kGC,
-                  o2 = (int64_t)(ci % nb2) * kGC;
-    for (int i = threadIdx.x; i < kGC * kGC * kGC; i += kThreads) {
-        const int i0 = i / (kGC * kGC), i1 = (i / kGC) % kGC, i2 = i % kGC;
-        fine[((o0 + i0) * nf1 + (o1 + i1)) * nf2 + (o2 + i2)] = cplx<R>{(R)0, (R)0};
-    }
-}
-
-// LDS bytes of a core and its stage. The complex64 pitch puts lane (ib, q) of a window
-// plane at bank pair (3 ib + q) mod 16, at most 4 lanes per pair for ns <= 9; a window of
-// 16 columns covers the banks by itself.
-template <typename R> inline size_t gather_lds_bytes(int ns)
-{
-    return sizeof(cplx<R>) * kGC * kGC * gather_row_pitch<R>(ns) + sizeof(R) * gather_part<R>() * (3 * ns + 2) +
-           sizeof(int) * gather_part<R>() * 3;
-}
-
-template <typename R, int NS> void launch_gather_ns(const GatherArgs<R>& a, int64_t blocks, hipStream_t s)
-{
-    const size_t smem = gather_lds_bytes<R>(NS);
-    allow_lds(gather_spread_kernel<R, NS>, smem);
-    hipLaunchKernelGGL((gather_spread_kernel<R, NS>), dim3((unsigned)blocks), dim3(64 * kGatherWaves), smem, s, a);
-}
-
-template <typename R> void launch_gather(int ns, const GatherArgs<R>& a, int64_t blocks, hipStream_t s)
-{
-    switch (ns) {
-#define HASTY_GATHER_CASE(K) \
-    case K: launch_gather_ns<R, K>(a, blocks, s); break;
-        HASTY_GATHER_CASE(2)
-        HASTY_GATHER_CASE(3)
-        HASTY_GATHER_CASE(4)
-        HASTY_GATHER_CASE(5)
-        HASTY_GATHER_CASE(6)
-        HASTY_GATHER_CASE(7)
-        HASTY_GATHER_CASE(8)
-        HASTY_GATHER_CASE(9)
-        HASTY_GATHER_CASE(10)
-        HASTY_GATHER_CASE(11)
-        HASTY_GATHER_CASE(12)
-        HASTY_GATHER_CASE(13)
-        HASTY_GATHER_CASE(14)
-        HASTY_GATHER_CASE(15)
-        HASTY_GATHER_CASE(16)
-#undef HASTY_GATHER_CASE
-    default: throw HastyError(kUnsupported, "kernel width out of range");
-    }
-    check_launch("gather_spread_kernel");
+    constexpr int cells = kGC * kGC * kGC;
+    const int k = blockIdx.x / (cells / kThreads), i = (blockIdx.x % (cells / kThreads)) * kThreads + threadIdx.x;
+    const int ci = cores[3 * k], np = cores[3 * k + 2];
+    const cplx<R>* src = partial + (int64_t)cores[3 * k + 1] * cells + i;
+    cplx<R> sum = src[0];
+#pragma unroll 8
+    for (int q = 1; q < np; ++q) sum = cadd(sum, src[(int64_t)q * cells]);
+    const int64_t g0 = (int64_t)(ci / (nb2 * nb1)) * kGC + i / (kGC * kGC);
+    const int64_t g1 = (int64_t)((ci / nb2) % nb1) * kGC + (i / kGC) % kGC;
+    const int64_t g2 = (int64_t)(ci % nb2) * kGC + i % kGC;
+    fine[(g0 * nf1 + g1) * nf2 + g2] = sum;
 }
 
 template <typename R, int NS, int DIM>
@@ -1442,6 +1427,7 @@ void nufft_destroy(NufftPlan* p)
     dev_free(p->g_pairs);
     dev_free(p->g_prel);
     dev_free(p->g_list);
+    dev_free(p->g_partial);
     delete p;
 }
 
@@ -1570,7 +1556,7 @@ template <typename R> void gather_build(NufftPlan* p, hipStream_t s)
         check_launch("gather_scatter_kernel");
     }
     hipLaunchKernelGGL((gather_pairs_kernel<R, true>), dim3((unsigned)(27 * ncore)), dim3(64), 0, s, g,
-                       (const int*)p->g_binstart, (const int*)p->g_l0, p->g_pcount, (const int*)nullptr, (int*)nullptr,
+                       (const int*)p->g_binstart, (const int*)p->g_l0, (const int*)nullptr, p->g_pcount, (const int*)nullptr, (int*)nullptr,
                        (int*)nullptr);
     check_launch("gather_pairs_kernel");
     hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, s, (const int*)p->g_pcount, p->g_pstart, 27 * ncore);
@@ -1595,49 +1581,65 @@ template <typename R> void gather_build(NufftPlan* p, hipStream_t s)
     }
     if (npairs > 0) {
         hipLaunchKernelGGL((gather_pairs_kernel<R, false>), dim3((unsigned)(27 * ncore)), dim3(64), 0, s, g,
-                           (const int*)p->g_binstart, (const int*)p->g_l0, (int*)nullptr, (const int*)p->g_pstart,
+                           (const int*)p->g_binstart, (const int*)p->g_l0, (const int*)p->g_idx, (int*)nullptr,
+                           (const int*)p->g_pstart,
                            p->g_pairs, p->g_prel);
         check_launch("gather_pairs_kernel");
     }
     std::vector<int> order((size_t)ncore);
     for (int64_t i = 0; i < ncore; ++i) order[(size_t)i] = (int)i;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cnt[x] > cnt[y]; });
-    // one launch: first every part of the crowded cores (more pairs than one part holds;
-    // their regions are zeroed beforehand and every part adds with atomics), most crowded
-    // first, then one part per other core, stored with plain whole-row stores
+    // one launch: first every part of the crowded cores (more pairs than one part holds),
+    // most crowded first, then the other cores
+    auto parts_of = [&](int ci, int part) { return (int)std::max<int64_t>(1, ceil_div(cnt[ci], part)); };
+    int part = kGatherMinPart;
+    for (;; part = (int)ceil_div(part + part / 4, kGatherChunk) * kGatherChunk) {
+        int64_t n = 0;
+        for (int ci : order) {
+            if (cnt[ci] <= part) break;
+            n += ceil_div(cnt[ci], part);
+        }
+        if (n <= kGatherMaxParts) break;
+    }
     std::vector<int> list, crowded;
     list.reserve((size_t)ncore * 2 + 64);
     for (int ci : order) {
-        const int parts = (int)std::max<int64_t>(1, ceil_div(cnt[ci], gather_part<R>()));
-        if (parts < 2) continue;
-        crowded.push_back(ci);
+        const int parts = parts_of(ci, part);
+        if (parts < 2) break;
+        crowded.insert(crowded.end(), {ci, (int)list.size() / 2, parts});
         for (int k = 0; k < parts; ++k) {
             list.push_back(ci);
             list.push_back(k);
         }
     }
-    const int64_t natomic = (int64_t)list.size() / 2;
+    const int64_t ncrowded = (int64_t)list.size() / 2;
     for (int ci : order) {
-        if (cnt[ci] > gather_part<R>()) continue;
+        if (parts_of(ci, part) > 1) continue;
         list.push_back(ci);
         list.push_back(0);
     }
     const size_t nlist = list.size();
     list.insert(list.end(), crowded.begin(), crowded.end());
-    const int64_t entries = (int64_t)nlist / 2;
-    if ((int64_t)list.size() > 2 * p->g_cap_list) {
+    if ((int64_t)list.size() > p->g_cap_list) {
         dev_free(p->g_list);
         p->g_list = nullptr;
         p->g_cap_list = 0;
-        const int64_t cap = ((int64_t)list.size() + 1) / 2;
-        p->g_list = (int*)dev_alloc(sizeof(int) * 2 * cap);
-        p->g_cap_list = cap;
+        p->g_list = (int*)dev_alloc(sizeof(int) * list.size());
+        p->g_cap_list = (int64_t)list.size();
+    }
+    if (ncrowded > p->g_cap_parts) {
+        dev_free(p->g_partial);
+        p->g_partial = nullptr;
+        p->g_cap_parts = 0;
+        p->g_partial = dev_alloc(sizeof(cplx<R>) * kGC * kGC * kGC * ncrowded);
+        p->g_cap_parts = ncrowded;
     }
     HASTY_HIP_CHECK(hipMemcpyAsync(p->g_list, list.data(), sizeof(int) * list.size(), hipMemcpyHostToDevice, s));
     HASTY_HIP_CHECK(hipStreamSynchronize(s));  // the host list goes out of scope
-    p->g_first = entries;
-    p->g_rest = natomic;
-    p->g_nzero = (int64_t)crowded.size();
+    p->g_part = part;
+    p->g_entries = (int64_t)nlist / 2;
+    p->g_ncrowded = ncrowded;
+    p->g_crowded_cores = (int64_t)crowded.size() / 3;
     p->gather_built = 1;
 }
 
@@ -1645,7 +1647,6 @@ template <typename R> void gather_spread(NufftPlan* p, const cplx<R>* c, cplx<R>
 {
     GatherArgs<R> a;
     a.frac = reinterpret_cast<const R*>(p->g_frac);
-    a.idx = p->g_idx;
     a.pstart = p->g_pstart;
     a.pairs = p->g_pairs;
     a.prel = p->g_prel;
@@ -1659,15 +1660,20 @@ template <typename R> void gather_spread(NufftPlan* p, const cplx<R>* c, cplx<R>
     }
     a.beta = (R)p->beta;
     a.cfac = (R)(4.0 / ((double)p->ns * p->ns));
-    a.rp = gather_row_pitch<R>(p->ns);
-    a.natomic = (int)p->g_rest;
+    a.ns = p->ns;
+    a.partial = reinterpret_cast<cplx<R>*>(p->g_partial);
+    a.part = p->g_part;
+    a.ncrowded = (int)p->g_ncrowded;
     KernelTimer t("nufft_spread", s);
-    if (p->g_nzero > 0) {
-        hipLaunchKernelGGL((zero_cores_kernel<R>), dim3((unsigned)p->g_nzero), dim3(kThreads), 0, s, fine,
-                           (const int*)(p->g_list + 2 * p->g_first), a.nb[1], a.nb[2], a.nf[1], a.nf[2]);
-        check_launch("zero_cores_kernel");
+    hipLaunchKernelGGL((gather_spread_kernel<R>), dim3((unsigned)p->g_entries), dim3(kGatherThreads), 0, s, a);
+    check_launch("gather_spread_kernel");
+    if (p->g_crowded_cores > 0) {
+        const int64_t blocks = p->g_crowded_cores * (kGC * kGC * kGC / kThreads);
+        hipLaunchKernelGGL((sum_parts_kernel<R>), dim3((unsigned)blocks), dim3(kThreads), 0, s,
+                           (const cplx<R>*)a.partial, (const int*)(p->g_list + 2 * p->g_entries), fine, a.nb[1], a.nb[2],
+                           a.nf[1], a.nf[2]);
+        check_launch("sum_parts_kernel");
     }
-    launch_gather<R>(p->ns, a, p->g_first, s);
 }
 
 template <typename R> void execute_type2(NufftPlan* p, cplx<R>* c, const cplx<R>* f, hipStream_t s)

@@ -47,20 +47,23 @@ struct NufftPlan {
     int* g_counts = nullptr;    // points per core bin
     int* g_binstart = nullptr;  // core bins + 1 (scan)
     int* g_l0 = nullptr;        // [3][M] first window cell per dim, in core-bin order
-    void* g_frac = nullptr;     // [3][M] fine-grid position minus that cell (plan precision)
+    void* g_frac = nullptr;     // [3][M] fine-grid position minus that cell, by point (plan precision)
     int* g_idx = nullptr;       // [M] point index, in core-bin order
     int* g_rank = nullptr;      // [M] rank within the core bin
     int* g_pcount = nullptr;    // (point, core) pairs per (core, neighbour bin): 27 per core
     int* g_pstart = nullptr;    // 27 cores + 1 (scan)
-    int* g_pairs = nullptr;     // sorted point of each pair, grouped by core
+    int* g_pairs = nullptr;     // point of each pair, grouped by core
     int* g_prel = nullptr;      // window corner relative to the core
-    int* g_list = nullptr;      // (core, part) entries, then the crowded cores
+    int* g_list = nullptr;      // (core, part) entries, then (core, first part, parts) of the crowded cores
+    void* g_partial = nullptr;  // [g_ncrowded][16^3] sums of the crowded cores' parts (plan precision)
     int64_t g_cap_M = 0;
     int64_t g_cap_pairs = 0;
     int64_t g_cap_list = 0;
-    int64_t g_first = 0;        // (core, part) entries of the spreading launch
-    int64_t g_rest = 0;         // of them the crowded cores' parts, first, adding with atomics
-    int64_t g_nzero = 0;        // crowded cores (listed after the entries), zeroed beforehand
+    int64_t g_cap_parts = 0;
+    int g_part = 0;               // pairs per part
+    int64_t g_entries = 0;        // (core, part) entries of the spreading launch
+    int64_t g_ncrowded = 0;       // of them the crowded cores' parts, first
+    int64_t g_crowded_cores = 0;  // crowded cores, summed from their parts
 };
 
 // nmodes in FINUFFT order (fastest-varying first), as the reference passes

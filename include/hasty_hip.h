@@ -144,9 +144,10 @@ int hasty_sense_normal_toeplitz_ex(const void* x, void* out, const void* smaps, 
  *     waves and LDS atomics, 3 four waves clearing and flushing the tile while one wave
  *     accumulates without atomics, 4 and 5 four and eight waves each owning the tile
  *     planes congruent to its index, 6 output-driven: one workgroup per 16^3-cell core
- *     of the fine grid spreads the points whose windows overlap it and stores the core
- *     once (no zero pass, no global atomics outside crowded cores; plans whose fine-grid
- *     dims are multiples of 16 and at least 48, binned at setpts; other plans run 3).
+ *     of the fine grid spreads the points whose windows overlap it on the matrix cores and
+ *     stores the core once (no zero pass, no atomics: crowded cores are summed from parts in
+ *     a fixed order; plans whose fine-grid dims are multiples of 16 and at least 48, binned
+ *     at setpts; other plans run 3).
  *   "fft_r16" 0 or 1 (default 1): complex64 axis FFT passes of length 128, 192, 256 or
  *     320 (the NUFFT at 64^3 .. 160^3 modes) without coil multipliers, accumulation or
  *     convolution run as a 16 x R four-step FFT in registers; 0 keeps them on the LDS

@@ -604,3 +604,33 @@ def test_svt_matrix_many_kept(N, R, F):
         e2 = O.rel_l2(h(Ah), O.svt_hard(A.astype(np.complex128), rank))
         print(f"svt R={R} F={F} hard rank={rank}: {e2:.2e}", flush=True)
         assert e2 < 1e-4
+
+
+@pytest.mark.parametrize("M", [1, 3, 64, 65, 129, 4000, 150000])
+@pytest.mark.parametrize("fp64,tol", [(False, 1e-1), (False, 1e-4), (False, 1e-6), (True, 1e-9), (True, 1e-14)])
+def test_output_spreader_parts_and_widths(N, M, fp64, tol):
+    """The output-driven spreader at its edges: steps and chunks that are not full, cores
+    split into few and into many parts (half the points piled up on one cell corner), and
+    kernel widths 2 to 15, against the direct sum; two runs give the same bits. Bound: ten
+    times the plan's tolerance, at least 3e-6 for float32 sums."""
+    n, ct = 24, torch.complex128 if fp64 else torch.complex64
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(M)
+    co = (torch.rand((3, M), dtype=torch.float64, device="cuda:0", generator=gen) * 2 - 1) * np.pi
+    co[:, : M // 2] = 1e-3 * co[:, : M // 2] + torch.tensor([[0.0], [np.pi / 3], [-2.0]], device="cuda:0")
+    co = co.to(torch.float64 if fp64 else torch.float32)
+    c = torch.randn((1, M), dtype=ct, device="cuda:0", generator=gen)
+    plan = N.NufftPlan(co, [n, n, n], 1, +1, 1, tol)
+    f, f2 = torch.empty((1, n, n, n), dtype=ct, device="cuda:0"), torch.empty((1, n, n, n), dtype=ct, device="cuda:0")
+    plan.execute(c, f)
+    plan.execute(c, f2)
+    assert torch.equal(f, f2)
+    m = torch.arange(n, dtype=torch.float64, device="cuda:0") - n // 2
+    e = [torch.exp(1j * m[:, None] * co[d].double()[None, :]) for d in range(3)]
+    ref = torch.zeros((n * n, n), dtype=torch.complex128, device="cuda:0")
+    for a in range(0, M, 20000):
+        s = slice(a, min(M, a + 20000))
+        left = ((c[0, s].to(torch.complex128) * e[0][:, s])[:, None, :] * e[1][None, :, s]).reshape(n * n, -1)
+        ref += left @ e[2][:, s].T.contiguous()
+    err = float(torch.linalg.vector_norm(f[0].reshape(n * n, n) - ref) / torch.linalg.vector_norm(ref))
+    assert err < max(10 * tol, 1e-12 if fp64 else 3e-6), err

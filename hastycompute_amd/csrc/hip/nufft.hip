@@ -1011,82 +1011,130 @@ __global__ void __launch_bounds__(kThreads) sum_parts_kernel(const cplx<R>* part
     fine[(g0 * nf1 + g1) * nf2 + g2] = sum;
 }
 
+// 3-D interpolation, a group of lanes per point: lane m of a group reads 16 bytes of every
+// window row (two complex64 cells, or one complex128 cell), so a group's loads of one row
+// are one contiguous segment and a wave touches 64 / kLanes rows per instruction. One lane
+// per point touched 64 rows with each of its W / 2 loads per row, and the address units'
+// one line per cycle bound it: 128^3 kooshball (147 200 points, ns = 7) 123 us, 68 us here;
+// 150 000 points on a 144 x 200 x 180 grid (ns = 6) 71 us, 31 us here.
+// complex64 windows start at the even cell at or below their first one; fine-grid dims are
+// even, so a pair never straddles the periodic edge.
+template <typename R, int NS> struct InterpShape {
+    static constexpr int cells = sizeof(R) == 4 ? 2 : 1;                     // cells per lane
+    static constexpr int used = sizeof(R) == 4 ? (NS + 2) / 2 : NS;          // lanes with cells
+    static constexpr int lanes = used <= 2 ? 2 : used <= 4 ? 4 : used <= 8 ? 8 : 16;
+    static constexpr int points = kThreads / lanes;  // per workgroup
+};
+
+template <typename R, int NS> __global__ void __launch_bounds__(kThreads) interp3_kernel(SpreadArgs<R> a)
+{
+    using Sh = InterpShape<R, NS>;
+    constexpr int GL = Sh::lanes, CPL = Sh::cells;
+    constexpr int WS = 2 * NS + 1;  // weights of a point along dims 0 and 1, odd pitch
+    __shared__ R ws[Sh::points * WS];
+    const PtsArgs<R>& pa = a.pa;
+    const int m = threadIdx.x % GL, pl = threadIdx.x / GL;
+    const int64_t p = xcd_block(a.xcd) * Sh::points + pl;
+    const bool on = p < pa.M;
+    const int j = on ? a.sortidx[p] : 0;
+    int l[3] = {0, 0, 0};
+    double fr[3] = {0, 0, 0};
+    if (on) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double t = fine_pos((double)pa.pts[d][j], pa.nf[d]);
+            const double l0 = ceil(t - 0.5 * NS);
+            l[d] = (int)l0;
+            fr[d] = t - l0;
+        }
+    }
+    // the group's weights along dims 0 and 1, dealt to its lanes, and this lane's own along 2
+#pragma unroll
+    for (int e = 0; e < 2 * NS; e += GL) {
+        const int q = e + m;
+        if (q < 2 * NS) ws[pl * WS + q] = es_eval<R>((R)(q < NS ? q - fr[0] : q - NS - fr[1]), a.beta, a.cfac);
+    }
+    const int c0 = sizeof(R) == 4 ? (l[2] & ~1) + 2 * m : l[2] + m;  // first cell of this lane
+    R w2[CPL];
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) {
+        const int q = c0 + k - l[2];
+        w2[k] = q >= 0 && q < NS ? es_eval<R>((R)(q - fr[2]), a.beta, a.cfac) : (R)0;
+    }
+    __syncthreads();
+    const int n0 = (int)pa.nf[0], n1 = (int)pa.nf[1], n2 = (int)pa.nf[2];
+    // lanes past the window read their group's first cells (zero weight)
+    const bool mine = on && m < Sh::used;
+    int cell = mine ? c0 : sizeof(R) == 4 ? (l[2] & ~1) : l[2];
+    cell += cell < 0 ? n2 : 0;
+    cell -= cell >= n2 ? n2 : 0;
+    int64_t row1[NS];
+    R w1[NS];
+#pragma unroll
+    for (int ib = 0; ib < NS; ++ib) {
+        int i1 = l[1] + ib;
+        i1 += i1 < 0 ? n1 : 0;
+        i1 -= i1 >= n1 ? n1 : 0;
+        row1[ib] = (int64_t)i1 * n2 + cell;
+        w1[ib] = ws[pl * WS + NS + ib];
+    }
+    R sr = 0, si = 0;
+#pragma unroll 1
+    for (int ia = 0; ia < NS; ++ia) {
+        int i0 = l[0] + ia;
+        i0 += i0 < 0 ? n0 : 0;
+        i0 -= i0 >= n0 ? n0 : 0;
+        const cplx<R>* plane = a.fine + (int64_t)i0 * n1 * n2;
+        const R w0 = ws[pl * WS + ia];
+        R tr = 0, ti = 0;
+#pragma unroll
+        for (int ib = 0; ib < NS; ++ib) {
+            if constexpr (sizeof(R) == 4) {
+                const float4 g = *reinterpret_cast<const float4*>(plane + row1[ib]);
+                tr += w1[ib] * (w2[0] * g.x + w2[1] * g.z);
+                ti += w1[ib] * (w2[0] * g.y + w2[1] * g.w);
+            } else {
+                const cplx<R> g = plane[row1[ib]];
+                tr += w1[ib] * (w2[0] * g.x);
+                ti += w1[ib] * (w2[0] * g.y);
+            }
+        }
+        sr += w0 * tr;
+        si += w0 * ti;
+    }
+    if (!mine) sr = si = (R)0;
+#pragma unroll
+    for (int o = GL / 2; o > 0; o >>= 1) {
+        sr += __shfl_xor(sr, o);
+        si += __shfl_xor(si, o);
+    }
+    if (on && m == 0) a.cout[j] = cplx<R>{sr, si};
+}
+
+// 1-D and 2-D interpolation, one lane per point.
 template <typename R, int NS, int DIM>
 __global__ void __launch_bounds__(kThreads) interp_kernel(SpreadArgs<R> a)
 {
+    static_assert(DIM <= 2, "3-D points go to interp3_kernel");
     const PtsArgs<R>& pa = a.pa;
     const int64_t p = xcd_block(a.xcd) * kThreads + threadIdx.x;
     if (p >= pa.M) return;
     const int j = a.sortidx[p];
     R w[2][NS];
     int64_t idx[2][NS];
-    double t0 = 0.0, l00 = 0.0;
 #pragma unroll
     for (int d = 3 - DIM; d < 3; ++d) {
         const double t = fine_pos((double)pa.pts[d][j], pa.nf[d]);
         const double l0 = ceil(t - 0.5 * NS);
-        if (d == 0) {
-            t0 = t;
-            l00 = l0;
-        } else {
-            const int64_t il0 = (int64_t)l0;
+        const int64_t il0 = (int64_t)l0;
 #pragma unroll
-            for (int q = 0; q < NS; ++q) {
-                w[d - 1][q] = es_eval<R>((R)(l0 + q - t), a.beta, a.cfac);
-                idx[d - 1][q] = wrapi(il0 + q, pa.nf[d]);
-            }
+        for (int q = 0; q < NS; ++q) {
+            w[d - 1][q] = es_eval<R>((R)(l0 + q - t), a.beta, a.cfac);
+            idx[d - 1][q] = wrapi(il0 + q, pa.nf[d]);
         }
     }
     R sr = 0, si = 0;
-    if (DIM == 3) {
-        // complex64 rows that do not wrap: the window's cells from the even cell at or
-        // below its first one, read as 16-byte pairs (W / 2 loads instead of NS) against
-        // the weights shifted by that offset
-        constexpr int W = (NS + 2) & ~1;
-        R w8[W];
-        bool pairs = false;
-        int64_t a2 = 0;
-        if constexpr (std::is_same<R, float>::value) {
-            const int off = (int)(idx[1][0] & 1);
-            a2 = idx[1][0] - off;
-            pairs = a2 + W <= pa.nf[2] && idx[1][NS - 1] == idx[1][0] + NS - 1;
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                R v = (R)0;
-#pragma unroll
-                for (int q = 0; q < NS; ++q) v = (k == q + off) ? w[1][q] : v;
-                w8[k] = v;
-            }
-        }
-        for (int ia = 0; ia < NS; ++ia) {
-            const R wa = es_eval<R>((R)(l00 + ia - t0), a.beta, a.cfac);
-            const int64_t i0 = wrapi((int64_t)l00 + ia, pa.nf[0]);
-#pragma unroll
-            for (int ib = 0; ib < NS; ++ib) {
-                const R wab = wa * w[0][ib];
-                const cplx<R>* row = a.fine + (i0 * pa.nf[1] + idx[0][ib]) * pa.nf[2];
-                R tr = 0, ti = 0;
-                if (pairs) {
-                    const float4* r4 = reinterpret_cast<const float4*>(row + a2);
-#pragma unroll
-                    for (int k = 0; k < W / 2; ++k) {
-                        const float4 g = r4[k];
-                        tr += w8[2 * k] * g.x + w8[2 * k + 1] * g.z;
-                        ti += w8[2 * k] * g.y + w8[2 * k + 1] * g.w;
-                    }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < NS; ++q) {
-                        const cplx<R> g = row[idx[1][q]];
-                        tr += w[1][q] * g.x;
-                        ti += w[1][q] * g.y;
-                    }
-                }
-                sr += wab * tr;
-                si += wab * ti;
-            }
-        }
-    } else if (DIM == 2) {
+    if (DIM == 2) {
 #pragma unroll
         for (int ib = 0; ib < NS; ++ib) {
             const cplx<R>* row = a.fine + idx[0][ib] * pa.nf[2];
@@ -1158,8 +1206,14 @@ void launch_spread_ns(const SpreadArgs<R>& a, int64_t nsub, size_t smem, hipStre
 template <typename R, int NS, int DIM> void launch_interp_ns(const SpreadArgs<R>& a, int64_t M, hipStream_t s)
 {
     KernelTimer t("nufft_interp", s);
-    hipLaunchKernelGGL((interp_kernel<R, NS, DIM>), dim3((unsigned)xcd_grid(ceil_div(M, kThreads), a.xcd)), dim3(kThreads), 0,
-                       s, a);
+    if constexpr (DIM == 3) {
+        hipLaunchKernelGGL((interp3_kernel<R, NS>),
+                           dim3((unsigned)xcd_grid(ceil_div(M, (InterpShape<R, NS>::points)), a.xcd)), dim3(kThreads), 0, s,
+                           a);
+    } else {
+        hipLaunchKernelGGL((interp_kernel<R, NS, DIM>), dim3((unsigned)xcd_grid(ceil_div(M, kThreads), a.xcd)),
+                           dim3(kThreads), 0, s, a);
+    }
 }
 
 template <typename R, int DIM>
@@ -1361,6 +1415,9 @@ NufftPlan* nufft_makeplan(int type, int dim, const int64_t* nmodes, int iflag, i
         if (dim == 3) {
             const double cells = 8000.0;
             int t = (int)std::floor(std::cbrt(cells) + 1e-9);
+            // interpolation only takes its point order from the tiles: 16^3 ones ran 5-12 %
+            // faster than 20^3 (71 -> 68 us at 128^3, 171 -> 159 us at 160^3, ns = 7)
+            if (type == 2) t = 16;
             if (g_tile.load() > 0) t = g_tile.load();
             int b = t - p->ns - 1;
             b = std::max(2, b);

@@ -634,3 +634,30 @@ def test_output_spreader_parts_and_widths(N, M, fp64, tol):
         ref += left @ e[2][:, s].T.contiguous()
     err = float(torch.linalg.vector_norm(f[0].reshape(n * n, n) - ref) / torch.linalg.vector_norm(ref))
     assert err < max(10 * tol, 1e-12 if fp64 else 3e-6), err
+
+
+@pytest.mark.parametrize("dims", [(24, 24, 24), (9, 30, 17), (4, 5, 90)])
+@pytest.mark.parametrize("fp64,tol", [(False, 1e-1), (False, 1e-2), (False, 1e-3), (False, 1e-5), (False, 1e-6),
+                                      (False, 1e-8), (True, 1e-6), (True, 1e-9), (True, 1e-14)])
+def test_interpolation_lane_groups(N, dims, fp64, tol):
+    """Type 2 with every lane-group size (kernel widths 2 to 15), windows across the
+    periodic edge in each dim, odd and even first cells, and a ragged last group, against
+    the direct sum. Bound: ten times the tolerance, at least 3e-6 for float32 sums."""
+    ct = torch.complex128 if fp64 else torch.complex64
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(sum(dims))
+    M = 1237
+    co = (torch.rand((3, M), dtype=torch.float64, device="cuda:0", generator=gen) * 2 - 1) * np.pi
+    co[:, :200] *= 0.01           # around fine-grid cell 0
+    co[0, 200:300] = -np.pi       # the lower end, and just below the upper one
+    co[2, 250:350] = np.pi - 1e-3
+    co = co.to(torch.float64 if fp64 else torch.float32)
+    f = torch.randn((2, *dims), dtype=ct, device="cuda:0", generator=gen)
+    got = N.nufft(co, f, dims, 2, -1, tol)
+    ax = [torch.arange(n, dtype=torch.float64, device="cuda:0") - n // 2 for n in dims]
+    e = [torch.exp(-1j * ax[d][:, None] * co[d].double()[None, :]) for d in range(3)]
+    for t in range(2):
+        v = (f[t].to(torch.complex128).reshape(-1, dims[2]) @ e[2]).reshape(dims[0], dims[1], M)
+        ref = ((v * e[1][None]).sum(1) * e[0]).sum(0)
+        err = float(torch.linalg.vector_norm(got[t] - ref) / torch.linalg.vector_norm(ref))
+        assert err < max(10 * tol, 1e-12 if fp64 else 3e-6), err

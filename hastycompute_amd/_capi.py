@@ -36,6 +36,8 @@ _SIGS = {
     "hasty_nufft_destroy": ([c_vp], c_int),
     "hasty_nufft_info": ([c_vp, P_i64, ctypes.POINTER(c_int), P_dbl], c_int),
     "hasty_toeplitz_build": ([c_vp, c_int, c_i64, c_int, P_i64, c_vp, c_vp, c_vp, c_dbl, c_vp], c_int),
+    "hasty_toeplitz_workspace_size": ([c_i64, c_int, P_i64, c_dbl], c_sz),
+    "hasty_toeplitz_build_ws": ([c_vp, c_int, c_i64, c_int, P_i64, c_vp, c_vp, c_vp, c_dbl, c_vp, c_sz, c_vp], c_int),
     "hasty_toeplitz_apply": ([c_vp, c_vp, c_vp, c_vp, c_int, c_int, P_i64, c_int, c_vp, c_vp, c_vp], c_int),
     "hasty_sense_normal_workspace_size": ([P_i64, c_int, c_int], c_sz),
     "hasty_sense_normal_prepare": ([c_vp, c_vp, c_i64, P_i64, ctypes.POINTER(c_int), c_vp], c_int),

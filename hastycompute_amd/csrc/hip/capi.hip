@@ -183,7 +183,29 @@ __global__ void zero_corner_kernel(int3* c)
 
 void set_last_error(const std::string& msg) { g_last_error = msg; }
 
-void* dev_alloc(size_t bytes)
+namespace {
+thread_local DeviceArena* t_arena = nullptr;
+}
+
+DeviceArena::DeviceArena(void* base, size_t bytes) : base_(static_cast<char*>(base)), size_(base ? bytes : 0), outer_(t_arena)
+{
+    const size_t skew = (256 - reinterpret_cast<uintptr_t>(base) % 256) % 256;
+    used_ = std::min(size_, skew);
+    t_arena = this;
+}
+
+DeviceArena::~DeviceArena() { t_arena = outer_; }
+
+void* DeviceArena::take(size_t bytes)
+{
+    const size_t need = (bytes + 255) / 256 * 256;
+    if (need > size_ - used_) return nullptr;
+    void* p = base_ + used_;
+    used_ += need;
+    return p;
+}
+
+void* dev_alloc_table(size_t bytes)
 {
     void* p = nullptr;
     if (bytes == 0) bytes = 16;
@@ -191,9 +213,16 @@ void* dev_alloc(size_t bytes)
     return p;
 }
 
+void* dev_alloc(size_t bytes)
+{
+    if (t_arena)
+        if (void* p = t_arena->take(std::max<size_t>(bytes, 16))) return p;
+    return dev_alloc_table(bytes);
+}
+
 void dev_free(void* p)
 {
-    if (p) (void)hipFree(p);
+    if (p && !(t_arena && t_arena->owns(p))) (void)hipFree(p);
 }
 
 int current_device()
@@ -287,6 +316,25 @@ int hasty_toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim
         HASTY_REQUIRE(nmodes != nullptr, "null nmodes");
         toeplitz_build(coords, coord_fp64, M, ndim, nmodes, weights, reinterpret_cast<float2*>(diag_ref), kernel, tol,
                        as_stream(stream));
+    });
+}
+
+size_t hasty_toeplitz_workspace_size(int64_t M, int ndim, const int64_t* nmodes, double tol)
+{
+    if (M < 0 || ndim < 1 || ndim > 3 || !nmodes || !(tol > 0.0)) return 0;
+    return toeplitz_workspace_bytes(M, ndim, nmodes, tol);
+}
+
+int hasty_toeplitz_build_ws(const void* coords, int coord_fp64, int64_t M, int ndim, const int64_t* nmodes,
+                            const float* weights, void* diag_ref, float* kernel, double tol, void* workspace,
+                            size_t workspace_bytes, void* stream)
+{
+    return guarded([&] {
+        HASTY_REQUIRE(coords != nullptr || M == 0, "null coords");
+        HASTY_REQUIRE(nmodes != nullptr, "null nmodes");
+        HASTY_REQUIRE(workspace != nullptr || workspace_bytes == 0, "null workspace");
+        toeplitz_build(coords, coord_fp64, M, ndim, nmodes, weights, reinterpret_cast<float2*>(diag_ref), kernel, tol,
+                       as_stream(stream), workspace, workspace_bytes);
     });
 }
 

@@ -98,6 +98,30 @@ void* dev_alloc(size_t bytes);
 void dev_free(void* p);
 int current_device();
 
+// While a DeviceArena is alive, dev_alloc on its thread takes from the caller's workspace
+// (in order, 256-byte aligned; hipMalloc once it is full) and dev_free leaves that memory
+// alone. For calls that own everything they allocate and have finished with it on their
+// stream when they return; hipMalloc and hipFree of a kernel build's gigabyte cost
+// milliseconds per call, at times tens of them.
+class DeviceArena {
+public:
+    DeviceArena(void* base, size_t bytes);
+    ~DeviceArena();
+    size_t mark() const { return used_; }
+    void reset(size_t m) { used_ = m; }  // what was taken since mark() is free again
+    void* take(size_t bytes);            // null when it does not fit
+    bool owns(const void* p) const { return p >= base_ && p < base_ + size_; }
+    DeviceArena(const DeviceArena&) = delete;
+    DeviceArena& operator=(const DeviceArena&) = delete;
+
+private:
+    char* base_;
+    size_t size_, used_ = 0;
+    DeviceArena* outer_;
+};
+// dev_alloc for tables that outlive the call (never from an arena).
+void* dev_alloc_table(size_t bytes);
+
 // Per-kernel timing with HIP events recorded on the launch stream around each launch
 // (off by default; hasty_timing_enable). Bracket a launch with a KernelTimer in scope.
 bool timing_on();

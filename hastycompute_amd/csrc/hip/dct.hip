@@ -69,7 +69,7 @@ const float* dct_tiles(int N, int inverse, hipStream_t s)
     if (it != g_tiles.end()) return it->second;
     const int rt = ((N + 1) / 2 + 15) / 16;
     const int n = 2 * rt * rt * 256;
-    float* t = (float*)dev_alloc(sizeof(float) * n);
+    float* t = (float*)dev_alloc_table(sizeof(float) * n);
     try {
         hipLaunchKernelGGL(dct_tiles_kernel, dim3((unsigned)ceil_div(n, kDctThreads)), dim3(kDctThreads), 0, s, t, N, rt,
                            inverse);

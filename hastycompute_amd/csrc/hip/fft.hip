@@ -551,7 +551,7 @@ template <typename R> const cplx<R>* twiddles(int L)
         const long double ang = -twopi * (long double)k / (long double)L;
         host[k] = cplx<R>{(R)std::cos(ang), (R)std::sin(ang)};
     }
-    void* d = dev_alloc(sizeof(cplx<R>) * L);
+    void* d = dev_alloc_table(sizeof(cplx<R>) * L);
     HASTY_HIP_CHECK(hipMemcpy(d, host.data(), sizeof(cplx<R>) * L, hipMemcpyHostToDevice));
     g_tw_cache[key] = d;
     return reinterpret_cast<const cplx<R>*>(d);

@@ -123,8 +123,30 @@ struct DevBuf {
 
 }  // namespace
 
+// Device memory of toeplitz_build: its own arrays, the plan's grids and point arrays, with
+// room for 4 (point, core) pairs per point (a window of 9 of 16 cells crosses 3.4 cores in
+// the mean). A build that needs more allocates the rest.
+size_t toeplitz_workspace_bytes(int64_t M, int ndim, const int64_t* nmodes, double tol)
+{
+    double grid = 1.0, fine = 1.0, tmp = 1.0;
+    int ns = 2;
+    double beta = 0.0;
+    es_params(tol, &ns, &beta);
+    for (int d = 0; d < ndim; ++d) {
+        const double L = 2.0 * (double)nmodes[d];
+        const double nf = (double)next235even(std::max<int64_t>(4 * nmodes[d], 2 * ns));
+        grid *= L;
+        fine *= nf;
+        tmp *= d == ndim - 1 ? L : nf;
+    }
+    const double points = (double)M * (8.0 * ndim + 16 + 12 + 24 + 4 + 4 + 8 + 8 + 4 * 8);
+    const double bins = fine / 64.0 * 24.0 + fine / 4096.0 * 27.0 * 8.0 + 1024.0 * 65536.0;
+    return (size_t)(16.0 * (grid + fine + tmp) + points + bins) + (1u << 20);
+}
+
 void toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, const int64_t* nmodes,
-                    const float* weights, float2* diag_ref, float* kernel, double tol, hipStream_t s)
+                    const float* weights, float2* diag_ref, float* kernel, double tol, hipStream_t s, void* workspace,
+                    size_t workspace_bytes)
 {
     HASTY_REQUIRE(ndim >= 1 && ndim <= 3, "Dimension must be 1,2 or 3");
     HASTY_REQUIRE(M >= 0, "M must be >= 0");
@@ -135,33 +157,40 @@ void toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, con
         L[3 - ndim + d] = 2 * nmodes[d];
     }
     const int64_t ngrid = L[0] * L[1] * L[2];
+    // the build ends with its stream synchronised, so nothing in the arena is in use after it
+    DeviceArena arena(workspace, workspace_bytes);
 
-    // FP64 coordinates and strengths.
-    DevBuf cd(sizeof(double) * std::max<int64_t>(1, (int64_t)ndim * M));
-    const double* cdp = reinterpret_cast<const double*>(coords);
-    if (!coord_fp64) {
-        launch1d(coords_to_double_kernel, (int64_t)ndim * M, s, (const float*)coords, (double*)cd.p, (int64_t)ndim * M);
-        cdp = (const double*)cd.p;
-    }
-    DevBuf cw(sizeof(double2) * std::max<int64_t>(1, M));
-    launch1d(strengths_kernel, M, s, weights, (double2*)cw.p, M);
-
-    // Type-1 (isign +1) FP64 NUFFT onto the doubled modes: psf[n] = sum_j w_j exp(+i (n - N).x_j).
-    int64_t nm_flip[3];
-    for (int d = 0; d < ndim; ++d) nm_flip[d] = 2 * nmodes[ndim - 1 - d];
-    NufftPlan* plan = nufft_makeplan(1, ndim, nm_flip, 1, 1, tol, 1);
     DevBuf psf(sizeof(double2) * ngrid);
-    try {
-        const double* row[3] = {nullptr, nullptr, nullptr};
-        for (int d = 0; d < ndim; ++d) row[d] = cdp + (int64_t)(ndim - 1 - d) * M;  // x = last row
-        nufft_setpts(plan, M, row[0], row[1], row[2], s);
-        nufft_execute(plan, cw.p, psf.p, s);
-        HASTY_HIP_CHECK(hipStreamSynchronize(s));
-    } catch (...) {
+    const size_t after_psf = arena.mark();
+    {
+        // FP64 coordinates and strengths.
+        DevBuf cd(coord_fp64 ? 16 : sizeof(double) * std::max<int64_t>(1, (int64_t)ndim * M));
+        const double* cdp = reinterpret_cast<const double*>(coords);
+        if (!coord_fp64) {
+            launch1d(coords_to_double_kernel, (int64_t)ndim * M, s, (const float*)coords, (double*)cd.p, (int64_t)ndim * M);
+            cdp = (const double*)cd.p;
+        }
+        DevBuf cw(sizeof(double2) * std::max<int64_t>(1, M));
+        launch1d(strengths_kernel, M, s, weights, (double2*)cw.p, M);
+
+        // Type-1 (isign +1) FP64 NUFFT onto the doubled modes: psf[n] = sum_j w_j exp(+i (n - N).x_j).
+        int64_t nm_flip[3];
+        for (int d = 0; d < ndim; ++d) nm_flip[d] = 2 * nmodes[ndim - 1 - d];
+        NufftPlan* plan = nufft_makeplan(1, ndim, nm_flip, 1, 1, tol, 1);
+        try {
+            const double* row[3] = {nullptr, nullptr, nullptr};
+            for (int d = 0; d < ndim; ++d) row[d] = cdp + (int64_t)(ndim - 1 - d) * M;  // x = last row
+            nufft_setpts(plan, M, row[0], row[1], row[2], s);
+            nufft_execute(plan, cw.p, psf.p, s);
+            HASTY_HIP_CHECK(hipStreamSynchronize(s));
+        } catch (...) {
+            (void)hipStreamSynchronize(s);
+            nufft_destroy(plan);
+            throw;
+        }
         nufft_destroy(plan);
-        throw;
     }
-    nufft_destroy(plan);
+    arena.reset(after_psf);
 
     const double inv_grid = 1.0 / (double)ngrid;
     DevBuf work(sizeof(double2) * ngrid);

@@ -14,8 +14,11 @@ namespace hasty_hip {
 //    2^d that turns the reference's Toeplitz scale into SenseNormal's.
 // coords: [ndim][M] (float or double), nmodes: image dims (slowest first), weights: [M]
 // real or null. Either output may be null.
+// Everything the build allocates comes from the workspace while it lasts.
 void toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, const int64_t* nmodes,
-                    const float* weights, float2* diag_ref, float* kernel, double tol, hipStream_t s);
+                    const float* weights, float2* diag_ref, float* kernel, double tol, hipStream_t s,
+                    void* workspace = nullptr, size_t workspace_bytes = 0);
+size_t toeplitz_workspace_bytes(int64_t M, int ndim, const int64_t* nmodes, double tol);
 
 // CUDANormalNufftToeplitz::apply* (nufft.cpp:1163-1197) on a complex diagonal:
 //   res = ifftn(fftn(in, s=2N) * diag)[:N]; mode 0: out = res, 1: out += res,

@@ -11,6 +11,20 @@ namespace hasty {
 
 namespace detail {
 
+void check(int rc);
+
+// hasty_toeplitz_build with its device memory from torch's caching allocator.
+void toeplitz_build(const at::Tensor& coords, const std::vector<int64_t>& img, const float* weights, void* diag,
+                    float* kernel, double tol)
+{
+    if (!coords.is_cuda()) throw std::runtime_error("Coordinates did not reside in cuda device");
+    const size_t bytes = hasty_toeplitz_workspace_size(coords.size(1), (int)img.size(), img.data(), tol);
+    at::Tensor ws = at::empty({(int64_t)bytes}, coords.options().dtype(at::kByte));
+    check(hasty_toeplitz_build_ws(coords.data_ptr(), coords.scalar_type() == at::kDouble ? 1 : 0, coords.size(1),
+                                  (int)img.size(), img.data(), weights, diag, kernel, tol, ws.data_ptr(), bytes,
+                                  (void*)c10::hip::getCurrentHIPStream().stream()));
+}
+
 void check(int rc)
 {
     if (rc != 0) throw std::runtime_error(hasty_last_error());
@@ -199,9 +213,7 @@ void CUDANormalNufftToeplitz::build_diagonal(const at::Tensor& coords, std::vect
     int64_t per = 1;
     for (size_t i = 1; i < ns.size(); ++i) per *= ns[i];
     at::Tensor d0 = diagonal.select(0, 0);
-    check(hasty_toeplitz_build(coords.data_ptr(), coords.scalar_type() == at::ScalarType::Double ? 1 : 0,
-                               coords.size(1), (int)img.size(), img.data(), nullptr, d0.data_ptr(), nullptr, 1e-10,
-                               detail::stream()));
+    detail::toeplitz_build(coords, img, nullptr, d0.data_ptr(), nullptr, 1e-10);
     for (int64_t t = 1; t < ns[0]; ++t) diagonal.select(0, t).copy_(d0);
     (void)per;
 }
@@ -504,9 +516,8 @@ CUDASenseNormalToeplitz::CUDASenseNormalToeplitz(const std::vector<at::Tensor>& 
         if (co.size(0) != 3) throw std::runtime_error("coords must be [3, M]");
         at::Tensor w;
         if (weights.has_value()) w = (*weights)[i].to(dev, at::kFloat).contiguous();
-        check(hasty_toeplitz_build(co.data_ptr(), co.scalar_type() == at::kDouble ? 1 : 0, co.size(1), 3,
-                                   nmodes.data(), w.defined() ? w.data_ptr<float>() : nullptr, nullptr,
-                                   natural[i].data_ptr<float>(), 1e-8, detail::stream()));
+        detail::toeplitz_build(co, nmodes, w.defined() ? w.data_ptr<float>() : nullptr, nullptr,
+                               natural[i].data_ptr<float>(), 1e-8);
     }
     _kernels = at::empty_like(natural);
     check(hasty_sense_normal_prepare(natural.data_ptr<float>(), _kernels.data_ptr<float>(), natural.size(0),

@@ -68,6 +68,14 @@ int hasty_nufft_info(hasty_nufft_plan plan, int64_t* nf, int* ns, double* beta);
 int hasty_toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, const int64_t* nmodes,
                          const float* weights, void* diag_ref, float* kernel, double tol, void* stream);
 
+/* The same with the build's device memory (grids, point lists) given by the caller:
+ * workspace of hasty_toeplitz_workspace_size bytes (0 for invalid arguments), or less (the
+ * rest is allocated and freed inside). It is free again when the call returns. */
+size_t hasty_toeplitz_workspace_size(int64_t M, int ndim, const int64_t* nmodes, double tol);
+int hasty_toeplitz_build_ws(const void* coords, int coord_fp64, int64_t M, int ndim, const int64_t* nmodes,
+                            const float* weights, void* diag_ref, float* kernel, double tol, void* workspace,
+                            size_t workspace_bytes, void* stream);
+
 /* Replaces CUDANormalNufftToeplitz::apply / apply_add / apply_addcmul / apply_inplace
  * (nufft.cpp:1163-1197): res = ifftn(fftn(in, s=2N) * diag)[:N];
  * mode 0: out = res; 1: out += res; 2: out += res * mul; 3: out = res (out may be in).

@@ -182,3 +182,34 @@ def test_precision_cg_l2_regularised(cg_setup):
     print(f"\nCG 15 it on A + {lam:.4g} I (0.1 lambda_max): device vs FP64 CG {e:.3e}", flush=True)
     assert e < 1e-5
     assert torch.equal(x, xg)
+
+
+@pytest.mark.parametrize("dims,M", [((20, 24, 30), 3000), ((64, 64, 64), 0), ((9, 30), 500), ((18,), 40)])
+@pytest.mark.parametrize("fp64,weighted", [(False, True), (True, False)])
+def test_toeplitz_build_workspace(dims, M, fp64, weighted):
+    """The kernel and the diagonal do not depend on where the build's memory comes from: the
+    caller's whole workspace, a part of it (unaligned), or none."""
+    import torch
+
+    from hastycompute_amd import _capi as C
+
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(M + len(dims))
+    co = ((torch.rand((len(dims), M), dtype=torch.float64, device="cuda:0", generator=gen) * 2 - 1) * 3.1415926)
+    co = co if fp64 else co.to(torch.float32)
+    w = torch.rand(M, dtype=torch.float32, device="cuda:0", generator=gen) if weighted else None
+    L = [2 * n for n in dims]
+    size = int(C.lib().hasty_toeplitz_workspace_size(M, len(dims), C.i64arr(dims), 1e-10))
+    assert size > 0
+    ws = torch.empty(size + 8, dtype=torch.uint8, device="cuda:0")
+    outs = []
+    for off, nbytes in ((0, size), (8, size), (8, size // 3), (0, 100), (0, 0)):
+        d = torch.empty(L, dtype=torch.complex64, device="cuda:0")
+        k = torch.empty(L, dtype=torch.float32, device="cuda:0")
+        C.call("hasty_toeplitz_build_ws", co.data_ptr(), int(fp64), M, len(dims), C.i64arr(dims), C.ptr(w), d.data_ptr(),
+               k.data_ptr(), 1e-10, ws.data_ptr() + off, nbytes, C.stream_ptr())
+        outs.append((d, k))
+    scale = float(outs[-1][1].abs().max()) + 1e-30
+    for d, k in outs[:-1]:  # tile spreaders add in another order from run to run: 1e-13, below float32
+        assert float((k - outs[-1][1]).abs().max()) <= 1e-7 * scale
+        assert torch.allclose(d, outs[-1][0], rtol=1e-6, atol=1e-6 * float(outs[-1][0].abs().max()))

@@ -486,6 +486,267 @@ template <int R> void launch_r16(const AxisKernelArgs<float>& args, int64_t bloc
         hipLaunchKernelGGL((axis_fft_r16_kernel<R, 1>), dim3((unsigned)blocks), dim3(threads), 0, stream, args);
 }
 
+// ---- lines of the lengths below as two register steps ----------------------------------
+//
+// The Stockham passes of a line, grouped in two: step A runs the first radices (product
+// RA) on x[n2 + RB m] in the thread that owns n2, step B the others (product RB = L / RA)
+// on the RB values k1 + RA n2 in the thread that owns k1; the line crosses LDS once between
+// them (three times with a convolution) instead of once per pass and once each for load and
+// store. 16 lines per workgroup; lanes run over the lines when these are adjacent in
+// memory, else over a line's elements. The radices, their order, the twiddles and every
+// rounding are those of axis_fft_kernel, so a pass gives the same bits on either kernel.
+// 72 x 100 x 90, 4 coils: K2 (90 -> 200-point lines) 60 -> 39 us, the convolution of
+// 144-point lines 189 -> 74 us, each K5 launch 28 -> 15 us; the type-2 passes of that size
+// 16 / 27 / 46 -> 11 / 15 / 23 us (2.7 TB/s of their reads and writes).
+
+// The value as a store to LDS would leave it (the compiler may not contract the product it
+// comes from into a later sum).
+__device__ __forceinline__ float2 rounded(float2 v)
+{
+    asm volatile("" : "+v"(v.x), "+v"(v.y));
+    return v;
+}
+// x w (S < 0) or x conj(w), with the products that are rounded before the sum spelled out
+template <int S> __device__ __forceinline__ float2 twiddled(float2 x, float2 w)
+{
+    if (S < 0) return float2{fmaf(x.x, w.x, -(x.y * w.y)), fmaf(x.x, w.y, x.y * w.x)};
+    return float2{fmaf(x.x, w.x, x.y * w.y), fmaf(x.y, w.x, -(x.x * w.y))};
+}
+
+template <int... Rad> struct RadixList {
+    static constexpr int product = (1 * ... * Rad);
+};
+
+// One Stockham pass of radix RAD over N values in registers (NS values already combined);
+// tw(r, k) is the twiddle of input r in the butterflies of index k.
+template <int RAD, int S, int N, int NS, typename Tw> __device__ __forceinline__ void reg_pass(float2 (&v)[N], Tw tw)
+{
+    float2 w[N];
+#pragma unroll
+    for (int j = 0; j < N / RAD; ++j) {
+        const int k = j % NS;
+        float2 u[RAD];
+        u[0] = v[j];
+#pragma unroll
+        for (int r = 1; r < RAD; ++r) u[r] = tw(v[j + r * (N / RAD)], r, k);
+        Dft<RAD, S, float2, float>::run(u);
+#pragma unroll
+        for (int r = 0; r < RAD; ++r) w[(j / NS) * NS * RAD + k + r * NS] = rounded(u[r]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = w[i];
+}
+
+// Step A of an L-point line: twiddle indices are compile-time constants (scalar loads).
+template <int L, int S, int N, int NS> __device__ __forceinline__ void step_a(float2 (&)[N], const float2*, RadixList<>) {}
+template <int L, int S, int N, int NS, int RAD, int... Rest>
+__device__ __forceinline__ void step_a(float2 (&v)[N], const float2* tw, RadixList<RAD, Rest...>)
+{
+    reg_pass<RAD, S, N, NS>(v, [&](float2 x, int r, int k) {
+        return k == 0 ? x : twiddled<S>(x, tw[r * k * (L / (NS * RAD))]);
+    });
+    step_a<L, S, N, NS * RAD>(v, tw, RadixList<Rest...>{});
+}
+// Step B: RA values are combined already and this thread owns k1 of them.
+template <int L, int S, int RA, int N, int NS>
+__device__ __forceinline__ void step_b(float2 (&)[N], const float2*, int, RadixList<>)
+{
+}
+template <int L, int S, int RA, int N, int NS, int RAD, int... Rest>
+__device__ __forceinline__ void step_b(float2 (&v)[N], const float2* tw, int k1, RadixList<RAD, Rest...>)
+{
+    reg_pass<RAD, S, N, NS>(v, [&](float2 x, int r, int k) {
+        return twiddled<S>(x, tw[r * (k1 + RA * k) * (L / (RA * NS * RAD))]);
+    });
+    step_b<L, S, RA, N, NS * RAD>(v, tw, k1, RadixList<Rest...>{});
+}
+
+constexpr int kLineThreads = 256;
+constexpr int kLinesPer = 16;
+
+// MODE 0: FFT of sign S; MODE 1: convolution with a real kernel.
+template <class A, class B, int MODE, int S>
+__global__ void __launch_bounds__(kLineThreads) line_fft_kernel(AxisKernelArgs<float> args)
+{
+    constexpr int RA = A::product, RB = B::product, L = RA * RB, LN = kLinesPer, PITCH = LN + 1;
+    constexpr int TA = (LN * RB + kLineThreads - 1) / kLineThreads;  // tasks per thread
+    constexpr int TB = (LN * RA + kLineThreads - 1) / kLineThreads;
+    __shared__ float2 buf[L * PITCH];  // element e of line l at e * PITCH + l
+    __shared__ float2 tws[L];
+    __shared__ int64_t base[5][LN];  // in, mul, out, omul, conv
+    const AxisFft<float>& a = args.a;
+    const int tid = threadIdx.x;
+    const int64_t l0 = (int64_t)blockIdx.x * LN;
+    const int nb = (int)min((int64_t)LN, a.nlines - l0);
+    if (tid < nb) {
+        const int64_t l = l0 + tid;
+        base[0][tid] = line_base(a.ain, l);
+        base[2][tid] = line_base(a.aout, l);
+        if (a.inmul) base[1][tid] = line_base(a.amul, l);
+        if (a.outmul) base[3][tid] = line_base(a.aomul, l);
+        if (MODE == 1) base[4][tid] = line_base(a.aconv, l);
+    }
+    for (int k = tid; k < L; k += kLineThreads) tws[k] = args.tw[k];
+    __syncthreads();
+    const bool in_fast = a.ain.stride != 1, out_fast = a.aout.stride != 1;
+    // task of a thread -> (line, index of `per`), lanes over the lines or over the indices
+    auto split = [&](int task, int per, bool lines_fast, int& line, int& idx) {
+        line = lines_fast ? task % LN : task / per;
+        idx = lines_fast ? task / LN : task - line * per;
+    };
+    constexpr int S1 = MODE == 0 ? S : -1;
+#pragma unroll
+    for (int t = 0; t < TA; ++t) {
+        const int task = tid + t * kLineThreads;
+        if (task >= LN * RB) break;
+        int line, n2;
+        split(task, RB, in_fast, line, n2);
+        float2 v[RA];
+#pragma unroll
+        for (int m = 0; m < RA; ++m) {
+            const int n = in_element(n2 + RB * m, L, a.n_in, a.in_centered);
+            float2 x = float2{0.f, 0.f};
+            if (n >= 0 && line < nb) {
+                x = a.in[base[0][line] + (int64_t)n * a.ain.stride];
+                if (a.inmul) {
+                    const float2 f = a.inmul[base[1][line] + (int64_t)n * a.amul.stride];
+                    x = a.inmul_conj ? cmulc(f, x) : cmul(f, x);
+                }
+                if (a.pre_scale) x = cscale(x, a.pre_scale[n]);
+            }
+            v[m] = rounded(x);
+        }
+        step_a<L, S1, RA, 1>(v, args.tw, A{});
+#pragma unroll
+        for (int k1 = 0; k1 < RA; ++k1) buf[(n2 * RA + k1) * PITCH + line] = v[k1];
+    }
+    __syncthreads();
+    if constexpr (MODE == 1) {
+        // forward step B, the kernel; its results lie where its inputs were
+#pragma unroll
+        for (int t = 0; t < TB; ++t) {
+            const int task = tid + t * kLineThreads;
+            if (task >= LN * RA) break;
+            int line, k1;
+            split(task, RA, in_fast, line, k1);
+            float2 v[RB];
+#pragma unroll
+            for (int n2 = 0; n2 < RB; ++n2) v[n2] = buf[(n2 * RA + k1) * PITCH + line];
+            step_b<L, -1, RA, RB, 1>(v, tws, k1, B{});
+#pragma unroll
+            for (int k2 = 0; k2 < RB; ++k2) {
+                const int k = k1 + RA * k2;
+                const float f = line < nb ? a.conv_real[base[4][line] + (int64_t)k * a.aconv.stride] : 0.f;
+                buf[k * PITCH + line] = cscale(v[k2], f);
+            }
+        }
+        __syncthreads();
+        // inverse step A: every read before the first write
+        float2 v[TA][RA];
+#pragma unroll
+        for (int t = 0; t < TA; ++t) {
+            const int task = min(tid + t * kLineThreads, LN * RB - 1);
+            int line, n2;
+            split(task, RB, in_fast, line, n2);
+#pragma unroll
+            for (int m = 0; m < RA; ++m) v[t][m] = buf[(n2 + RB * m) * PITCH + line];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TA; ++t) {
+            const int task = tid + t * kLineThreads;
+            if (task >= LN * RB) break;
+            int line, n2;
+            split(task, RB, in_fast, line, n2);
+            step_a<L, 1, RA, 1>(v[t], args.tw, A{});
+#pragma unroll
+            for (int k1 = 0; k1 < RA; ++k1) buf[(n2 * RA + k1) * PITCH + line] = v[t][k1];
+        }
+        __syncthreads();
+    }
+    constexpr int S2 = MODE == 0 ? S : 1;
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        const int task = tid + t * kLineThreads;
+        if (task >= LN * RA) break;
+        int line, k1;
+        split(task, RA, out_fast, line, k1);
+        float2 v[RB];
+#pragma unroll
+        for (int n2 = 0; n2 < RB; ++n2) v[n2] = buf[(n2 * RA + k1) * PITCH + line];
+        step_b<L, S2, RA, RB, 1>(v, tws, k1, B{});
+        if (line >= nb) continue;
+        const int64_t bo = base[2][line];
+#pragma unroll
+        for (int k2 = 0; k2 < RB; ++k2) {
+            const int k = k1 + RA * k2;
+            int n = k;
+            if (a.out_centered) {
+                n = k + a.n_out / 2;  // inverse of k = (n - n_out / 2) mod L
+                if (n >= L) n -= L;
+            }
+            if (n >= a.n_out) continue;
+            float2 y = cscale(v[k2], a.scale);
+            if (a.post_scale) y = cscale(y, a.post_scale[n]);
+            if (a.outmul) {
+                const float2 f = a.outmul[base[3][line] + (int64_t)n * a.aomul.stride];
+                y = a.outmul_conj ? cmulc(f, y) : cmul(f, y);
+            }
+            const int64_t addr = bo + (int64_t)n * a.aout.stride;
+            if (a.accumulate) y = cadd(a.out[addr], y);
+            a.out[addr] = y;
+        }
+    }
+}
+
+template <class A, class B> void launch_line(const AxisKernelArgs<float>& args, int mode, hipStream_t s)
+{
+    const unsigned blocks = (unsigned)ceil_div(args.a.nlines, kLinesPer);
+    if (mode == 1)
+        hipLaunchKernelGGL((line_fft_kernel<A, B, 1, -1>), dim3(blocks), dim3(kLineThreads), 0, s, args);
+    else if (args.a.sign < 0)
+        hipLaunchKernelGGL((line_fft_kernel<A, B, 0, -1>), dim3(blocks), dim3(kLineThreads), 0, s, args);
+    else
+        hipLaunchKernelGGL((line_fft_kernel<A, B, 0, 1>), dim3(blocks), dim3(kLineThreads), 0, s, args);
+    check_launch("line_fft_kernel");
+}
+
+// The even 2,3,5-smooth lengths of 48 .. 320 other than 54 and 50 (doubled images of 24 ..
+// 160); false for others. Radices in the order of make_radix_plan; the split keeps both
+// steps within 40 values per thread.
+bool run_line_fft(const AxisKernelArgs<float>& args, int mode, hipStream_t s)
+{
+    switch (args.a.L) {
+    case 48: launch_line<RadixList<8>, RadixList<2, 3>>(args, mode, s); return true;
+    case 60: launch_line<RadixList<4, 3>, RadixList<5>>(args, mode, s); return true;
+    case 64: launch_line<RadixList<8>, RadixList<8>>(args, mode, s); return true;
+    case 72: launch_line<RadixList<8>, RadixList<3, 3>>(args, mode, s); return true;
+    case 80: launch_line<RadixList<8>, RadixList<2, 5>>(args, mode, s); return true;
+    case 90: launch_line<RadixList<2, 3>, RadixList<3, 5>>(args, mode, s); return true;
+    case 96: launch_line<RadixList<8>, RadixList<4, 3>>(args, mode, s); return true;
+    case 100: launch_line<RadixList<4, 5>, RadixList<5>>(args, mode, s); return true;
+    case 108: launch_line<RadixList<4, 3>, RadixList<3, 3>>(args, mode, s); return true;
+    case 120: launch_line<RadixList<8>, RadixList<3, 5>>(args, mode, s); return true;
+    case 128: launch_line<RadixList<8>, RadixList<8, 2>>(args, mode, s); return true;
+    case 144: launch_line<RadixList<8, 2>, RadixList<3, 3>>(args, mode, s); return true;
+    case 150: launch_line<RadixList<2, 3>, RadixList<5, 5>>(args, mode, s); return true;
+    case 160: launch_line<RadixList<8>, RadixList<4, 5>>(args, mode, s); return true;
+    case 162: launch_line<RadixList<2, 3, 3>, RadixList<3, 3>>(args, mode, s); return true;
+    case 180: launch_line<RadixList<4, 3>, RadixList<3, 5>>(args, mode, s); return true;
+    case 192: launch_line<RadixList<8>, RadixList<8, 3>>(args, mode, s); return true;
+    case 200: launch_line<RadixList<8>, RadixList<5, 5>>(args, mode, s); return true;
+    case 216: launch_line<RadixList<8, 3>, RadixList<3, 3>>(args, mode, s); return true;
+    case 240: launch_line<RadixList<8, 2>, RadixList<3, 5>>(args, mode, s); return true;
+    case 250: launch_line<RadixList<2, 5>, RadixList<5, 5>>(args, mode, s); return true;
+    case 256: launch_line<RadixList<8>, RadixList<8, 4>>(args, mode, s); return true;
+    case 270: launch_line<RadixList<2, 3, 3>, RadixList<3, 5>>(args, mode, s); return true;
+    case 288: launch_line<RadixList<8, 4>, RadixList<3, 3>>(args, mode, s); return true;
+    case 300: launch_line<RadixList<4, 3>, RadixList<5, 5>>(args, mode, s); return true;
+    case 320: launch_line<RadixList<8>, RadixList<8, 5>>(args, mode, s); return true;
+    default: return false;
+    }
+}
+
 RadixPlan make_radix_plan(int L)
 {
     RadixPlan p;
@@ -606,6 +867,12 @@ template <typename R> void run_axis_fft(const AxisFft<R>& a, hipStream_t stream)
             }
             check_launch("axis_fft_r16_kernel");
             return;
+        }
+    }
+    if constexpr (std::is_same<R, float>::value) {
+        if (g_r16.load() && mode <= 1) {
+            HASTY_REQUIRE(ceil_div(a.nlines, kLinesPer) < (1ll << 31), "too many FFT lines for one launch");
+            if (run_line_fft(args, mode, stream)) return;
         }
     }
     if (mode == 0) {

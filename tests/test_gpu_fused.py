@@ -259,3 +259,35 @@ def test_z_convolution_lengths(N, n0, narrow):
         for out in outs:
             err = float(torch.linalg.vector_norm(out[p] - ref) / torch.linalg.vector_norm(ref))
             assert err < 1.8e-6, err
+
+
+@pytest.mark.parametrize("n", [24, 30, 32, 36, 40, 45, 48, 50, 54, 60, 64, 72, 75, 80, 81, 90, 96, 100, 108, 120, 125,
+                               128, 135, 144, 150, 160])
+def test_register_lines_equal_lds_passes(N, n):
+    """Generic normal operator (multiplied, plain, convolved and accumulated passes; each
+    axis in turn as the long one; line counts that are no multiple of a bundle): the
+    two-step register lines give the LDS passes' bits. Lengths 128, 192, 256 and 320 also
+    have a four-step form for the plain passes, with its own roundings: there 15 levels
+    there and back bound the distance, 2e-6."""
+    from hastycompute_amd import _capi
+
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(n)
+    for dims in ([n, 10, 15], [10, n, 15], [10, 15, n]):
+        smaps = torch.randn([3] + dims, dtype=torch.complex64, device="cuda:0", generator=gen)
+        kern = torch.rand([2 * d for d in dims], dtype=torch.float32, device="cuda:0", generator=gen)
+        x = torch.randn([2] + dims, dtype=torch.complex64, device="cuda:0", generator=gen)
+        op = N.SenseNormalToeplitz(smaps, kern, coil_batch=2, fused=False)
+        prev = _capi.get_option("fft_r16")
+        outs = []
+        try:
+            for v in (0, 1):
+                _capi.set_option("fft_r16", v)
+                outs.append(op.apply(x, sub=x))
+        finally:
+            _capi.set_option("fft_r16", prev)
+        if 2 * n in (128, 192, 256, 320):
+            err = float(torch.linalg.vector_norm(outs[0] - outs[1]) / torch.linalg.vector_norm(outs[0]))
+            assert err < 2e-6, err
+        else:
+            assert torch.equal(outs[0], outs[1])

@@ -36,9 +36,10 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
 ]
-# Per-file additions. nufft.hip: the spreader's MFMA sums stay in VGPRs; in AGPRs they were
-# copied there and back around every skipped tile (8 moves per 2 MFMAs).
-FILE_FLAGS = {"nufft.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# Per-file additions. MFMA sums stay in VGPRs: in AGPRs nufft.hip's spreader copied them there
+# and back around every skipped tile (8 moves per 2 MFMAs), and llr.hip's Gram kernel around
+# the additions of every tile.
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("llr.hip", "nufft.hip")}
 
 
 def _run(cmd):

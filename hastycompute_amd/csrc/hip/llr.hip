@@ -6,8 +6,9 @@
 // thresholded through its Gram matrix: G = A^H A = V diag(s^2) V^H, and
 //     U diag(s') V^H = A V diag(s'/s) V^H = A W,   W = V diag(g) V^H,
 // with g = max(s - lambda, 0)/s (soft) or 1 for the `rank` largest s (hard).
-//   1. gram:  MFMA 16x16x4 f32 (FP32 accumulate), upper triangle of G, rows split over
-//             workgroups into partial Grams summed in a fixed order (deterministic);
+//   1. gram:  MFMA 16x16x32 bf16 on float32 values split in three (FP32 accumulate), upper
+//             triangle of G, rows split over workgroups into partial Grams summed in a fixed
+//             order (deterministic);
 //   2. eig:   cyclic complex Jacobi in FP32 on the upper triangle in LDS, parallel
 //             (round-robin) ordering, rotations recorded; the eigenvectors that survive
 //             the threshold are rebuilt from them, then W = V diag(g) V^H;
@@ -32,7 +33,7 @@ constexpr int kThreads = 256;
 // it until the padded block slots and the waves meeting at each barrier cost more than
 // they save. 100 frames, 343 blocks: 256 threads 1.16 ms, 512 1.04 ms, 1024 1.40 ms.
 std::atomic<int> g_eig_threads{512};
-constexpr int kMaxTilesPerWave = 9;  // F <= 128 -> 8x8 tiles -> 36 upper tiles / 4 waves
+constexpr int kSmallGroups = 3;      // Gram with up to so many groups of 16 frames: one wave, all tiles
 constexpr int kMaxSweeps = 15;       // Jacobi sweeps per block (4-6 reach FP32 rounding)
 std::atomic<int> g_max_sweeps{kMaxSweeps};  // cap in force (option "llr_max_sweeps")
 
@@ -48,20 +49,6 @@ __device__ __forceinline__ int64_t row_addr(const LlrGeom& g, int3 c, int64_t r)
     return (e * xyz + (int64_t)(c.x + ix) * g.Y * g.Z + (int64_t)(c.y + iy) * g.Z + (c.z + iz)) * g.rstride;
 }
 
-// Partial Gram G = A^H A over rows [split * rows_per_split, ...) of each block.
-//
-// No LDS and no barriers: each wave streams every 16-row slab of the split and owns a
-// fixed set of upper 16x16 tiles of G (tile t = wave + 4 k, as compile-time lists). A
-// slab is loaded straight into the v_mfma_f32_16x16x4f32 operand layout: lane (m, kg)
-// holds A[row][16 t + m] for the four rows 4 kg + ks (ks = 0..3) of frame group t; the
-// same registers are the A operand (conjugated through the product below) of the tiles
-// in row group t and the B operand of those in column group t. Row order inside a slab
-// does not matter for A^H A, so each lane takes four consecutive rows (one row address).
-// The four waves of a workgroup read the same slab (cache hits after the first); the
-// next slab is loaded while the current one's MFMAs run. conj(a) b takes three real
-// MFMAs: P1 = ar br, P2 = ai bi, P3 = (ar - ai)(br + bi); Re = P1 + P2, Im = P3 - P1 + P2.
-// Frames past F read frame F - 1 (they only feed entries of G beyond F, which nothing
-// reads); rows past the split's end are zero.
 // row_addr for r < 2^31 (checked on the host) with 32-bit division.
 __device__ __forceinline__ int64_t row_addr32(const LlrGeom& g, int3 c, uint32_t r)
 {
@@ -73,7 +60,170 @@ __device__ __forceinline__ int64_t row_addr32(const LlrGeom& g, int3 c, uint32_t
             (c.z + (int)iz)) * g.rstride;
 }
 
-__host__ __device__ constexpr int tile_ti(int t, int nt)
+// A block lies inside the image: corners handed over on the device are not seen by the
+// host, so the kernels skip a block that does not (its Gram is zero, its rows untouched).
+__device__ __forceinline__ bool block_inside(const LlrGeom& g, int3 c)
+{
+    return c.x >= 0 && c.y >= 0 && c.z >= 0 && c.x + g.bx <= g.X && c.y + g.by <= g.Y && c.z + g.bz <= g.Z;
+}
+
+// Partial Gram G = A^H A over rows [split * rows_per_split, ...) of each block, on the
+// bf16 matrix units at float32 precision.
+//
+// Every float is the exact sum of three bf16 numbers (high, middle, low: 8 bits each, each
+// the nearest to what is left), and of the nine products of two such sums the six that
+// reach 2^-24 of the whole are taken: l h, h l, m m, m h, h m, h h, each exact in the
+// float32 the unit adds in. One v_mfma_f32_16x16x32_bf16 takes 32 rows in half the time
+// that v_mfma_f32_16x16x4_f32 takes 4, so the six cost 3/8 of the float32 products. The
+// sums of 32 rows start from zero and are added to the running Gram once, so that one
+// rounds at its size per 32 rows (one per 4 rows before): the error of an entry against 64
+// bits, over the norms of its two columns, is 1/4 to 2/5 of that of the float32 units
+// (4096 rows: 1.6e-7 against 4.1e-7 on the diagonal, 3e-9 against 1.2e-8 off it).
+//
+// Lane (m, q) of a fragment holds rows 8 q .. 8 q + 7 of a 32-row slab for frame 16 t + m;
+// the same registers are the A operand of the tiles in row group t and the B operand of
+// those in column group t, and the order of the rows in a slab does not matter for A^H A.
+// conj(a) b takes four real products (the sums of the three-product form would have to be
+// split as well).
+//
+// More than 3 frame groups (gram_kernel): each of the eight waves of a workgroup loads and
+// splits one frame group, they share the fragments through LDS (6 NT kB, two workgroups
+// per CU), and each owns a fixed run of upper 16 x 16 tiles along the rows of tiles; the
+// next slab is loaded during the products. Up to 3
+// groups (gram_small_kernel): a wave keeps all tiles and takes every fourth slab, without
+// LDS or barriers, and the four waves' sums are added at the end in a fixed order.
+//
+// Frames past F read frame F - 1 (they only feed entries of G beyond F, which nothing
+// reads); rows past the split's end are zero.
+// 343 blocks of 4096 x 100 (1.12 GB read): 1.06 -> 0.56 ms; 168 blocks of 8640 x 20 (0.23
+// GB): 267 -> 112 us. Bounds: 0.22 and 0.05 ms of reads, 0.19 ms of bf16 products.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// x = p[0] + p[1] + p[2], eight values at a time
+__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[3])
+{
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        p[0][i] = (__bf16)x[i];
+        r[i] = x[i] - (float)p[0][i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        p[1][i] = (__bf16)r[i];
+        p[2][i] = (__bf16)(r[i] - (float)p[1][i]);
+    }
+}
+
+// A frame group's fragment of one slab: real and imaginary part, three bf16 each.
+struct GramFrag {
+    bf16x8 re[3], im[3];
+};
+
+// Pairs of rows can be read as one 16-byte word: contiguous rows, and no pair split over
+// two lines or off a 16-byte boundary.
+__device__ __forceinline__ bool gram_pairs(const float2* data, const LlrGeom& g, int3 c)
+{
+    return g.rstride == 1 && ((g.bz | g.Z | g.fstride | c.z) & 1) == 0 && (reinterpret_cast<uintptr_t>(data) & 15) == 0;
+}
+
+// Rows rr .. rr + 7 of NF frames (16 t + the lane's, up to the last), one (STEP = 1) or two
+// (STEP = 2) per load; returns how many of the rows exist, the others hold some row of the
+// block. One division chain finds the first row; the next ones follow it along the line
+// and from line to line.
+template <int NF, int STEP>
+__device__ __forceinline__ int load_rows(const float2* __restrict__ data, const LlrGeom& g, int3 c, int64_t rr,
+                                         int64_t r_begin, int64_t r_end, int frame0, float2 (&v)[NF][8])
+{
+    const int ok = (int)max((int64_t)0, min((int64_t)8, r_end - rr));
+    const uint32_t r = (uint32_t)(ok > 0 ? rr : r_begin);
+    const uint32_t bz = (uint32_t)g.bz, by = (uint32_t)g.by, bx = (uint32_t)g.bx;
+    const uint32_t q = r / bz, q2 = q / by;
+    uint32_t iz = r - q * bz, iy = q - q2 * by, ix = q2 % bx;
+    const int64_t base = row_addr32(g, c, r);
+    int64_t at[8];
+    if (__all(ok == 8 && iz + 7 < bz)) {  // every lane's rows lie in one line
+#pragma unroll
+        for (int i = 0; i < 8; i += STEP) at[i] = base + i * g.rstride;
+    } else {
+        const int64_t dz = (g.Z - g.bz) * g.rstride, dy = (g.Y - g.by) * g.Z * g.rstride,
+                      dx = (g.X - g.bx) * g.Y * g.Z * g.rstride;
+        int64_t a = base;
+#pragma unroll
+        for (int i = 0; i < 8; i += STEP) {
+            if (i > 0) {
+                iz += STEP;
+                a += STEP * g.rstride;
+                if (iz >= bz) {
+                    iz = 0;
+                    a += dz;
+                    if (++iy == by) {
+                        iy = 0;
+                        a += dy;
+                        if (++ix == bx) {
+                            ix = 0;
+                            a += dx;
+                        }
+                    }
+                }
+            }
+            at[i] = i < ok ? a : base;
+        }
+    }
+    const int last = (int)g.F - 1;
+#pragma unroll
+    for (int t = 0; t < NF; ++t) {
+        const float2* d = data + (int64_t)min(frame0 + 16 * t, last) * g.fstride;
+#pragma unroll
+        for (int i = 0; i < 8; i += STEP) {
+            if constexpr (STEP == 2) {
+                const float4 w = *reinterpret_cast<const float4*>(d + at[i]);
+                v[t][i] = float2{w.x, w.y};
+                v[t][i + 1] = float2{w.z, w.w};
+            } else {
+                v[t][i] = d[at[i]];
+            }
+        }
+    }
+    return ok;
+}
+
+__device__ __forceinline__ void split_lane(const float2 (&v)[8], int ok, GramFrag& f)
+{
+    float re[8], im[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        re[i] = i < ok ? v[i].x : 0.f;
+        im[i] = i < ok ? v[i].y : 0.f;
+    }
+    split8(re, f.re);
+    split8(im, f.im);
+}
+
+__device__ __forceinline__ void gram_products(const bf16x8 (&a)[3], const bf16x8 (&b)[3], floatx4& t)
+{
+    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], t, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], t, 0, 0, 0);
+}
+
+// conj(a) b of one slab, added to the tile's Gram
+__device__ __forceinline__ void gram_tile(const GramFrag& a, const GramFrag& b, floatx4& re, floatx4& im)
+{
+    floatx4 tr = floatx4{0.f, 0.f, 0.f, 0.f}, t1 = tr, t2 = tr;
+    gram_products(a.re, b.re, tr);
+    gram_products(a.re, b.im, t1);
+    gram_products(a.im, b.re, t2);
+    gram_products(a.im, b.im, tr);
+    re += tr;
+    im += t1 - t2;
+}
+
+// Tile t of the upper triangle of NT x NT, rows in turn.
+__host__ __device__ constexpr int tile_row(int t, int nt)
 {
     int i = 0;
     while (t >= nt - i) {
@@ -82,7 +232,7 @@ __host__ __device__ constexpr int tile_ti(int t, int nt)
     }
     return i;
 }
-__host__ __device__ constexpr int tile_tj(int t, int nt)
+__host__ __device__ constexpr int tile_col(int t, int nt)
 {
     int i = 0;
     while (t >= nt - i) {
@@ -91,147 +241,224 @@ __host__ __device__ constexpr int tile_tj(int t, int nt)
     }
     return i + t;
 }
-
-// MFMAs of tiles K.. of a wave's list for one slab; the tile's frame groups are
-// constant expressions, so the operands stay in registers.
-template <int NT, int WAVE, int K, int NTW> struct GramTiles {
-    __device__ __forceinline__ static void mfma(const float2 (&a)[NT][4], floatx4* p1, floatx4* p2, floatx4* p3)
-    {
-        constexpr int t = WAVE + 4 * K;
-        constexpr int ti = tile_ti(t, NT), tj = tile_tj(t, NT);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const float2 x = a[ti][ks], y = a[tj][ks];
-            p1[K] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y.x, p1[K], 0, 0, 0);
-            p2[K] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y.y, p2[K], 0, 0, 0);
-            p3[K] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x - x.y, y.x + y.y, p3[K], 0, 0, 0);
-        }
-        GramTiles<NT, WAVE, K + 1, NTW>::mfma(a, p1, p2, p3);
-    }
-};
-template <int NT, int WAVE, int NTW> struct GramTiles<NT, WAVE, NTW, NTW> {
-    __device__ __forceinline__ static void mfma(const float2 (&)[NT][4], floatx4*, floatx4*, floatx4*) {}
-};
-
-// A block lies inside the image: corners handed over on the device are not seen by the
-// host, so the kernels skip a block that does not (its Gram is zero, its rows untouched).
-__device__ __forceinline__ bool block_inside(const LlrGeom& g, int3 c)
+// The first tile of a wave's run. Waves w and w + 4 share a SIMD: an even number of tiles
+// is dealt so that both together own the same number, to one.
+constexpr int kGramThreads = 512;
+__host__ __device__ constexpr int gram_first(int wave, int nt)
 {
-    return c.x >= 0 && c.y >= 0 && c.z >= 0 && c.x + g.bx <= g.X && c.y + g.by <= g.Y && c.z + g.bz <= g.Z;
+    const int n = nt * (nt + 1) / 2;
+    return wave <= 4 || (n & 1) ? wave * n / 8 : n - (8 - wave) * n / 8;
+}
+__host__ __device__ constexpr int gram_run(int nt)  // the longest run
+{
+    int m = 0;
+    for (int w = 0; w < 8; ++w) m = gram_first(w + 1, nt) - gram_first(w, nt) > m ? gram_first(w + 1, nt) - gram_first(w, nt) : m;
+    return m;
 }
 
-template <int NT, int WAVE>
-__device__ __forceinline__ void gram_wave(const float2* __restrict__ data, const LlrGeom& g, int3 c, int64_t r_begin,
-                                          int64_t r_end, float2* __restrict__ G)
+// acc: [2 k] real, [2 k + 1] imaginary part of tile k of the run
+__device__ __forceinline__ void store_gram_tile(float2* G, int Fp, int ti, int tj, const floatx4& re, const floatx4& im)
 {
-    constexpr int Fp = 16 * NT;
-    constexpr int NTILE = NT * (NT + 1) / 2;
-    constexpr int NTW = NTILE > WAVE ? (NTILE - WAVE + 3) / 4 : 0;
-    if constexpr (NTW > 0) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int i = ti * 16 + 4 * (lane >> 4) + v;
+        const int j = tj * 16 + (lane & 15);
+        G[(int64_t)i * Fp + j] = float2{re[v], im[v]};
+        if (ti != tj) G[(int64_t)j * Fp + i] = float2{re[v], -im[v]};
+    }
+}
+
+// Tiles T .. END - 1 of a wave that starts at tile BEGIN, with the operands of tile T - 1 at hand.
+template <int NT, int BEGIN, int T, int END> struct GramRun {
+    static constexpr int ti = tile_row(T, NT), tj = tile_col(T, NT);
+    __device__ __forceinline__ static void load(const bf16x8 (*sfr)[64], bf16x8 (&f)[3])
+    {
         const int lane = threadIdx.x & 63;
-        const int m = lane & 15, kg = lane >> 4;
-        const int F = (int)g.F;
-        floatx4 p1[NTW], p2[NTW], p3[NTW];
 #pragma unroll
-        for (int k = 0; k < NTW; ++k) {
-            p1[k] = floatx4{0.f, 0.f, 0.f, 0.f};
-            p2[k] = floatx4{0.f, 0.f, 0.f, 0.f};
-            p3[k] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-        auto load_slab = [&](int64_t r0, float2 (&a)[NT][4]) {
-            int64_t fs = g.fstride;
-            int fm = F - 1;
-            asm volatile("" : "+s"(fs), "+s"(fm));  // opaque per slab: nothing is hoisted out of the slab loop
-            // the lane's rows rr0 .. rr0 + 3: one address when they lie in one z-line
-            const int64_t rr0 = r0 + 4 * kg;
-            int64_t addr[4];
-            bool ok[4];
-            if (rr0 + 3 < r_end && (uint32_t)rr0 % (uint32_t)g.bz + 3 < (uint32_t)g.bz) {
-                const int64_t base = row_addr32(g, c, (uint32_t)rr0);
-                if (g.rstride == 1 && ((base | fs) & 1) == 0) {
-                    // four consecutive complex values per frame, 16-byte aligned: two 16-byte loads
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        const float2* p = data + base + (int64_t)min(16 * t + m, fm) * fs;
-                        const float4 v0 = *reinterpret_cast<const float4*>(p);
-                        const float4 v1 = *reinterpret_cast<const float4*>(p + 2);
-                        a[t][0] = float2{v0.x, v0.y};
-                        a[t][1] = float2{v0.z, v0.w};
-                        a[t][2] = float2{v1.x, v1.y};
-                        a[t][3] = float2{v1.z, v1.w};
-                    }
-                    return;
-                }
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    addr[ks] = base + ks * g.rstride;
-                    ok[ks] = true;
-                }
+        for (int p = 0; p < 3; ++p) f[p] = sfr[p][lane];
+    }
+    // The column operand is read one part (real, imaginary) at a time, and nothing is read
+    // ahead across these barriers: four waves per SIMD fit without spills and cover the
+    // waits. (A spill of a prefetched row waits for it: 1.10 ms where 128 registers did not do.)
+    __device__ __forceinline__ static void slab(const bf16x8 (*sfr)[6][64], GramFrag a, floatx4* acc)
+    {
+        if constexpr (T < END) {
+            constexpr int pi = T > BEGIN ? tile_row(T > 0 ? T - 1 : 0, NT) : -1;
+            if constexpr (ti != pi) {
+                load(sfr[ti], a.re);
+                load(sfr[ti] + 3, a.im);
+            }
+            floatx4 tr = floatx4{0.f, 0.f, 0.f, 0.f}, t1 = tr, t2 = tr;
+            if constexpr (ti == tj) {
+                gram_products(a.re, a.re, tr);
+                gram_products(a.im, a.re, t2);
+                gram_products(a.re, a.im, t1);
+                gram_products(a.im, a.im, tr);
             } else {
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    ok[ks] = rr0 + ks < r_end;
-                    addr[ks] = row_addr32(g, c, (uint32_t)(ok[ks] ? rr0 + ks : r_begin));
-                }
+                bf16x8 b[3];
+                load(sfr[tj], b);
+                gram_products(a.re, b, tr);
+                gram_products(a.im, b, t2);
+                __builtin_amdgcn_sched_barrier(0);
+                load(sfr[tj] + 3, b);
+                gram_products(a.re, b, t1);
+                gram_products(a.im, b, tr);
             }
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const float2 v = data[addr[ks] + (int64_t)min(16 * t + m, fm) * fs];
-                    a[t][ks] = ok[ks] ? v : float2{0.f, 0.f};
-                }
-            }
-        };
-        auto mfma_slab = [&](const float2 (&a)[NT][4]) { GramTiles<NT, WAVE, 0, NTW>::mfma(a, p1, p2, p3); };
-        float2 a0[NT][4], a1[NT][4];
-        int64_t r0 = r_begin;
-        if (r0 < r_end) load_slab(r0, a0);
-        while (r0 < r_end) {
-            if (r0 + 16 < r_end) load_slab(r0 + 16, a1);
-            mfma_slab(a0);
-            r0 += 16;
-            if (r0 >= r_end) break;
-            if (r0 + 16 < r_end) load_slab(r0 + 16, a0);
-            mfma_slab(a1);
-            r0 += 16;
+            acc[2 * (T - BEGIN)] += tr;
+            acc[2 * (T - BEGIN) + 1] += t1 - t2;
+            // added here, not after the waves' paths join (tr, t1, t2 of all tiles kept)
+            asm volatile("" : "+v"(acc[2 * (T - BEGIN)]), "+v"(acc[2 * (T - BEGIN) + 1]));
+            __builtin_amdgcn_sched_barrier(0);
+            GramRun<NT, BEGIN, T + 1, END>::slab(sfr, a, acc);
         }
-#pragma unroll
-        for (int k = 0; k < NTW; ++k) {
-            const int t = WAVE + 4 * k;
-            const int ti = tile_ti(t, NT), tj = tile_tj(t, NT);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = ti * 16 + 4 * kg + v;
-                const int j = tj * 16 + m;
-                const float re = p1[k][v] + p2[k][v];
-                const float im = p3[k][v] - p1[k][v] + p2[k][v];
-                G[(int64_t)i * Fp + j] = float2{re, im};
-                if (ti != tj) G[(int64_t)j * Fp + i] = float2{re, -im};
+    }
+    __device__ __forceinline__ static void store(float2* G, const floatx4* acc)
+    {
+        if constexpr (T < END) {
+            store_gram_tile(G, 16 * NT, ti, tj, acc[2 * (T - BEGIN)], acc[2 * (T - BEGIN) + 1]);
+            GramRun<NT, BEGIN, T + 1, END>::store(G, acc);
+        }
+    }
+};
+template <int NT, int WAVE>
+using GramWave = GramRun<NT, gram_first(WAVE, NT), gram_first(WAVE, NT), gram_first(WAVE + 1, NT)>;
+
+template <int NT, int STEP>
+__device__ __forceinline__ void gram_slabs(const float2* __restrict__ data, const LlrGeom& g, int3 c, int wave,
+                                           int64_t r_begin, int64_t r_end, int slabs, bf16x8 (*sfr)[6][64], floatx4* acc)
+{
+    const int lane = threadIdx.x & 63;
+    // slab n - 1 is multiplied while slab n is on its way
+    for (int n = 0; n <= slabs; ++n) {
+        float2 v[1][8];
+        int ok = 0;
+        if (wave < NT && n < slabs)
+            ok = load_rows<1, STEP>(data, g, c, r_begin + 32 * n + 8 * (lane >> 4), r_begin, r_end,
+                                    16 * wave + (lane & 15), v);
+        if (n > 0) {
+            GramFrag a;
+            switch (wave) {
+            case 0: GramWave<NT, 0>::slab(sfr, a, acc); break;
+            case 1: GramWave<NT, 1>::slab(sfr, a, acc); break;
+            case 2: GramWave<NT, 2>::slab(sfr, a, acc); break;
+            case 3: GramWave<NT, 3>::slab(sfr, a, acc); break;
+            case 4: GramWave<NT, 4>::slab(sfr, a, acc); break;
+            case 5: GramWave<NT, 5>::slab(sfr, a, acc); break;
+            case 6: GramWave<NT, 6>::slab(sfr, a, acc); break;
+            default: GramWave<NT, 7>::slab(sfr, a, acc); break;
             }
         }
+        if (n == slabs) break;
+        __syncthreads();  // the last slab's fragments are read
+        if (wave < NT) {
+            GramFrag f;
+            split_lane(v[0], ok, f);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                sfr[wave][p][lane] = f.re[p];
+                sfr[wave][3 + p][lane] = f.im[p];
+            }
+        }
+        __syncthreads();
     }
 }
 
 template <int NT>
-__global__ void __launch_bounds__(kThreads) gram_kernel(const float2* __restrict__ data, LlrGeom g, const int3* corners,
+__global__ void __launch_bounds__(kGramThreads, NT < 8 ? 4 : 2) gram_kernel(const float2* __restrict__ data, LlrGeom g, const int3* corners,
                                                        int64_t rows_per_split, float2* __restrict__ gpart)
 {
-    constexpr int Fp = 16 * NT;
+    __shared__ bf16x8 sfr[NT][6][64];
     const int blk = blockIdx.x;
     const int split = blockIdx.y;
-    const int nsplit = gridDim.y;
     const int3 c = corners[blk];
     const int64_t R = g.E * g.bx * g.by * g.bz;
     const int64_t r_begin = split * rows_per_split;
     // a block outside the image gets an empty row range: its partial Gram is zero
     const int64_t r_end = block_inside(g, c) ? min(R, r_begin + rows_per_split) : r_begin;
-    float2* G = gpart + ((int64_t)blk * nsplit + split) * Fp * Fp;
-    switch (threadIdx.x >> 6) {
-    case 0: gram_wave<NT, 0>(data, g, c, r_begin, r_end, G); break;
-    case 1: gram_wave<NT, 1>(data, g, c, r_begin, r_end, G); break;
-    case 2: gram_wave<NT, 2>(data, g, c, r_begin, r_end, G); break;
-    default: gram_wave<NT, 3>(data, g, c, r_begin, r_end, G); break;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    floatx4 acc[2 * gram_run(NT)];
+#pragma unroll
+    for (int k = 0; k < 2 * gram_run(NT); ++k) acc[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int slabs = (int)((max(r_end - r_begin, (int64_t)0) + 31) / 32);
+    if (gram_pairs(data, g, c)) gram_slabs<NT, 2>(data, g, c, wave, r_begin, r_end, slabs, sfr, acc);
+    else gram_slabs<NT, 1>(data, g, c, wave, r_begin, r_end, slabs, sfr, acc);
+    float2* G = gpart + ((int64_t)blk * gridDim.y + split) * (16 * NT) * (16 * NT);
+    switch (wave) {
+    case 0: GramWave<NT, 0>::store(G, acc); break;
+    case 1: GramWave<NT, 1>::store(G, acc); break;
+    case 2: GramWave<NT, 2>::store(G, acc); break;
+    case 3: GramWave<NT, 3>::store(G, acc); break;
+    case 4: GramWave<NT, 4>::store(G, acc); break;
+    case 5: GramWave<NT, 5>::store(G, acc); break;
+    case 6: GramWave<NT, 6>::store(G, acc); break;
+    default: GramWave<NT, 7>::store(G, acc); break;
+    }
+}
+
+template <int NT, int STEP>
+__device__ __forceinline__ void gram_small_slabs(const float2* __restrict__ data, const LlrGeom& g, int3 c, int wave,
+                                                 int64_t r_begin, int64_t r_end, floatx4* acc)
+{
+    const int lane = threadIdx.x & 63;
+    int64_t r0 = r_begin + 32 * wave;
+    if (r0 >= r_end) return;
+    float2 v[NT][8];
+    auto load = [&](int64_t r) {
+        return load_rows<NT, STEP>(data, g, c, r + 8 * (lane >> 4), r_begin, r_end, lane & 15, v);
+    };
+    int ok = load(r0);
+    for (; r0 < r_end; r0 += 32 * (kThreads / 64)) {
+        GramFrag f[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) split_lane(v[t], ok, f[t]);
+        const int64_t next = r0 + 32 * (kThreads / 64);
+        if (next < r_end) ok = load(next);
+#pragma unroll
+        for (int ti = 0, k = 0; ti < NT; ++ti)
+#pragma unroll
+            for (int tj = ti; tj < NT; ++tj, ++k) gram_tile(f[ti], f[tj], acc[2 * k], acc[2 * k + 1]);
+    }
+}
+
+template <int NT>
+__global__ void __launch_bounds__(kThreads) gram_small_kernel(const float2* __restrict__ data, LlrGeom g,
+                                                              const int3* corners, int64_t rows_per_split,
+                                                              float2* __restrict__ gpart)
+{
+    constexpr int NTILE = NT * (NT + 1) / 2;
+    constexpr int kWaves = kThreads / 64;
+    __shared__ floatx4 part[2][2 * NTILE][64];
+    const int blk = blockIdx.x;
+    const int split = blockIdx.y;
+    const int3 c = corners[blk];
+    const int64_t R = g.E * g.bx * g.by * g.bz;
+    const int64_t r_begin = split * rows_per_split;
+    const int64_t r_end = block_inside(g, c) ? min(R, r_begin + rows_per_split) : r_begin;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    floatx4 acc[2 * NTILE];
+#pragma unroll
+    for (int k = 0; k < 2 * NTILE; ++k) acc[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (gram_pairs(data, g, c)) gram_small_slabs<NT, 2>(data, g, c, wave, r_begin, r_end, acc);
+    else gram_small_slabs<NT, 1>(data, g, c, wave, r_begin, r_end, acc);
+    // (wave 0 + wave 2) + (wave 1 + wave 3)
+    for (int h = kWaves / 2; h > 0; h /= 2) {
+        if (wave >= h && wave < 2 * h)
+#pragma unroll
+            for (int k = 0; k < 2 * NTILE; ++k) part[wave - h][k][lane] = acc[k];
+        __syncthreads();
+        if (wave < h)
+#pragma unroll
+            for (int k = 0; k < 2 * NTILE; ++k) acc[k] += part[wave][k][lane];
+        __syncthreads();
+    }
+    if (wave == 0) {
+        float2* G = gpart + ((int64_t)blk * gridDim.y + split) * (16 * NT) * (16 * NT);
+#pragma unroll
+        for (int ti = 0, k = 0; ti < NT; ++ti)
+#pragma unroll
+            for (int tj = ti; tj < NT; ++tj, ++k) store_gram_tile(G, 16 * NT, ti, tj, acc[2 * k], acc[2 * k + 1]);
     }
 }
 
@@ -239,8 +466,12 @@ template <int NT>
 void launch_gram(const float2* data, const LlrGeom& g, const int3* corners, int64_t nblk, int nsplit, int64_t rps,
                  float2* gpart, hipStream_t s)
 {
-    hipLaunchKernelGGL(gram_kernel<NT>, dim3((unsigned)nblk, (unsigned)nsplit), dim3(kThreads), 0, s, data, g,
-                       corners, rps, gpart);
+    if constexpr (NT <= kSmallGroups)
+        hipLaunchKernelGGL(gram_small_kernel<NT>, dim3((unsigned)nblk, (unsigned)nsplit), dim3(kThreads), 0, s, data,
+                           g, corners, rps, gpart);
+    else
+        hipLaunchKernelGGL(gram_kernel<NT>, dim3((unsigned)nblk, (unsigned)nsplit), dim3(kGramThreads), 0, s, data,
+                           g, corners, rps, gpart);
     check_launch("gram_kernel");
 }
 
@@ -869,7 +1100,7 @@ void llr_blocks(float2* data, const LlrGeom& g, const int3* corners_dev, int64_t
     float2* gpart = reinterpret_cast<float2*>(ws);
     float2* W = gpart + (int64_t)nblk * nsplit * Fp * Fp;
     float4* rot = reinterpret_cast<float4*>(W + (int64_t)nblk * Fp * Fp);
-    int64_t rps = ceil_div(ceil_div(R, nsplit), 16) * 16;
+    int64_t rps = ceil_div(ceil_div(R, nsplit), 32) * 32;
     {
         KernelTimer t("llr_gram", s);
         const float2* d = data;

@@ -525,6 +525,45 @@ def test_llr_normal_blocks_vs_oracle(N, F, E, X, blk, it, soft, rel):
     assert e < 1e-4
 
 
+@pytest.mark.parametrize("F,E,dims,blk,corners", [
+    (1, 1, (9, 8, 16), (5, 4, 3), [(0, 0, 0), (4, 4, 13)]),       # one frame; lines of 3, odd corner
+    (16, 1, (8, 9, 15), (3, 7, 5), [(1, 2, 4), (5, 0, 10)]),      # whole group, odd lines
+    (17, 2, (13, 8, 20), (6, 4, 7), [(0, 1, 3), (7, 4, 12)]),     # first remainder, two encodes
+    (32, 1, (8, 16, 24), (8, 8, 8), [(0, 0, 0), (0, 8, 16)]),
+    (33, 5, (12, 12, 24), (12, 12, 12), [(0, 0, 0), (0, 0, 12)]),  # lines end inside a lane's rows
+    (48, 1, (9, 11, 14), (4, 5, 6), [(0, 0, 1), (4, 6, 8)]),
+    (49, 1, (16, 16, 34), (16, 16, 16), [(0, 0, 1), (0, 0, 18)]),  # first shared size; odd corner
+    (64, 2, (11, 7, 12), (5, 7, 10), [(0, 0, 2), (6, 0, 0)]),
+    (80, 1, (12, 12, 13), (6, 12, 13), [(0, 0, 0), (6, 0, 0)]),
+    (97, 1, (9, 9, 40), (9, 9, 9), [(0, 0, 0), (0, 0, 31)]),
+    (113, 1, (16, 16, 16), (8, 16, 16), [(0, 0, 0), (8, 0, 0)]),
+    (128, 3, (8, 8, 24), (8, 8, 12), [(0, 0, 0), (0, 0, 12)]),
+])
+def test_llr_gram_shapes(N, F, E, dims, blk, corners):
+    """Frame groups of both Gram kernels and the ways a lane's eight rows can lie in the image."""
+    rng = np.random.default_rng(F)
+    r = min(3, F)
+    n = int(np.prod(dims))
+    x = (rnd(rng, (F, r)) @ rnd(rng, (r, E * n)) / math.sqrt(r) + 0.05 * rnd(rng, (F, E * n))).reshape(F, E, *dims)
+    x = x.astype(np.complex64)
+    xg = g(x)
+    N.llr_blocks(xg, blk, corners, r, False)
+    got = h(xg)
+    ref = x.astype(np.complex128)
+    outside = np.ones(x.shape, bool)
+    for c in corners:
+        A = O.extract_block(ref, c, blk)
+        B = O.svt_hard(A, r)
+        s2 = np.append(np.linalg.svd(A, compute_uv=False), 0.0) ** 2
+        # projector on r directions: the Gram's relative error, (R / 32 + 12) 2^-24 (one
+        # rounding of the sum per 32 rows, 12 inside), and the Jacobi sweeps' stop, 1e-5,
+        # over the relative gap; twice for the rounding of W and of A W
+        tol = 2 * ((A.shape[0] / 32 + 12) * 2.0**-24 + 1e-5) * s2[0] / (s2[r - 1] - s2[r])
+        assert O.rel_l2(O.extract_block(got, c, blk), B) < tol, c
+        outside[(slice(None), slice(None)) + tuple(slice(a, a + b) for a, b in zip(c, blk))] = False
+    assert np.array_equal(got[outside], x[outside])
+
+
 @pytest.mark.parametrize("F,soft", [(100, True), (20, False)])
 def test_llr_repeatable(N, F, soft):
     """The LLR prox is deterministic: partial Grams are summed in a fixed order, the

@@ -12,7 +12,8 @@
 //   2. eig:   cyclic complex Jacobi in FP32 on the upper triangle in LDS, parallel
 //             (round-robin) ordering, rotations recorded; the eigenvectors that survive
 //             the threshold are rebuilt from them, then W = V diag(g) V^H;
-//   3. apply: MFMA A <- A W in place, 16-row slabs staged through LDS.
+//   3. apply: MFMA A <- A W in place by 16-row slabs, or A <- (A V) (diag(g) V^H) where few
+//             singular values survive.
 // Blocks are read and written directly in the image; no gather/scatter copies.
 #include <atomic>
 #include <algorithm>
@@ -37,19 +38,7 @@ constexpr int kSmallGroups = 3;      // Gram with up to so many groups of 16 fra
 constexpr int kMaxSweeps = 15;       // Jacobi sweeps per block (4-6 reach FP32 rounding)
 std::atomic<int> g_max_sweeps{kMaxSweeps};  // cap in force (option "llr_max_sweeps")
 
-__device__ __forceinline__ int64_t row_addr(const LlrGeom& g, int3 c, int64_t r)
-{
-    const int iz = (int)(r % g.bz);
-    int64_t t = r / g.bz;
-    const int iy = (int)(t % g.by);
-    t /= g.by;
-    const int ix = (int)(t % g.bx);
-    const int64_t e = t / g.bx;
-    const int64_t xyz = g.X * g.Y * g.Z;
-    return (e * xyz + (int64_t)(c.x + ix) * g.Y * g.Z + (int64_t)(c.y + iy) * g.Z + (c.z + iz)) * g.rstride;
-}
-
-// row_addr for r < 2^31 (checked on the host) with 32-bit division.
+// Offset of row r of a block, r < 2^31 (checked on the host).
 __device__ __forceinline__ int64_t row_addr32(const LlrGeom& g, int3 c, uint32_t r)
 {
     const uint32_t bz = (uint32_t)g.bz, by = (uint32_t)g.by, bx = (uint32_t)g.bx;
@@ -96,7 +85,7 @@ __device__ __forceinline__ bool block_inside(const LlrGeom& g, int3 c)
 // Frames past F read frame F - 1 (they only feed entries of G beyond F, which nothing
 // reads); rows past the split's end are zero.
 // 343 blocks of 4096 x 100 (1.12 GB read): 1.06 -> 0.56 ms; 168 blocks of 8640 x 20 (0.23
-// GB): 267 -> 112 us. Bounds: 0.22 and 0.05 ms of reads, 0.19 ms of bf16 products.
+// GB): 267 -> 105 us. Bounds: 0.22 and 0.05 ms of reads, 0.19 ms of bf16 products.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // x = p[0] + p[1] + p[2], eight values at a time
@@ -573,6 +562,21 @@ __device__ __forceinline__ int moved_loc(int s, int t, int h, int nb1)
     return (idx << 1) | (s2 > t2 ? 1 : 0);
 }
 
+// Groups of 16 kept vectors r for which A <- (A V) (diag(g) V^H) takes fewer matrix
+// instructions than A <- A W, 3 r (K4 + 4 NT) against 3 K4 NT per 16 rows (K4 = ceil(F / 4),
+// NT = ceil(F / 16)); 0 where A W does not: more than 32 vectors, fewer than 33 frames, or
+// 17 .. 32 vectors of fewer than 65. Then the block's W holds the kept vectors v_k as
+// rows and g_k conj(v_k) below them, 16 r rows each, and the first of its rotations,
+// which are dead by then, holds r. 343 blocks of 4096 rows, A W and
+// this: 100 frames, 5 kept 1.03 and 0.55 ms (2.25 GB of traffic), 24 kept 1.04 and 0.72;
+// 72 frames, 24 kept 0.63 and 0.51; 48 and 36 frames, 8 kept 0.26 and 0.22, 0.21 and 0.17.
+__host__ __device__ inline int low_groups(int nk, int F)
+{
+    const int nt = (F + 15) / 16, k4 = (F + 3) / 4;
+    const int r = nk > 16 ? (nk + 15) / 16 : 1;
+    return r <= 2 && r * (k4 + 4 * nt) < k4 * nt && 16 * r <= (F + 1) / 2 ? r : 0;
+}
+
 // Jacobi eigensolver + W = V diag(g) V^H, one workgroup per block.
 //
 // G (n = F rounded up to even) lives in LDS in slot order as upper 2x2 blocks; thread
@@ -796,6 +800,7 @@ __global__ void __launch_bounds__(NTH) eig_w_kernel(const float2* __restrict__ g
     float2* W = Wout + (int64_t)blk * Fp * Fp;
     const int R = sweeps * (n - 1);
     const int cap = half;
+    const int low = low_groups(nk, F);  // 16 low <= cap: all kept vectors are in X at once
     for (int c0 = 0; c0 < max(nk, 1); c0 += cap) {
         const int nkc = min(cap, nk - c0);
         for (int e = tid; e < nkc * n; e += NTH) {
@@ -847,6 +852,20 @@ __global__ void __launch_bounds__(NTH) eig_w_kernel(const float2* __restrict__ g
             }
         }
         __syncthreads();
+        if (low > 0) {
+            for (int e = tid; e < 16 * low * Fp; e += NTH) {
+                const int k = e / Fp, j = e - (e / Fp) * Fp;
+                float2 v = float2{0.f, 0.f};
+                float gv = 0.f;
+                if (k < nk && j < F) {
+                    v = X[k * n + j];
+                    gv = gk[kl[k]];
+                }
+                W[e] = v;
+                W[16 * low * Fp + e] = float2{gv * v.x, -gv * v.y};
+            }
+            break;
+        }
         // W (+)= sum_v g_v X_v X_v^H
         for (int e = tid; e < Fp * Fp; e += NTH) {
             const int i = e / Fp, j = e - (e / Fp) * Fp;
@@ -864,6 +883,7 @@ __global__ void __launch_bounds__(NTH) eig_w_kernel(const float2* __restrict__ g
         }
         __syncthreads();
     }
+    if (tid == 0) rot[0].x = __int_as_float(low);  // every replay is over
 }
 
 // A <- A W for rows [chunk*rows_per_wg, ...) of each block, in place in the image.
@@ -884,10 +904,114 @@ constexpr int kApplySlabsPerWave = 4;
 // MFMA operand reads fall in disjoint bank groups.
 __host__ __device__ inline int apply_stride(int Fp) { return ((Fp / 16) % 2 == 0) ? Fp + 16 : Fp; }
 
+// LDS row stride of the two factors (complex elements): the operands of either product
+// (16 rows of 4 elements, 4 rows of 16) fall in all banks.
+__host__ __device__ constexpr int low_stride(int Fp) { return Fp + 4; }
+
+// A <- (A V) (diag(g) V^H) for 16 RT vectors, laid out as the full product below: the first
+// product leaves (A V)^T with vector 4 kg + v and row n in lane (n, kg), which is the second
+// one's operand if its step v takes vectors 4 kg + v. A slab's values are done with after the
+// first product, so the next slab's loads run behind the second and the stores.
+template <int NT, int RT>
+__device__ __forceinline__ void apply_low(float2* __restrict__ data, const LlrGeom& g, int3 c, int64_t r_begin,
+                                          int64_t r_end, const float2* __restrict__ W, float2* __restrict__ sF)
+{
+    constexpr int Fp = 16 * NT;
+    constexpr int KS = 4 * NT;
+    constexpr int S = low_stride(Fp);
+    const int F = (int)g.F;
+    const int K4 = (F + 3) / 4;
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int n = lane & 15, kg = lane >> 4;
+    for (int e = threadIdx.x; e < 32 * RT * Fp; e += kApplyThreads) {
+        const int k = e / Fp, j = e - (e / Fp) * Fp;
+        sF[k * S + j] = W[e];
+    }
+    __syncthreads();
+    const float2* sV = sF + n * S + kg;                            // v_n[kg]
+    const float2* sG = sF + 16 * RT * S + 4 * kg * S + n;          // g_k conj(v_k)[n], k = 4 kg
+    const int waves = kApplyThreads / 64;
+    float2 a[KS];
+    int64_t addr = 0;
+    bool valid = false;
+    auto load = [&](int64_t r0) {
+        const int64_t r = r0 + n;
+        valid = r < r_end;
+        addr = row_addr32(g, c, (uint32_t)(valid ? r : r_end - 1));
+        int64_t fs = g.fstride;
+        int fm = F - 1, k4 = K4;
+        asm volatile("" : "+s"(fs), "+s"(fm), "+s"(k4));  // opaque per slab: nothing here is hoisted out of the slab loop
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            a[ks] = ks < k4 ? data[addr + (int64_t)min(4 * ks + kg, fm) * fs] : float2{0.f, 0.f};
+    };
+    int64_t r0 = r_begin + 16 * wave;
+    if (r0 >= r_end) return;  // no barrier follows
+    load(r0);
+    for (; r0 < r_end; r0 += 16 * waves) {
+        floatx4 p1[RT], p2[RT], p3[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) p1[t] = p2[t] = p3[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        int k4 = K4;
+        asm volatile("" : "+s"(k4));
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            if (ks < k4) {
+                const float ar = a[ks].x, ai = a[ks].y;
+#pragma unroll
+                for (int t = 0; t < RT; ++t) {
+                    const float2 w = sV[16 * t * S + 4 * ks];
+                    p1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, ar, p1[t], 0, 0, 0);
+                    p2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, ai, p2[t], 0, 0, 0);
+                    p3[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x + w.y, ar + ai, p3[t], 0, 0, 0);
+                }
+            }
+        }
+        const int64_t at = addr;
+        const bool store = valid;
+        if (r0 + 16 * waves < r_end) load(r0 + 16 * waves);
+        float br[RT][4], bi[RT][4];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                br[t][v] = p1[t][v] - p2[t][v];
+                bi[t][v] = p3[t][v] - p1[t][v] - p2[t][v];
+            }
+        }
+        int64_t fs = g.fstride;
+        asm volatile("" : "+s"(fs));
+        float2* q = data + at + (int64_t)(4 * kg) * fs;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            floatx4 o1 = floatx4{0.f, 0.f, 0.f, 0.f}, o2 = o1, o3 = o1;
+#pragma unroll
+            for (int u = 0; u < 4 * RT; ++u) {
+                const float2 w = sG[(16 * (u >> 2) + (u & 3)) * S + 16 * t];
+                const float xr = br[u >> 2][u & 3], xi = bi[u >> 2][u & 3];
+                o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, xr, o1, 0, 0, 0);
+                o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, xi, o2, 0, 0, 0);
+                o3 = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x + w.y, xr + xi, o3, 0, 0, 0);
+            }
+            // lane holds out[row n][frame 16 t + 4 kg + v]; only the last tile can pass F
+            if (store) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    if (t < NT - 1 || 16 * t + 4 * kg + v < F)
+                        *q = float2{o1[v] - o2[v], o3[v] - o1[v] - o2[v]};
+                    q += v < 3 ? fs : 13 * fs;
+                }
+            }
+        }
+    }
+}
+
 template <int NT>
 __global__ void __launch_bounds__(kApplyThreads) apply_kernel(float2* __restrict__ data, LlrGeom g,
                                                               const int3* corners, int64_t rows_per_wg,
-                                                              const float2* __restrict__ Wall)
+                                                              const float2* __restrict__ Wall,
+                                                              const float4* __restrict__ rot_all, int64_t rot_stride)
 {
     constexpr int Fp = 16 * NT;
     constexpr int KS = 4 * NT;  // k-steps for F = Fp
@@ -908,6 +1032,19 @@ __global__ void __launch_bounds__(kApplyThreads) apply_kernel(float2* __restrict
     const int kg = lane >> 4;  // k within a k-step
 
     const float2* W = Wall + (int64_t)blk * Fp * Fp;
+    if constexpr (NT >= 3) {
+        const int low = __float_as_int(rot_all[blk * rot_stride].x);
+        if (low == 1) {
+            apply_low<NT, 1>(data, g, c, r_begin, r_end, W, sW);
+            return;
+        }
+        if constexpr (NT >= 5) {
+            if (low == 2) {
+                apply_low<NT, 2>(data, g, c, r_begin, r_end, W, sW);
+                return;
+            }
+        }
+    }
     for (int e = threadIdx.x; e < 4 * K4 * Fp; e += kApplyThreads) {
         const int k = e / Fp, j = e - (e / Fp) * Fp;
         sW[k * S + j] = k < F ? W[(int64_t)k * Fp + j] : float2{0.f, 0.f};
@@ -923,7 +1060,7 @@ __global__ void __launch_bounds__(kApplyThreads) apply_kernel(float2* __restrict
     auto slab_row = [&](int64_t r0, int64_t& addr, bool& valid) {
         const int64_t r = r0 + n;
         valid = r < r_end;
-        addr = row_addr(g, c, valid ? r : r_end - 1);
+        addr = row_addr32(g, c, (uint32_t)(valid ? r : r_end - 1));
     };
     auto load_ks = [&](float2* a, int64_t addr, int ks0, int ks1) {
         int64_t fs = g.fstride;
@@ -1016,28 +1153,31 @@ __global__ void __launch_bounds__(kApplyThreads) apply_kernel(float2* __restrict
 size_t apply_smem(int64_t F)
 {
     const int Fp = llr_padded(F);
-    return sizeof(float) * 2 * (size_t)(4 * ((F + 3) / 4)) * apply_stride(Fp);
+    size_t rows = (size_t)(4 * ((F + 3) / 4)) * apply_stride(Fp);
+    for (int r = 1; r <= 2; ++r)
+        if (low_groups(16 * r, (int)F) == r) rows = std::max(rows, (size_t)(32 * r) * low_stride(Fp));
+    return sizeof(float2) * rows;
 }
 
 template <int NT>
 void launch_apply(float2* data, const LlrGeom& g, const int3* corners, int64_t nblk, int64_t rows_per_wg,
-                  int64_t nchunk, const float2* W, hipStream_t s)
+                  int64_t nchunk, const float2* W, const float4* rot, int64_t rot_stride, hipStream_t s)
 {
     const size_t smem = apply_smem(g.F);
     allow_lds(apply_kernel<NT>, smem);
     hipLaunchKernelGGL(apply_kernel<NT>, dim3((unsigned)nblk, (unsigned)nchunk), dim3(kApplyThreads), smem, s, data,
-                       g, corners, rows_per_wg, W);
+                       g, corners, rows_per_wg, W, rot, rot_stride);
     check_launch("apply_kernel");
 }
 
 template <int NTH, int B>
 void launch_eig(const float2* gpart, int nsplit, const LlrGeom& g, int Fp, float thresh, int soft, int rank,
-                float4* rot, float2* W, float* eig_out, int64_t nblk, hipStream_t s)
+                int max_sweeps, float4* rot, float2* W, float* eig_out, int64_t nblk, hipStream_t s)
 {
     const size_t smem = (size_t)EigLayout((int)(g.F + (g.F & 1))).bytes;
     allow_lds(eig_w_kernel<NTH, B>, smem);
     hipLaunchKernelGGL((eig_w_kernel<NTH, B>), dim3((unsigned)nblk), dim3(NTH), smem, s, gpart, nsplit, (int)g.F, Fp,
-                       thresh, soft, rank, g_max_sweeps, rot, W, eig_out);
+                       thresh, soft, rank, max_sweeps, rot, W, eig_out);
     check_launch("eig_w_kernel");
 }
 
@@ -1100,6 +1240,9 @@ void llr_blocks(float2* data, const LlrGeom& g, const int3* corners_dev, int64_t
     float2* gpart = reinterpret_cast<float2*>(ws);
     float2* W = gpart + (int64_t)nblk * nsplit * Fp * Fp;
     float4* rot = reinterpret_cast<float4*>(W + (int64_t)nblk * Fp * Fp);
+    const int n = (int)(g.F + (g.F & 1));
+    const int max_sweeps = g_max_sweeps;
+    const int64_t rot_stride = (int64_t)max_sweeps * (n - 1) * (n / 2);
     int64_t rps = ceil_div(ceil_div(R, nsplit), 32) * 32;
     {
         KernelTimer t("llr_gram", s);
@@ -1117,11 +1260,11 @@ void llr_blocks(float2* data, const LlrGeom& g, const int3* corners_dev, int64_t
     }
     {
         KernelTimer t("llr_eig", s);
-        const int n = (int)(g.F + (g.F & 1));
         const float2* gp = gpart;
         const int nth = g_eig_threads.load();
         const int bpt = eig_blk_per_thread(n, nth);
-#define HASTY_EIG(NTH, B) launch_eig<NTH, B>(gp, nsplit, g, Fp, thresh, soft, rank, rot, W, eig_out, nblk, s)
+#define HASTY_EIG(NTH, B) \
+    launch_eig<NTH, B>(gp, nsplit, g, Fp, thresh, soft, rank, max_sweeps, rot, W, eig_out, nblk, s)
         if (nth == 768) {
             switch (bpt) {
             case 1: HASTY_EIG(768, 1); break;
@@ -1157,16 +1300,19 @@ void llr_blocks(float2* data, const LlrGeom& g, const int3* corners_dev, int64_t
         HASTY_REQUIRE(nchunk < 65536, "LLR block has too many rows for one launch");
         KernelTimer t("llr_apply", s);
         const float2* Wc = W;
+        const float4* rc = rot;
+#define HASTY_APPLY(NT) launch_apply<NT>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, rc, rot_stride, s)
         switch (Fp / 16) {
-        case 1: launch_apply<1>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
-        case 2: launch_apply<2>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
-        case 3: launch_apply<3>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
-        case 4: launch_apply<4>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
-        case 5: launch_apply<5>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
-        case 6: launch_apply<6>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
-        case 7: launch_apply<7>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
-        default: launch_apply<8>(data, g, corners_dev, nblk, rows_per_wg, nchunk, Wc, s); break;
+        case 1: HASTY_APPLY(1); break;
+        case 2: HASTY_APPLY(2); break;
+        case 3: HASTY_APPLY(3); break;
+        case 4: HASTY_APPLY(4); break;
+        case 5: HASTY_APPLY(5); break;
+        case 6: HASTY_APPLY(6); break;
+        case 7: HASTY_APPLY(7); break;
+        default: HASTY_APPLY(8); break;
         }
+#undef HASTY_APPLY
     }
 }
 

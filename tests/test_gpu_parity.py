@@ -564,6 +564,32 @@ def test_llr_gram_shapes(N, F, E, dims, blk, corners):
     assert np.array_equal(got[outside], x[outside])
 
 
+@pytest.mark.parametrize("F,rank,soft", [
+    (32, 3, False), (33, 0, False), (33, 1, True), (33, 16, False), (33, 17, False), (64, 16, True), (64, 17, True),
+    (65, 17, False), (65, 32, True), (65, 33, False), (100, 5, True), (100, 16, False), (100, 32, False),
+    (100, 33, True), (112, 5, False), (113, 32, True), (128, 1, False), (128, 32, False), (128, 33, True)])
+@pytest.mark.parametrize("R", [48, 719])
+def test_llr_kept_vectors(N, F, rank, soft, R):
+    """A V (g V^H) against A W: kept vectors at the edges of the groups of 16, ragged rows."""
+    rng = np.random.default_rng(100 * F + rank)
+    k = min(R, F)
+    rank = min(rank, k - 1)
+    U = np.linalg.qr(rnd(rng, (R, k)))[0]
+    V = np.linalg.qr(rnd(rng, (F, k)))[0]
+    s = np.r_[np.linspace(1.0, 0.8, rank), np.linspace(0.2, 0.1, k - rank)]
+    A = ((U * s) @ V.conj().T).astype(np.complex64)
+    ref = O.svt_soft(A.astype(np.complex128), 0.5) if soft else O.svt_hard(A.astype(np.complex128), rank)
+    Ag = g(A)
+    N.svt_matrix(Ag, 0.5 if soft else rank, soft)
+    got = h(Ag)
+    if rank == 0:
+        assert not got.any()
+        return
+    # the Gram's error and the sweeps' stop, 1e-5 |G|_F, over the gap 0.6 |G|_2 (soft: the
+    # slope of (s - l) / s over the kept vectors is below that); twice for the products
+    assert O.rel_l2(got, ref) < 2 * (1e-5 * math.sqrt(rank) + (R / 32 + 12) * 2.0**-24) / 0.6
+
+
 @pytest.mark.parametrize("F,soft", [(100, True), (20, False)])
 def test_llr_repeatable(N, F, soft):
     """The LLR prox is deterministic: partial Grams are summed in a fixed order, the

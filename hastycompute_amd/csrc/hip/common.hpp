@@ -102,7 +102,9 @@ int current_device();
 // (in order, 256-byte aligned; hipMalloc once it is full) and dev_free leaves that memory
 // alone. For calls that own everything they allocate and have finished with it on their
 // stream when they return; hipMalloc and hipFree of a kernel build's gigabyte cost
-// milliseconds per call, at times tens of them.
+// milliseconds per call, at times tens of them. The workspace may still be in use by work
+// its owner queued on that stream, so whatever is done with the memory is queued there too
+// (no null-stream copies or fills).
 class DeviceArena {
 public:
     DeviceArena(void* base, size_t bytes);

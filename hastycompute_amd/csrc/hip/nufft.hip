@@ -1334,11 +1334,14 @@ std::vector<double> es_deconv(int64_t nf, int ns, double beta, int64_t n)
     return out;
 }
 
-template <typename R> void upload_real(void*& dst, const std::vector<double>& v)
+// Written in the order of stream s: memory of an arena may still be in use by what its
+// owner has queued there, which a copy on the null stream does not wait for.
+template <typename R> void upload_real(void*& dst, const std::vector<double>& v, hipStream_t s)
 {
     std::vector<R> h(v.begin(), v.end());
     dst = dev_alloc(sizeof(R) * h.size());
-    HASTY_HIP_CHECK(hipMemcpy(dst, h.data(), sizeof(R) * h.size(), hipMemcpyHostToDevice));
+    HASTY_HIP_CHECK(hipMemcpyAsync(dst, h.data(), sizeof(R) * h.size(), hipMemcpyHostToDevice, s));
+    HASTY_HIP_CHECK(hipStreamSynchronize(s));  // the host copy goes out of scope
 }
 
 void launch_fill(int* p, int64_t n, int v, hipStream_t s)
@@ -1394,7 +1397,8 @@ template <typename R> void zero_fill(cplx<R>* p, int64_t n, hipStream_t s)
 template void zero_fill<float>(cplx<float>*, int64_t, hipStream_t);
 template void zero_fill<double>(cplx<double>*, int64_t, hipStream_t);
 
-NufftPlan* nufft_makeplan(int type, int dim, const int64_t* nmodes, int iflag, int ntransf, double tol, int fp64)
+NufftPlan* nufft_makeplan(int type, int dim, const int64_t* nmodes, int iflag, int ntransf, double tol, int fp64,
+                          hipStream_t s)
 {
     HASTY_REQUIRE(type == 1 || type == 2, "Only Nufft Type 1 and Type 2 is supported");
     HASTY_REQUIRE(dim >= 1 && dim <= 3, "Dimension must be 1,2 or 3");
@@ -1449,9 +1453,9 @@ NufftPlan* nufft_makeplan(int type, int dim, const int64_t* nmodes, int iflag, i
             if (d == 3 - dim || p->nf[d] != p->nf[d - 1] || p->n[d] != p->n[d - 1])
                 v = es_deconv(p->nf[d], p->ns, p->beta, p->n[d]);
             if (p->fp64)
-                upload_real<double>(p->phiinv[d], v);
+                upload_real<double>(p->phiinv[d], v, s);
             else
-                upload_real<float>(p->phiinv[d], v);
+                upload_real<float>(p->phiinv[d], v, s);
             if (p->fp64)
                 twiddles<double>((int)p->nf[d]);
             else

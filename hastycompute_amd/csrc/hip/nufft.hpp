@@ -67,9 +67,10 @@ struct NufftPlan {
 };
 
 // nmodes in FINUFFT order (fastest-varying first), as the reference passes
-// _nmodes_flipped (lib/fft/nufft.cpp:430-432).
-NufftPlan* nufft_makeplan(int type, int dim, const int64_t* nmodes, int iflag, int ntransf, double tol,
-                          int fp64);
+// _nmodes_flipped (lib/fft/nufft.cpp:430-432). The plan's tables are written on stream s
+// and complete when the call returns.
+NufftPlan* nufft_makeplan(int type, int dim, const int64_t* nmodes, int iflag, int ntransf, double tol, int fp64,
+                          hipStream_t s = nullptr);
 // x pairs with nmodes[0] (fastest), y with nmodes[1], z with nmodes[2].
 void nufft_setpts(NufftPlan* p, int64_t M, const void* x, const void* y, const void* z, hipStream_t s);
 // type 1: c [ntransf][M] -> f [ntransf][modes]; type 2: f -> c.

@@ -176,7 +176,7 @@ void toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, con
         // Type-1 (isign +1) FP64 NUFFT onto the doubled modes: psf[n] = sum_j w_j exp(+i (n - N).x_j).
         int64_t nm_flip[3];
         for (int d = 0; d < ndim; ++d) nm_flip[d] = 2 * nmodes[ndim - 1 - d];
-        NufftPlan* plan = nufft_makeplan(1, ndim, nm_flip, 1, 1, tol, 1);
+        NufftPlan* plan = nufft_makeplan(1, ndim, nm_flip, 1, 1, tol, 1, s);
         try {
             const double* row[3] = {nullptr, nullptr, nullptr};
             for (int d = 0; d < ndim; ++d) row[d] = cdp + (int64_t)(ndim - 1 - d) * M;  // x = last row

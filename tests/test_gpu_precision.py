@@ -213,3 +213,32 @@ def test_toeplitz_build_workspace(dims, M, fp64, weighted):
     for d, k in outs[:-1]:  # tile spreaders add in another order from run to run: 1e-13, below float32
         assert float((k - outs[-1][1]).abs().max()) <= 1e-7 * scale
         assert torch.allclose(d, outs[-1][0], rtol=1e-6, atol=1e-6 * float(outs[-1][0].abs().max()))
+
+
+@pytest.mark.parametrize("dims", [(32, 24, 32), (20, 24, 30)])
+def test_toeplitz_build_waits_for_its_stream(dims):
+    """The workspace may still be in use by what its owner queued on the build's stream (a
+    block that torch's caching allocator hands on): some 30 ms of fills of the workspace are
+    queued before a build on a side stream, which gives the default stream's kernel."""
+    from hastycompute_amd import _capi as C
+
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(5)
+    M = 5000
+    co = (torch.rand((3, M), dtype=torch.float32, device="cuda:0", generator=gen) * 2 - 1) * 3.1415926
+    L = [2 * n for n in dims]
+    size = int(C.lib().hasty_toeplitz_workspace_size(M, 3, C.i64arr(dims), 1e-10))
+    ks = []
+    torch.cuda.synchronize()
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            ws = torch.empty(size, dtype=torch.uint8, device="cuda:0")
+            k = torch.empty(L, dtype=torch.float32, device="cuda:0")
+            for _ in range(1000):
+                ws.fill_(255)  # NaN in every table it would reach
+            C.call("hasty_toeplitz_build_ws", co.data_ptr(), 0, M, 3, C.i64arr(dims), None, None, k.data_ptr(), 1e-10,
+                   ws.data_ptr(), size, C.stream_ptr())
+            ks.append(k)
+        stream.synchronize()
+    # the tile spreader of the second size adds in another order from run to run
+    assert float((ks[1] - ks[0]).abs().max()) <= 1e-7 * float(ks[0].abs().max())

@@ -1428,12 +1428,21 @@ NufftPlan* nufft_makeplan(int type, int dim, const int64_t* nmodes, int iflag, i
         if (dim == 3) {
             const double cells = 8000.0;
             int t = (int)std::floor(std::cbrt(cells) + 1e-9);
-            // interpolation only takes its point order from the tiles: 16^3 ones ran 5-12 %
-            // faster than 20^3 (71 -> 68 us at 128^3, 171 -> 159 us at 160^3, ns = 7)
-            if (type == 2) t = 16;
-            if (g_tile.load() > 0) t = g_tile.load();
-            int b = t - p->ns - 1;
-            b = std::max(2, b);
+            // Interpolation only takes its point order from the tiles: 16^3 ones ran 5-12 %
+            // faster than 20^3 (71 -> 68 us at 128^3, 171 -> 159 us at 160^3, ns = 7). No
+            // halo is staged, so wide kernels keep bins of 8 cells: with 2 (16 - ns - 1 at ns =
+            // 13..16) a complex128 plan of 128^3 at ns = 15 took 2.7 ms and 44 MB for its
+            // two million bins, 0.32 ms and under 1 MB here; interpolation within 4 % of either.
+            int least = 2;
+            if (type == 2) {
+                t = 16;
+                least = 8;
+            }
+            if (g_tile.load() > 0) {
+                t = g_tile.load();
+                least = 2;
+            }
+            const int b = std::max(least, t - p->ns - 1);
             for (int d = 0; d < 3; ++d) p->bs[d] = b;
         } else if (dim == 2) {
             const int b = p->fp64 ? 24 : 32;

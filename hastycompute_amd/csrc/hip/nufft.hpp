@@ -92,7 +92,8 @@ int nufft_get_spread_variant();
 // type-1 plans, 0 for type-2 plans (measured best for spreading and for interpolation).
 void nufft_set_locality(int v);
 int nufft_get_locality();
-// 3-D tile edge including the halo (0: 20 cells) and points per spreader subproblem
+// 3-D tile edge including the halo (0: 20 cells for type-1 plans, 16 and at least 8 without
+// the halo for type-2 plans) and points per spreader subproblem
 // (0: 128 for complex64, 1024 for complex128) of new plans
 void nufft_set_tile(int v);
 int nufft_get_tile();

@@ -143,9 +143,9 @@ int hasty_sense_normal_toeplitz_ex(const void* x, void* out, const void* smaps, 
  *     0 and 2 sixteen (ky, kx) columns per workgroup, 1 and 3 eight.
  *   "llr_max_sweeps" 1..15 (default 15): cap on the Jacobi sweeps of the LLR eigensolver.
  *   "llr_eig_threads" 256, 512 or 768 (default 512): the LLR eigensolver's workgroup.
- *   "nufft_spread_tile" 0 or 12..28 (default 0 = 20 for type-1, 16 for type-2 plans): 3-D
- *     point-binning tile edge in fine-grid cells, halo included, of new plans (a tile
- *     spreader's tile must fit in LDS: 20 for complex128).
+ *   "nufft_spread_tile" 0 or 12..28 (default 0 = 20 for type-1 plans, 16 but bins of at
+ *     least 8 cells for type-2 plans): 3-D point-binning tile edge in fine-grid cells, halo
+ *     included, of new plans (a tile spreader's tile must fit in LDS: 20 for complex128).
  *   "nufft_spread_chunk" 0 or 32..8192 (default 0 = 128 for complex64, 1024 for
  *     complex128): points per spreading workgroup of new plans.
  *   "nufft_spread_variant" 0..6 (default 6): 3-D type-1 spreader; 0 one lane per

@@ -701,6 +701,24 @@ def test_output_spreader_parts_and_widths(N, M, fp64, tol):
     assert err < max(10 * tol, 1e-12 if fp64 else 3e-6), err
 
 
+@pytest.mark.parametrize("tol,ns", [(1e-6, 7), (1e-12, 13), (1e-15, 16)])
+def test_type2_bins_do_not_grow_with_the_kernel(N, tol, ns):
+    """A type-2 plan's bins are an ordering of its points: 8^3 cells or more each at every
+    kernel width, so five int arrays of 32^3 bins for a 256^3 grid (0.7 MB; 42 MB with bins
+    of 2 cells), in the driver's pages of 2 MB."""
+    co = torch.zeros((3, 16), dtype=torch.float64, device="cuda:0")
+    N.NufftPlan(co, [128, 128, 128], 2, 1, 1, tol).close()  # tables that outlive a plan
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    plan = N.NufftPlan(co, [128, 128, 128], 2, 1, 1, tol)
+    used = free0 - torch.cuda.mem_get_info()[0]
+    nf, width, _ = plan.info()
+    plan.close()
+    assert width == ns and nf == [256, 256, 256]
+    grids = 16 * 256 * 256 * (256 + 128)
+    assert used - grids < 12 * 2**21, used - grids
+
+
 @pytest.mark.parametrize("dims", [(24, 24, 24), (9, 30, 17), (4, 5, 90)])
 @pytest.mark.parametrize("fp64,tol", [(False, 1e-1), (False, 1e-2), (False, 1e-3), (False, 1e-5), (False, 1e-6),
                                       (False, 1e-8), (True, 1e-6), (True, 1e-9), (True, 1e-14)])

@@ -62,7 +62,7 @@ def parse():
     ap.add_argument("--zconv-variant", type=int, default=None,
                     help="z-convolution bundles at N0 = 128 and 160 (library option sense_zconv_variant, 0..3)")
     ap.add_argument("--zconv-batch", type=int, default=None,
-                    help="problems per z-convolution launch at N0 = 128 (library option sense_zconv_batch, 1..16)")
+                    help="problems per z-convolution launch at 2 N0 = 64 k <= 320 (library option sense_zconv_batch, 1..16)")
     ap.add_argument("--cg-iters", type=int, default=15)
     ap.add_argument("--no-cg", action="store_true")
     ap.add_argument("--plain", type=int, default=3, help="problems solved by the plain per-frame path (0: skip)")

@@ -1777,7 +1777,7 @@ namespace {
 // with the inverse fed by direct-to-LDS loads. The kernel permutation follows the
 // variant, so it is set before kernels are prepared.
 std::atomic<int> g_xy_variant{2};
-std::atomic<int> g_zconv_batch{16};  // problems per z-convolution launch (N0 = 128), 1..16
+std::atomic<int> g_zconv_batch{16};  // problems per register z-convolution launch, 1..16
 // z-convolution bundles at N0 = 128 and 160: 0, 2 (default) 16 columns, 1, 3 8 columns
 // (half-used 128-byte lines: 3.6 ms where 16 take 1.66 ms, 128^3 x 16 coils x 4 problems)
 std::atomic<int> g_zconv_variant{2};
@@ -1791,6 +1791,9 @@ int sense_fused_get_xy_variant() { return g_xy_variant; }
 int sense_fused_get_zconv_batch() { return g_zconv_batch; }
 void sense_fused_set_zconv_variant(int v) { g_zconv_variant = v; }
 int sense_fused_get_zconv_variant() { return g_zconv_variant; }
+
+// The register z-convolutions take several problems per launch.
+bool sense_fused_zconv_batched(const int64_t* n3) { return 2 * n3[0] % 64 == 0 && 2 * n3[0] <= 320; }
 
 // The z-convolution has register forms for 2 N0 = 64 k (k <= 5); other
 // lengths use z_conv_kernel, which holds two 32-column blocks of the line in LDS.
@@ -1896,7 +1899,7 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
     allow_lds(fwd, smem_xy);
     allow_lds(inv, smem_xy);
     if (inv_split) allow_lds(inv_split, smem_xy);
-    const bool zreg = L0 % 64 == 0 && L0 <= 320;  // register z-convolution
+    const bool zreg = sense_fused_zconv_batched(n3);  // register z-convolution
     if (!zreg) allow_lds(z_conv_kernel, smem_z);
     // workgroups of a plane kernel the GPU runs at once: one or two per CU, by LDS
     const int64_t slots = NB <= 2 ? 512 : 256;

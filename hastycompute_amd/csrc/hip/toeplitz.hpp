@@ -69,6 +69,8 @@ bool sense_fused_supported(const int64_t* n3);
 void sense_fused_set_xy_variant(int v);
 // problems per register z-convolution launch of the fused operator (1..16)
 void sense_fused_set_zconv_batch(int v);
+// whether the z-convolution at this size is a register one (2 N0 = 64 k <= 320)
+bool sense_fused_zconv_batched(const int64_t* n3);
 int sense_fused_get_xy_variant();
 int sense_fused_get_zconv_batch();
 // z-convolution bundles at N0 = 128 and 160 (0..3, see sense_fused.hip)

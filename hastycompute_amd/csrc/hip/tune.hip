@@ -174,7 +174,7 @@ SenseChoice autotune_sense_normal(const int64_t* n3, int ncoil, int nproblems, b
                     best.problem_batch = pb;
                 }
             }
-            if (2 * n3[0] == 256) {
+            if (sense_fused_zconv_batched(n3)) {
                 // problems per z-convolution launch: values at or above the problem batch
                 // all mean one launch per chunk, so each effective value is timed once
                 std::vector<int> seen = {std::min(best.zconv_batch, best.problem_batch)};

@@ -57,6 +57,21 @@ def test_autotune_sense_normal(N, restore_options, shape, C):
     assert e < 1e-5, e
 
 
+@pytest.mark.parametrize("shape", [(32, 32, 32), (96, 32, 32)])
+def test_autotune_times_the_z_convolution_batch(N, restore_options, shape):
+    """The launches per z-convolution count at every register length (2 N0 = 64 k <= 320):
+    with one problem per launch to start from, 8 small problems of a chunk end in fewer
+    launches."""
+    from hastycompute_amd import _capi as Cap
+    from hastycompute_amd import autotune
+
+    Cap.set_option("sense_zconv_batch", 1)
+    t = autotune.sense_normal(shape, 5, 8)
+    print(f"autotune {shape}: {t}", flush=True)
+    assert t["problem_batch"] > 1 and t["sense_zconv_batch"] > 1
+    assert Cap.get_option("sense_zconv_batch") == t["sense_zconv_batch"]
+
+
 def test_autotune_nufft_type1(N, restore_options):
     from hastycompute_amd import autotune
 

@@ -174,6 +174,16 @@ SenseChoice autotune_sense_normal(const int64_t* n3, int ncoil, int nproblems, b
                     best.problem_batch = pb;
                 }
             }
+            // a narrow z-convolution, where the option selects one, against the 16-column form
+            if ((2 * n3[0] == 256 || 2 * n3[0] == 320) && (best.zconv_variant & 1)) {
+                sense_fused_set_zconv_variant(2);
+                const double t = run_with(best.coil_batch, best.problem_batch);
+                if (t < kGain * tbest) {
+                    tbest = t;
+                    best.zconv_variant = 2;
+                }
+                sense_fused_set_zconv_variant(best.zconv_variant);
+            }
             if (sense_fused_zconv_batched(n3)) {
                 // problems per z-convolution launch: values at or above the problem batch
                 // all mean one launch per chunk, so each effective value is timed once

@@ -10,7 +10,7 @@ namespace hasty_hip {
 struct SenseChoice {
     int xy_variant = 2;     // plane kernels of the fused operator (library option sense_xy_variant)
     int zconv_batch = 16;   // problems per register z-convolution launch (sense_zconv_batch)
-    int zconv_variant = 2;  // z-convolution bundles (sense_zconv_variant; not swept, 16 columns are best)
+    int zconv_variant = 2;  // z-convolution bundles (sense_zconv_variant; 16 columns or an inherited 8)
     int problem_batch = 1;  // problems per launch (workspace sized for this many)
     int coil_batch = 1;     // coils sharing one oversampled-grid workspace
     double ms_per_problem = 0.0;

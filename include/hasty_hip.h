@@ -179,8 +179,8 @@ int hasty_get_option(const char* name, int64_t* value);
  * while `stream` is being captured.
  * hasty_autotune_sense_normal: the batched Toeplitz SENSE normal operator at image size
  *   nmodes3 with ncoil coils and nproblems problems (at most 8 timed), on synthetic
- *   data: plane kernels, problems per launch, problems per z-convolution launch and
- *   coils per workspace. Sets
+ *   data: plane kernels, problems per launch, z-convolution bundles where the option asks
+ *   for narrow ones, problems per z-convolution launch and coils per workspace. Sets
  *   sense_xy_variant, sense_zconv_variant and sense_zconv_batch to the winners (prepare
  *   kernels after this call) and writes choice[5] = {sense_xy_variant,
  *   sense_zconv_batch, problem_batch, coil_batch, sense_zconv_variant} (size the

@@ -72,6 +72,19 @@ def test_autotune_times_the_z_convolution_batch(N, restore_options, shape):
     assert Cap.get_option("sense_zconv_batch") == t["sense_zconv_batch"]
 
 
+@pytest.mark.parametrize("shape", [(128, 64, 64), (160, 64, 64)])
+def test_autotune_leaves_the_narrow_z_convolution(N, restore_options, shape):
+    """Bundles of 8 columns use half of each line they read; an autotuner that starts from
+    them ends with 16."""
+    from hastycompute_amd import _capi as Cap
+    from hastycompute_amd import autotune
+
+    Cap.set_option("sense_zconv_variant", 1)
+    t = autotune.sense_normal(shape, 9, 4)
+    print(f"autotune {shape}: {t}", flush=True)
+    assert t["sense_zconv_variant"] in (0, 2) and Cap.get_option("sense_zconv_variant") == t["sense_zconv_variant"]
+
+
 def test_autotune_nufft_type1(N, restore_options):
     from hastycompute_amd import autotune
 

@@ -125,7 +125,7 @@ struct DevBuf {
 
 // Device memory of toeplitz_build: its own arrays, the plan's grids and point arrays, with
 // room for 4 (point, core) pairs per point (a window of 9 of 16 cells crosses 3.4 cores in
-// the mean). A build that needs more allocates the rest.
+// the mean). A build that needs more allocates the rest. 0 for sizes the build refuses.
 size_t toeplitz_workspace_bytes(int64_t M, int ndim, const int64_t* nmodes, double tol)
 {
     double grid = 1.0, fine = 1.0, tmp = 1.0;
@@ -133,8 +133,10 @@ size_t toeplitz_workspace_bytes(int64_t M, int ndim, const int64_t* nmodes, doub
     double beta = 0.0;
     es_params(tol, &ns, &beta);
     for (int d = 0; d < ndim; ++d) {
+        if (nmodes[d] < 1 || nmodes[d] > 4096) return 0;  // grids of 4 n are at most 8192 long
         const double L = 2.0 * (double)nmodes[d];
         const double nf = (double)next235even(std::max<int64_t>(4 * nmodes[d], 2 * ns));
+        if (!fft_size_supported((int)nf)) return 0;
         grid *= L;
         fine *= nf;
         tmp *= d == ndim - 1 ? L : nf;

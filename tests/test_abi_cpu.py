@@ -31,6 +31,26 @@ def test_host_queries():
     assert L.hasty_svt_workspace_size(4096, 100) > 0
 
 
+@pytest.mark.parametrize("M,nmodes,tol", [
+    (100, [16, -5, 16], 1e-8), (100, [0, 16, 16], 1e-8), (100, [-16, -16, 16], 1e-8), (-1, [16, 16, 16], 1e-8),
+    (100, [16, 16, 16], 0.0), (100, [16, 16, 16], float("nan")), (100, [4096, 4096, 4096], 1e-8),
+    (100, [100000] * 3, 1e-8), (100, [2**62, 16, 16], 1e-8), (100, [2**63 - 1], 1e-8), (100, [16] * 4, 1e-8), (100, [], 1e-8)])
+def test_toeplitz_workspace_size_of_refused_builds(M, nmodes, tol):
+    """What the build refuses needs no workspace: 0, so that the build's own error is the one
+    the caller sees."""
+    assert _capi.lib().hasty_toeplitz_workspace_size(M, len(nmodes), _capi.i64arr(nmodes), tol) == 0
+
+
+@pytest.mark.parametrize("nmodes", [[16, 16, 16], [1, 1, 1], [2048], [2000, 30]])
+def test_toeplitz_workspace_size_of_builds(nmodes):
+    """Above all the two double-complex doubled grids the build holds at once."""
+    size = _capi.lib().hasty_toeplitz_workspace_size(100, len(nmodes), _capi.i64arr(nmodes), 1e-8)
+    grid = 16
+    for n in nmodes:
+        grid *= 2 * n
+    assert 2 * grid < size < 2**40
+
+
 def test_llr_shifts_host():
     """hasty_llr_shifts is host code: it must reproduce the oracle's restatement."""
     from oracle import oracle as O

@@ -1376,6 +1376,13 @@ int nufft_get_tile() { return g_tile; }
 void nufft_set_chunk(int v) { g_chunk = v; }
 int nufft_get_chunk() { return g_chunk; }
 
+size_t nufft_parts_bytes(int fp64)
+{
+    return (size_t)kGatherMaxParts * kGC * kGC * kGC * (fp64 ? sizeof(double2) : sizeof(float2));
+}
+
+double nufft_mean_pairs(int ns) { return std::pow(1.0 + (ns - 1) / (double)kGC, 3); }
+
 void es_params(double tol, int* ns, double* beta)
 {
     int w = (int)std::ceil(-std::log10(tol / 10.0));

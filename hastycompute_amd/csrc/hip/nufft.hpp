@@ -109,6 +109,11 @@ int nufft_tile_edge(const NufftPlan* p);
 // returning the current spreader.
 int nufft_autotune(NufftPlan* p, void* c, void* f, hipStream_t s, double* ms);
 
+// Most device memory that the part sums of a 3-D type-1 plan take (g_partial), and the mean
+// number of 16^3 cores that a point's window touches.
+size_t nufft_parts_bytes(int fp64);
+double nufft_mean_pairs(int ns);
+
 // ES kernel parameters for upsampling factor 2.
 void es_params(double tol, int* ns, double* beta);
 

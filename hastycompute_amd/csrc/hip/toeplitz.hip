@@ -123,9 +123,9 @@ struct DevBuf {
 
 }  // namespace
 
-// Device memory of toeplitz_build: its own arrays, the plan's grids and point arrays, with
-// room for 4 (point, core) pairs per point (a window of 9 of 16 cells crosses 3.4 cores in
-// the mean). A build that needs more allocates the rest. 0 for sizes the build refuses.
+// Device memory of toeplitz_build: its own arrays, the plan's grids, point arrays and, in
+// 3-D, the spreader's (point, core) pairs (their mean number and 5 %) and part sums. A
+// build that needs more allocates the rest. 0 for sizes the build refuses.
 size_t toeplitz_workspace_bytes(int64_t M, int ndim, const int64_t* nmodes, double tol)
 {
     double grid = 1.0, fine = 1.0, tmp = 1.0;
@@ -141,9 +141,10 @@ size_t toeplitz_workspace_bytes(int64_t M, int ndim, const int64_t* nmodes, doub
         fine *= nf;
         tmp *= d == ndim - 1 ? L : nf;
     }
-    const double points = (double)M * (8.0 * ndim + 16 + 12 + 24 + 4 + 4 + 8 + 8 + 4 * 8);
-    const double bins = fine / 64.0 * 24.0 + fine / 4096.0 * 27.0 * 8.0 + 1024.0 * 65536.0;
-    return (size_t)(16.0 * (grid + fine + tmp) + points + bins) + (1u << 20);
+    const double pairs = ndim == 3 ? 1.05 * nufft_mean_pairs(ns) : 0.0;
+    const double points = (double)M * (8.0 * ndim + 16 + 12 + 24 + 4 + 4 + 8 + 8 + 8 * pairs);
+    const double bins = fine / 64.0 * 24.0 + fine / 4096.0 * 27.0 * 8.0;
+    return (size_t)(16.0 * (grid + fine + tmp) + points + bins) + (ndim == 3 ? nufft_parts_bytes(1) : 0) + (1u << 20);
 }
 
 void toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, const int64_t* nmodes,

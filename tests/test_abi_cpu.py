@@ -51,6 +51,18 @@ def test_toeplitz_workspace_size_of_builds(nmodes):
     assert 2 * grid < size < 2**40
 
 
+def test_toeplitz_workspace_size_counts_what_the_build_has():
+    """The part sums (at most 768 x 16^3 complex128 values, 3-D only) and the pairs of the
+    kernel's width: 1 + 15/16 cores per dim at ns = 16, 1 + 8/16 at 9."""
+    size = lambda M, nmodes, tol: _capi.lib().hasty_toeplitz_workspace_size(M, len(nmodes), _capi.i64arr(nmodes), tol)
+    assert size(40, [18], 1e-8) < 2**21
+    parts = 768 * 16**3 * 16
+    assert parts < size(40, [16, 16, 16], 1e-8) < parts + 16 * (32**3 + 64**3 + 64**2 * 32) + 2**21
+    per_point = [(size(10**6, [16, 16, 16], tol) - size(0, [16, 16, 16], tol)) / 1e6 for tol in (1e-8, 1e-15)]
+    assert 8 * 1.5**3 <= per_point[0] - 100 < 1.1 * 8 * 1.5**3
+    assert 8 * 1.9375**3 <= per_point[1] - 100 < 1.1 * 8 * 1.9375**3
+
+
 def test_llr_shifts_host():
     """hasty_llr_shifts is host code: it must reproduce the oracle's restatement."""
     from oracle import oracle as O

@@ -18,10 +18,15 @@ void toeplitz_build(const at::Tensor& coords, const std::vector<int64_t>& img, c
                     float* kernel, double tol)
 {
     if (!coords.is_cuda()) throw std::runtime_error("Coordinates did not reside in cuda device");
-    const size_t bytes = hasty_toeplitz_workspace_size(coords.size(1), (int)img.size(), img.data(), tol);
-    at::Tensor ws = at::empty({(int64_t)bytes}, coords.options().dtype(at::kByte));
+    size_t bytes = hasty_toeplitz_workspace_size(coords.size(1), (int)img.size(), img.data(), tol);
+    at::Tensor ws;
+    try {
+        ws = at::empty({(int64_t)bytes}, coords.options().dtype(at::kByte));
+    } catch (const c10::OutOfMemoryError&) {  // the size is an estimate: the build allocates what it needs itself
+        bytes = 0;
+    }
     check(hasty_toeplitz_build_ws(coords.data_ptr(), coords.scalar_type() == at::kDouble ? 1 : 0, coords.size(1),
-                                  (int)img.size(), img.data(), weights, diag, kernel, tol, ws.data_ptr(), bytes,
+                                  (int)img.size(), img.data(), weights, diag, kernel, tol, bytes ? ws.data_ptr() : nullptr, bytes,
                                   (void*)c10::hip::getCurrentHIPStream().stream()));
 }
 

@@ -111,7 +111,10 @@ def toeplitz_build(coords: torch.Tensor, nmodes: Sequence[int], weights: Optiona
         _require(weights.dtype == torch.float32, "weights must be float32")
     # the build's gigabyte of grids from torch's caching allocator, not hipMalloc / hipFree
     wsb = int(C.lib().hasty_toeplitz_workspace_size(int(coords.shape[1]), len(nmodes), C.i64arr(nmodes), float(tol)))
-    ws = torch.empty(wsb, dtype=torch.uint8, device=coords.device)
+    try:
+        ws = torch.empty(wsb, dtype=torch.uint8, device=coords.device)
+    except torch.OutOfMemoryError:  # the size is an estimate: the build allocates what it needs itself
+        ws, wsb = None, 0
     C.call("hasty_toeplitz_build_ws", coords.data_ptr(), int(coords.dtype == torch.float64), int(coords.shape[1]),
            len(nmodes), C.i64arr(nmodes), C.ptr(weights), C.ptr(d), C.ptr(k), float(tol), C.ptr(ws), wsb, C.stream_ptr())
     return d, k

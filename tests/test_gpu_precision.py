@@ -242,3 +242,36 @@ def test_toeplitz_build_waits_for_its_stream(dims):
         stream.synchronize()
     # the tile spreader of the second size adds in another order from run to run
     assert float((ks[1] - ks[0]).abs().max()) <= 1e-7 * float(ks[0].abs().max())
+
+
+def test_toeplitz_build_without_torch_memory():
+    """The workspace is an estimate and comes from torch: where torch has no room for it the
+    build allocates what it needs, through the Python wrapper and the C++ operator alike."""
+    from hastycompute_amd import native
+    from hastycompute_amd.ffi import hasty_sense
+
+    n, M = 64, 20000
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(7)
+    co = (torch.rand((3, M), dtype=torch.float32, device="cuda:0", generator=gen) * 2 - 1) * 3.1415926
+    S = torch.randn((1, n, n, n), dtype=torch.complex64)
+    x = torch.randn((1, 1, n, n, n), dtype=torch.complex64)
+
+    def both():
+        out = torch.zeros_like(x)
+        hasty_sense.BatchedSenseNormal([co], S).apply(x, out)
+        return native.toeplitz_build(co, [n] * 3, diag=False)[1], out
+
+    k, out = both()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    # room for the images, kernels and the operator's grids (some 100 MB), not for 500 MB more
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2**28) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(2**29 - 2**26, dtype=torch.uint8, device="cuda:0")
+        k2, out2 = both()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(k, k2) and torch.equal(out, out2)

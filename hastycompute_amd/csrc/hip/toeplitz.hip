@@ -160,8 +160,13 @@ void toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, con
         L[3 - ndim + d] = 2 * nmodes[d];
     }
     const int64_t ngrid = L[0] * L[1] * L[2];
-    // the build ends with its stream synchronised, so nothing in the arena is in use after it
+    // the build ends with its stream synchronised, also when it fails, so nothing in the arena
+    // is in use after it
     DeviceArena arena(workspace, workspace_bytes);
+    struct StreamIdle {
+        hipStream_t s;
+        ~StreamIdle() { (void)hipStreamSynchronize(s); }
+    } idle{s};
 
     DevBuf psf(sizeof(double2) * ngrid);
     const size_t after_psf = arena.mark();
@@ -187,7 +192,6 @@ void toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim, con
             nufft_execute(plan, cw.p, psf.p, s);
             HASTY_HIP_CHECK(hipStreamSynchronize(s));
         } catch (...) {
-            (void)hipStreamSynchronize(s);
             nufft_destroy(plan);
             throw;
         }

@@ -275,3 +275,24 @@ def test_toeplitz_build_without_torch_memory():
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(k, k2) and torch.equal(out, out2)
+
+
+def test_failed_toeplitz_build_leaves_its_stream_idle():
+    """The workspace is free again when the call returns, also when the build refuses its
+    sizes after its first launches (a 1-D grid of 20000): what was queued is through."""
+    from hastycompute_amd import _capi as C
+
+    M, n = 1000, C.i64arr([5000])
+    co = torch.zeros((1, M), dtype=torch.float32, device="cuda:0")
+    k = torch.empty(10000, dtype=torch.float32, device="cuda:0")
+    ws = torch.empty(2**27, dtype=torch.uint8, device="cuda:0")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(1000):
+            ws.fill_(0)
+        with pytest.raises(C.HastyError, match="fine grid too large"):
+            C.call("hasty_toeplitz_build_ws", co.data_ptr(), 0, M, 1, n, None, None, k.data_ptr(), 1e-8, ws.data_ptr(),
+                   ws.numel(), C.stream_ptr())
+        assert stream.query()
+    stream.synchronize()

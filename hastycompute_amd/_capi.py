@@ -148,8 +148,20 @@ def stream_ptr(stream=None) -> int:
     return s.cuda_stream
 
 
+# Calls that allocate device memory of their own (hipMalloc) and may be made again when that
+# failed. torch's caching allocator keeps what it no longer uses (a kernel build's workspace
+# among it), which hipMalloc cannot have.
+_ALLOCATING = frozenset({"hasty_nufft_makeplan", "hasty_nufft_setpts", "hasty_toeplitz_build", "hasty_toeplitz_build_ws",
+                         "hasty_circulant_precond_build", "hasty_autotune_sense_normal", "hasty_autotune_llr"})
+OUT_OF_MEMORY = 5
+
+
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    rc = getattr(lib(), name)(*args)
+    if rc == OUT_OF_MEMORY and name in _ALLOCATING:
+        torch.cuda.empty_cache()
+        rc = getattr(lib(), name)(*args)
+    check(rc)
 
 
 def get_option(name: str) -> int:

@@ -1555,6 +1555,7 @@ template <typename R> void setpts_typed(NufftPlan* p, hipStream_t s)
         dev_free(p->suboff);
         p->subbin = nullptr;
         p->suboff = nullptr;
+        p->cap_sub = 0;
         p->subbin = (int*)dev_alloc(sizeof(int) * total);
         p->suboff = (int*)dev_alloc(sizeof(int) * total);
         p->cap_sub = total;
@@ -1610,7 +1611,11 @@ template <typename R> void gather_build(NufftPlan* p, hipStream_t s)
     g.M = p->M;
     g.ns = p->ns;
     const int64_t ncore = (int64_t)nb[0] * nb[1] * nb[2];
-    if (!p->g_counts) {
+    if (!p->g_pstart) {  // the last of the four: set when all are
+        for (int** q : {&p->g_counts, &p->g_binstart, &p->g_pcount}) {
+            dev_free(*q);
+            *q = nullptr;
+        }
         p->g_counts = (int*)dev_alloc(sizeof(int) * ncore);
         p->g_binstart = (int*)dev_alloc(sizeof(int) * (ncore + 1));
         p->g_pcount = (int*)dev_alloc(sizeof(int) * 27 * ncore);
@@ -1624,6 +1629,7 @@ template <typename R> void gather_build(NufftPlan* p, hipStream_t s)
         p->g_l0 = nullptr;
         p->g_frac = nullptr;
         p->g_idx = p->g_rank = nullptr;
+        p->g_cap_M = 0;
         p->g_l0 = (int*)dev_alloc(sizeof(int) * 3 * p->M);
         p->g_frac = dev_alloc(sizeof(R) * 3 * p->M);
         p->g_idx = (int*)dev_alloc(sizeof(int) * p->M);
@@ -2034,6 +2040,7 @@ void nufft_setpts(NufftPlan* p, int64_t M, const void* x, const void* y, const v
         dev_free(p->sortidx);
         p->rank = nullptr;
         p->sortidx = nullptr;
+        p->cap_M = 0;
         p->rank = (int*)dev_alloc(sizeof(int) * need);
         p->sortidx = (int*)dev_alloc(sizeof(int) * need);
         p->cap_M = need;

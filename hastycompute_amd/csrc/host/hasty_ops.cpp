@@ -1,5 +1,6 @@
 #include "hasty_ops.hpp"
 
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cmath>
@@ -13,6 +14,19 @@ namespace detail {
 
 void check(int rc);
 
+// A call that allocates device memory of its own (hipMalloc): made again without what torch's
+// caching allocator keeps unused when that failed.
+template <typename Fn> void check_allocating(Fn&& fn)
+{
+    constexpr int kOutOfMemory = 5;
+    int rc = fn();
+    if (rc == kOutOfMemory) {
+        c10::hip::HIPCachingAllocator::emptyCache();
+        rc = fn();
+    }
+    check(rc);
+}
+
 // hasty_toeplitz_build with its device memory from torch's caching allocator.
 void toeplitz_build(const at::Tensor& coords, const std::vector<int64_t>& img, const float* weights, void* diag,
                     float* kernel, double tol)
@@ -25,9 +39,12 @@ void toeplitz_build(const at::Tensor& coords, const std::vector<int64_t>& img, c
     } catch (const c10::OutOfMemoryError&) {  // the size is an estimate: the build allocates what it needs itself
         bytes = 0;
     }
-    check(hasty_toeplitz_build_ws(coords.data_ptr(), coords.scalar_type() == at::kDouble ? 1 : 0, coords.size(1),
-                                  (int)img.size(), img.data(), weights, diag, kernel, tol, bytes ? ws.data_ptr() : nullptr, bytes,
-                                  (void*)c10::hip::getCurrentHIPStream().stream()));
+    check_allocating([&] {
+        return hasty_toeplitz_build_ws(coords.data_ptr(), coords.scalar_type() == at::kDouble ? 1 : 0, coords.size(1),
+                                       (int)img.size(), img.data(), weights, diag, kernel, tol,
+                                       bytes ? ws.data_ptr() : nullptr, bytes,
+                                       (void*)c10::hip::getCurrentHIPStream().stream());
+    });
 }
 
 void check(int rc)
@@ -88,14 +105,17 @@ CUDANufft::CUDANufft(const at::Tensor& coords, const std::vector<int64_t>& nmode
     std::vector<int64_t> flipped(_ndim);
     for (int i = 0; i < _ndim; ++i) flipped[i] = _nmodes[_ndim - i];
     const int fp64 = _type == at::ScalarType::Double ? 1 : 0;
-    check(hasty_nufft_makeplan((int)_opts.get_type(), _ndim, flipped.data(), _opts.get_positive(), _ntransf,
-                               _opts.get_tol(), fp64, &_plan));
+    detail::check_allocating([&] {
+        return hasty_nufft_makeplan((int)_opts.get_type(), _ndim, flipped.data(), _opts.get_positive(), _ntransf,
+                                    _opts.get_tol(), fp64, &_plan);
+    });
     check(hasty_nufft_set_scale(_plan, 1.0 / std::sqrt((double)_nvoxels)));
     const char* base = static_cast<const char*>(_coords.data_ptr());
     const int64_t es = _coords.element_size();
     const void* rows[3] = {nullptr, nullptr, nullptr};
     for (int i = 0; i < _ndim; ++i) rows[i] = base + (int64_t)(_ndim - 1 - i) * _nfreq * es;  // x = last row
-    check(hasty_nufft_setpts(_plan, _nfreq, rows[0], rows[1], rows[2], detail::stream()));
+    detail::check_allocating(
+        [&] { return hasty_nufft_setpts(_plan, _nfreq, rows[0], rows[1], rows[2], detail::stream()); });
 }
 
 void CUDANufft::close()

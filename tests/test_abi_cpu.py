@@ -63,6 +63,30 @@ def test_toeplitz_workspace_size_counts_what_the_build_has():
     assert 8 * 1.9375**3 <= per_point[1] - 100 < 1.1 * 8 * 1.9375**3
 
 
+@pytest.mark.parametrize("name,codes,retried", [
+    ("hasty_nufft_makeplan", [5, 0], True), ("hasty_nufft_setpts", [5, 5], True), ("hasty_toeplitz_build_ws", [5, 0], True),
+    ("hasty_nufft_makeplan", [1], False), ("hasty_nufft_execute", [5], False)])
+def test_library_allocations_get_what_torch_caches(monkeypatch, name, codes, retried):
+    """A call whose hipMalloc fails is made once more after torch's cache is given back; other
+    errors and calls that allocate nothing are not repeated."""
+    left, emptied = list(codes), []
+
+    class Lib:
+        def __getattr__(self, _):
+            return lambda *args: left.pop(0)
+
+    monkeypatch.setattr(_capi, "lib", lambda: Lib())
+    monkeypatch.setattr(_capi, "last_error", lambda: "")
+    monkeypatch.setattr(torch.cuda, "empty_cache", lambda: emptied.append(len(left)))
+    if codes[-1]:
+        with pytest.raises(_capi.HastyError) as e:
+            _capi.call(name, 1, 2)
+        assert e.value.code == codes[-1]
+    else:
+        _capi.call(name, 1, 2)
+    assert not left and emptied == ([1] if retried else [])
+
+
 def test_llr_shifts_host():
     """hasty_llr_shifts is host code: it must reproduce the oracle's restatement."""
     from oracle import oracle as O

@@ -699,8 +699,39 @@ __global__ void __launch_bounds__(kLineThreads) line_fft_kernel(AxisKernelArgs<f
     }
 }
 
-template <class A, class B> void launch_line(const AxisKernelArgs<float>& args, int mode, hipStream_t s)
+// Fewest lines of a pass from which the two steps are the faster form. A workgroup carries
+// 16 lines through two long register transforms where the LDS kernel spreads 2048 / L lines
+// over its 256 threads, so a pass that leaves the GPU unfilled is bound by one workgroup's
+// chain: the longer a step (above 16 values) and the more it loads, the more lines it takes to
+// pay (two steps over LDS passes, by lines):
+//   convolution: 320 1.5 at 256, 1.0 at 2304, 0.8 at 6144; 240 at most 0.8
+//   contiguous padded input: 320 1.4 up to 2304, 0.9 at 7200; 250 at most 1.05
+//   strided padded input: 288 1.2 up to 1152, 1.0 at 2048 to 4608, 0.7 at 8192; 150 at most 0.96
+//   strided full input: 216 1.4 at 128, 1.15 at 4608, 0.85 at 8192; 300 1.5 at 128, 0.98 at 4608
+//   contiguous full input: 200 1.5 up to 4096, 1.2 at 10000, 0.86 at 12800; 216 1.6, 1.2 at
+//   7200, 0.9 at 10000; 320 2.2 at 1024 and 1.1 to 1.4 from 10000 on; 100 (steps of 20 and 5:
+//   lanes run over 5 elements) 1.3, 0.84 at 25600
+// Shorter steps are ahead at any number of lines (0.4 to 1.05).
+int64_t line_fft_from(const AxisFft<float>& a, int mode, int ra, int rb)
 {
+    const int L = a.L;
+    const bool contiguous = a.ain.stride == 1, wide = ra > 16 || rb > 16;
+    if (mode == 1) return L < 256 ? 0 : 2304;
+    if (a.n_in < L) {
+        if (contiguous) return L < 256 ? 0 : 7168;
+        return wide && L > 150 ? 3072 : 0;
+    }
+    if (!contiguous) return !wide ? 0 : L > 256 ? 5120 : 7168;
+    if (!wide && L < 240) return 0;
+    if (L > 270) return INT64_MAX;
+    if (rb < 8) return 24576;
+    return ra > 8 ? 9216 : 12288;
+}
+
+// False where the LDS kernel serves the pass better.
+template <class A, class B> bool launch_line(const AxisKernelArgs<float>& args, int mode, hipStream_t s)
+{
+    if (args.a.nlines < line_fft_from(args.a, mode, A::product, B::product)) return false;
     const unsigned blocks = (unsigned)ceil_div(args.a.nlines, kLinesPer);
     if (mode == 1)
         hipLaunchKernelGGL((line_fft_kernel<A, B, 1, -1>), dim3(blocks), dim3(kLineThreads), 0, s, args);
@@ -709,40 +740,41 @@ template <class A, class B> void launch_line(const AxisKernelArgs<float>& args, 
     else
         hipLaunchKernelGGL((line_fft_kernel<A, B, 0, 1>), dim3(blocks), dim3(kLineThreads), 0, s, args);
     check_launch("line_fft_kernel");
+    return true;
 }
 
-// The even 2,3,5-smooth lengths of 48 .. 320 other than 54 and 50 (doubled images of 24 ..
-// 160); false for others. Radices in the order of make_radix_plan; the split keeps both
-// steps within 40 values per thread.
+// The even 2,3,5-smooth lengths of 48 .. 320 (doubled images of 24 .. 160) but 50 and 54, which
+// were not measured and stay on the LDS passes; false for others. Radices in the order of
+// make_radix_plan; the split keeps both steps within 40 values per thread.
 bool run_line_fft(const AxisKernelArgs<float>& args, int mode, hipStream_t s)
 {
     switch (args.a.L) {
-    case 48: launch_line<RadixList<8>, RadixList<2, 3>>(args, mode, s); return true;
-    case 60: launch_line<RadixList<4, 3>, RadixList<5>>(args, mode, s); return true;
-    case 64: launch_line<RadixList<8>, RadixList<8>>(args, mode, s); return true;
-    case 72: launch_line<RadixList<8>, RadixList<3, 3>>(args, mode, s); return true;
-    case 80: launch_line<RadixList<8>, RadixList<2, 5>>(args, mode, s); return true;
-    case 90: launch_line<RadixList<2, 3>, RadixList<3, 5>>(args, mode, s); return true;
-    case 96: launch_line<RadixList<8>, RadixList<4, 3>>(args, mode, s); return true;
-    case 100: launch_line<RadixList<4, 5>, RadixList<5>>(args, mode, s); return true;
-    case 108: launch_line<RadixList<4, 3>, RadixList<3, 3>>(args, mode, s); return true;
-    case 120: launch_line<RadixList<8>, RadixList<3, 5>>(args, mode, s); return true;
-    case 128: launch_line<RadixList<8>, RadixList<8, 2>>(args, mode, s); return true;
-    case 144: launch_line<RadixList<8, 2>, RadixList<3, 3>>(args, mode, s); return true;
-    case 150: launch_line<RadixList<2, 3>, RadixList<5, 5>>(args, mode, s); return true;
-    case 160: launch_line<RadixList<8>, RadixList<4, 5>>(args, mode, s); return true;
-    case 162: launch_line<RadixList<2, 3, 3>, RadixList<3, 3>>(args, mode, s); return true;
-    case 180: launch_line<RadixList<4, 3>, RadixList<3, 5>>(args, mode, s); return true;
-    case 192: launch_line<RadixList<8>, RadixList<8, 3>>(args, mode, s); return true;
-    case 200: launch_line<RadixList<8>, RadixList<5, 5>>(args, mode, s); return true;
-    case 216: launch_line<RadixList<8, 3>, RadixList<3, 3>>(args, mode, s); return true;
-    case 240: launch_line<RadixList<8, 2>, RadixList<3, 5>>(args, mode, s); return true;
-    case 250: launch_line<RadixList<2, 5>, RadixList<5, 5>>(args, mode, s); return true;
-    case 256: launch_line<RadixList<8>, RadixList<8, 4>>(args, mode, s); return true;
-    case 270: launch_line<RadixList<2, 3, 3>, RadixList<3, 5>>(args, mode, s); return true;
-    case 288: launch_line<RadixList<8, 4>, RadixList<3, 3>>(args, mode, s); return true;
-    case 300: launch_line<RadixList<4, 3>, RadixList<5, 5>>(args, mode, s); return true;
-    case 320: launch_line<RadixList<8>, RadixList<8, 5>>(args, mode, s); return true;
+    case 48: return launch_line<RadixList<8>, RadixList<2, 3>>(args, mode, s);
+    case 60: return launch_line<RadixList<4, 3>, RadixList<5>>(args, mode, s);
+    case 64: return launch_line<RadixList<8>, RadixList<8>>(args, mode, s);
+    case 72: return launch_line<RadixList<8>, RadixList<3, 3>>(args, mode, s);
+    case 80: return launch_line<RadixList<8>, RadixList<2, 5>>(args, mode, s);
+    case 90: return launch_line<RadixList<2, 3>, RadixList<3, 5>>(args, mode, s);
+    case 96: return launch_line<RadixList<8>, RadixList<4, 3>>(args, mode, s);
+    case 100: return launch_line<RadixList<4, 5>, RadixList<5>>(args, mode, s);
+    case 108: return launch_line<RadixList<4, 3>, RadixList<3, 3>>(args, mode, s);
+    case 120: return launch_line<RadixList<8>, RadixList<3, 5>>(args, mode, s);
+    case 128: return launch_line<RadixList<8>, RadixList<8, 2>>(args, mode, s);
+    case 144: return launch_line<RadixList<8, 2>, RadixList<3, 3>>(args, mode, s);
+    case 150: return launch_line<RadixList<2, 3>, RadixList<5, 5>>(args, mode, s);
+    case 160: return launch_line<RadixList<8>, RadixList<4, 5>>(args, mode, s);
+    case 162: return launch_line<RadixList<2, 3, 3>, RadixList<3, 3>>(args, mode, s);
+    case 180: return launch_line<RadixList<4, 3>, RadixList<3, 5>>(args, mode, s);
+    case 192: return launch_line<RadixList<8>, RadixList<8, 3>>(args, mode, s);
+    case 200: return launch_line<RadixList<8>, RadixList<5, 5>>(args, mode, s);
+    case 216: return launch_line<RadixList<8, 3>, RadixList<3, 3>>(args, mode, s);
+    case 240: return launch_line<RadixList<8, 2>, RadixList<3, 5>>(args, mode, s);
+    case 250: return launch_line<RadixList<2, 5>, RadixList<5, 5>>(args, mode, s);
+    case 256: return launch_line<RadixList<8>, RadixList<8, 4>>(args, mode, s);
+    case 270: return launch_line<RadixList<2, 3, 3>, RadixList<3, 5>>(args, mode, s);
+    case 288: return launch_line<RadixList<8, 4>, RadixList<3, 3>>(args, mode, s);
+    case 300: return launch_line<RadixList<4, 3>, RadixList<5, 5>>(args, mode, s);
+    case 320: return launch_line<RadixList<8>, RadixList<8, 5>>(args, mode, s);
     default: return false;
     }
 }

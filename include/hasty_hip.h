@@ -160,8 +160,9 @@ int hasty_sense_normal_toeplitz_ex(const void* x, void* out, const void* smaps, 
  *   "fft_r16" 0 or 1 (default 1): complex64 axis FFT passes in registers: lines of 128,
  *     192, 256 or 320 (the NUFFT at 64^3 .. 160^3 modes) without coil multipliers,
  *     accumulation or convolution as a 16 x R four-step FFT, other passes of the common
- *     lengths from 48 to 320 as two register steps with the LDS passes' roundings; 0 keeps
- *     them on the LDS Stockham passes.
+ *     lengths from 48 to 320 as two register steps with the LDS passes' roundings (long
+ *     lines from the number of lines on where that is faster); 0 keeps them on the LDS
+ *     Stockham passes.
  *   "fft_strided_lines" 0..64 (default 0 = auto): lines per workgroup of the axis FFT
  *     passes whose lines are strided (the NUFFT's outer axes, the Toeplitz kernel build,
  *     the generic normal operator); auto gives every pass 2048 / L (complex64) or

@@ -261,6 +261,65 @@ def test_z_convolution_lengths(N, n0, narrow):
             assert err < 1.8e-6, err
 
 
+@pytest.mark.parametrize("n", [50, 75, 80, 81, 96, 100, 108, 120, 125, 128, 135, 144, 150, 160])
+def test_long_register_lines_equal_lds_passes(N, n):
+    """The lengths with a step of more than 16 values, which take the register form from some
+    number of lines on: passes above it (convolved, strided, contiguous), as below."""
+    from hastycompute_amd import _capi
+
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(n)
+    for dims in ([n, 25, 24], [72, n, 60], [125, 108, n] if n > 50 else [162, 162, n]):
+        smaps = torch.randn([2] + dims, dtype=torch.complex64, device="cuda:0", generator=gen)
+        kern = torch.rand([2 * d for d in dims], dtype=torch.float32, device="cuda:0", generator=gen)
+        x = torch.randn([1] + dims, dtype=torch.complex64, device="cuda:0", generator=gen)
+        op = N.SenseNormalToeplitz(smaps, kern, coil_batch=2, fused=False)
+        prev = _capi.get_option("fft_r16")
+        outs = []
+        try:
+            for v in (0, 1):
+                _capi.set_option("fft_r16", v)
+                outs.append(op.apply(x))
+        finally:
+            _capi.set_option("fft_r16", prev)
+        if any(2 * d in (128, 192, 256, 320) for d in dims):  # four-step plain passes, see below
+            err = float(torch.linalg.vector_norm(outs[0] - outs[1]) / torch.linalg.vector_norm(outs[0]))
+            assert err < 2e-6, err
+        else:
+            assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("dims", [(16, 16, 50), (16, 16, 100), (16, 16, 144), (16, 16, 160), (160, 8, 8), (8, 108, 8)])
+def test_short_launches_of_long_lines(N, dims):
+    """Passes of few long lines run no slower than on the LDS kernel (a fifth allowed for the
+    clock; two register steps for every pass took 1.2 to 1.5 times as long)."""
+    from hastycompute_amd import _capi
+
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(1)
+    smaps = torch.randn((8, *dims), dtype=torch.complex64, device="cuda:0", generator=gen)
+    kern = torch.rand([2 * d for d in dims], dtype=torch.float32, device="cuda:0", generator=gen)
+    x = torch.randn((1, *dims), dtype=torch.complex64, device="cuda:0", generator=gen)
+    op = N.SenseNormalToeplitz(smaps, kern, coil_batch=4, fused=False)
+    prev = _capi.get_option("fft_r16")
+    best = {}
+    try:
+        for v in (0, 1) * 6:
+            _capi.set_option("fft_r16", v)
+            op.apply(x)
+            N.timing_enable(True)
+            for _ in range(5):
+                op.apply(x)
+            torch.cuda.synchronize()
+            ms = N.timing_read()["fft_axis"][0]
+            best[v] = min(ms, best.get(v, ms))
+    finally:
+        N.timing_enable(False)
+        _capi.set_option("fft_r16", prev)
+    print(f"passes of {dims} x 8 coils: {200 * best[0]:.0f} us LDS, {200 * best[1]:.0f} us as chosen", flush=True)
+    assert best[1] <= 1.2 * best[0], best
+
+
 @pytest.mark.parametrize("n", [24, 30, 32, 36, 40, 45, 48, 50, 54, 60, 64, 72, 75, 80, 81, 90, 96, 100, 108, 120, 125,
                                128, 135, 144, 150, 160])
 def test_register_lines_equal_lds_passes(N, n):

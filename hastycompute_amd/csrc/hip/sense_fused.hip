@@ -1441,6 +1441,22 @@ int coil_groups(int64_t wgs, int coils, int64_t slots)
     return g;
 }
 
+// Whether one workgroup per coil and the coil sum beat one workgroup per (z-plane, problem)
+// pair that loops over the coils, for `wgs` pairs that the GPU takes at once. The split's
+// rounds of workgroups each cost a coil and a share of writing and re-reading its image, so
+// they have to be so many fewer than the coils. Inverse and sum over the loop at 128 x 128: 2
+// rounds for 4 coils 0.78, 2 for 3 0.92, 5 for 8 0.99, 3 for 4 1.05, 2 for 2 1.24 (64 x 64:
+// 3 for 4 0.85, 6 for 8 0.78, 2 for 2 1.0 to 1.06). 32 x 32 planes take 10 us either way, two
+// a CU at once: 1 round for 2 coils 1.2, for 3 0.9, 3 for 4 1.0.
+bool inverse_split_pays(int NB, int64_t wgs, int coils)
+{
+    const int64_t slots = NB == 1 ? 512 : 256;
+    if (wgs >= slots) return false;
+    const int64_t rounds = ceil_div(wgs * coils, slots);
+    if (NB == 1 && coils < 4) return coils == 3 && rounds == 1;
+    return 20 * rounds <= (NB <= 2 ? 15 : 14) * (int64_t)coils;
+}
+
 // z-axis pass for L0 = 2 N0 = R1 R2 as a four-step FFT with the data in registers:
 // z = R2 n1 + n2 (n1 < R1 / 2 nonzero) and k = k1 + R1 k2. In steps A and A' (the R1-point
 // DFTs) thread g of a column owns n2 = g, in step B (the R2-point DFTs, the kernel and
@@ -1939,7 +1955,7 @@ void sense_fused_apply(const float2* x, float2* out, const float2* smaps, const 
                 hipLaunchKernelGGL(z_conv_kernel, dim3((unsigned)(L * L / kW)), dim3(kZ), smem_z, s, a, L * L, pl, K);
                 check_launch("z_conv_kernel");
             }
-            if (inv_split && a.ccount > 1 && (int64_t)N0 * np < slots) {
+            if (inv_split && inverse_split_pays(NB, (int64_t)N0 * np, a.ccount)) {
                 {
                     KernelTimer t("sense_inv_xy", s);
                     hipLaunchKernelGGL(inv_split, dim3(N0, np, a.ccount), dim3(nxy), smem_xy, s, a);

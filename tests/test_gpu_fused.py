@@ -230,6 +230,29 @@ def test_split_launches_equal_whole_launches(N, n, coil_batch):
     assert err < 1e-6, err
 
 
+@pytest.mark.parametrize("n,n0,P,C,split", [
+    (128, 128, 1, 16, True), (128, 128, 1, 2, True), (128, 96, 2, 2, False), (128, 160, 1, 2, False), (128, 96, 2, 3, False),
+    (96, 160, 1, 2, False), (96, 96, 1, 3, True), (64, 64, 1, 8, True), (64, 96, 4, 3, False), (64, 96, 2, 4, True),
+    (32, 32, 1, 4, True), (32, 32, 1, 2, False), (32, 48, 4, 2, False), (128, 128, 2, 8, False)])
+def test_inverse_split_by_coils_where_it_pays(N, n, n0, P, C, split):
+    """The inverse plane launch writes coil images and sums them only where that was measured
+    to be faster; the result is the same to the bit (see the test above)."""
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(n0)
+    smaps = torch.randn((C, n0, n, n), dtype=torch.complex64, device="cuda:0", generator=gen)
+    kern = torch.rand((2 * n0, 2 * n, 2 * n), dtype=torch.float32, device="cuda:0", generator=gen)
+    x = torch.randn((P, n0, n, n), dtype=torch.complex64, device="cuda:0", generator=gen)
+    op = N.SenseNormalToeplitz(smaps, kern, coil_batch=C, problem_batch=P)
+    assert op.layout != 0
+    op.apply(x)
+    N.timing_enable(True)
+    op.apply(x)
+    torch.cuda.synchronize()
+    names = N.timing_read()
+    N.timing_enable(False)
+    assert ("sense_coil_sum" in names) == split, names
+
+
 @pytest.mark.parametrize("n0", [32, 64, 96, 128, 160])
 @pytest.mark.parametrize("narrow", [False, True])
 def test_z_convolution_lengths(N, n0, narrow):

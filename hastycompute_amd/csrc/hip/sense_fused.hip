@@ -1700,10 +1700,14 @@ __global__ void __launch_bounds__(8 * kZ8Cols) z_conv_r8_kernel(FusedArgs a, int
     }
 }
 
-// Coils per workgroup of a z-convolution launch of `wgs` (bundle, problem) pairs.
-int zconv_group(const FusedArgs& a, int64_t wgs)
+// Coils per workgroup of a z-convolution launch of `wgs` (bundle, problem) pairs: split by
+// coils up to 1024 workgroups, but not where `full` pairs already keep the GPU busy (every
+// group reads the kernel again): 512 pairs of 192 points or more split in two took 1.05 to 1.3
+// times as long, 2304 and more 1.0 to 1.2, 2304 and more of 64 or 128 points 0.95 to 1.15. 256
+// pairs of 320 points gain from two groups (0.87), not from four (1.11).
+int zconv_group(const FusedArgs& a, int64_t wgs, int64_t full)
 {
-    const int groups = coil_groups(wgs, a.ccount, 1024);
+    const int groups = wgs >= full ? 1 : coil_groups(wgs, a.ccount, a.L0 == 320 ? 512 : 1024);
     return (a.ccount + groups - 1) / groups;
 }
 
@@ -1715,7 +1719,7 @@ void launch_zconv_reg(const FusedArgs& a, int LL, int q0, int nq, const ZKernels
     // with four, 2.07 ms with two or three, 128^3 x 16 coils x 5 problems)
     constexpr size_t smem = std::max(Sh::lds_bytes(), (size_t)(Sh::T >= 256 ? 53 * 1024 : 0));
     allow_lds(z_conv_reg_kernel<R1, R2, COLS>, smem);
-    const int gcoils = zconv_group(a, (int64_t)(LL / COLS) * nq);
+    const int gcoils = zconv_group(a, (int64_t)(LL / COLS) * nq, 512);
     hipLaunchKernelGGL((z_conv_reg_kernel<R1, R2, COLS>),
                        dim3((unsigned)(LL / COLS), (unsigned)nq, (unsigned)ceil_div(a.ccount, gcoils)), dim3(Sh::T), smem,
                        s, a, LL, q0, zk, gcoils);
@@ -1724,7 +1728,7 @@ void launch_zconv_reg(const FusedArgs& a, int LL, int q0, int nq, const ZKernels
 template <int NB>
 void launch_zconv_r8(const FusedArgs& a, int LL, int q0, int nq, const ZKernels& zk, hipStream_t s)
 {
-    const int gcoils = zconv_group(a, (int64_t)(LL / kZ8Cols) * nq);
+    const int gcoils = zconv_group(a, (int64_t)(LL / kZ8Cols) * nq, 2048);
     hipLaunchKernelGGL(z_conv_r8_kernel<NB>,
                        dim3((unsigned)(LL / kZ8Cols), (unsigned)nq, (unsigned)ceil_div(a.ccount, gcoils)),
                        dim3(8 * kZ8Cols), 0, s, a, LL, q0, zk, gcoils);

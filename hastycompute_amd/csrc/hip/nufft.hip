@@ -1207,9 +1207,16 @@ template <typename R, int NS, int DIM> void launch_interp_ns(const SpreadArgs<R>
 {
     KernelTimer t("nufft_interp", s);
     if constexpr (DIM == 3) {
-        hipLaunchKernelGGL((interp3_kernel<R, NS>),
-                           dim3((unsigned)xcd_grid(ceil_div(M, (InterpShape<R, NS>::points)), a.xcd)), dim3(kThreads), 0, s,
-                           a);
+        // a launch holds less than 2^32 threads, 2 to 16 of them per point
+        constexpr int64_t points = InterpShape<R, NS>::points;
+        constexpr int64_t most = ((int64_t(1) << 32) / kThreads - kXcds) * points;
+        for (int64_t p0 = 0; p0 < M; p0 += most) {
+            SpreadArgs<R> b = a;
+            b.sortidx += p0;
+            b.pa.M = std::min(M - p0, most);
+            hipLaunchKernelGGL((interp3_kernel<R, NS>), dim3((unsigned)xcd_grid(ceil_div(b.pa.M, points), a.xcd)),
+                               dim3(kThreads), 0, s, b);
+        }
     } else {
         hipLaunchKernelGGL((interp_kernel<R, NS, DIM>), dim3((unsigned)xcd_grid(ceil_div(M, kThreads), a.xcd)),
                            dim3(kThreads), 0, s, a);

@@ -701,6 +701,25 @@ def test_output_spreader_parts_and_widths(N, M, fp64, tol):
     assert err < max(10 * tol, 1e-12 if fp64 else 3e-6), err
 
 
+def test_type2_more_points_than_one_launch_holds(N):
+    """16 lanes per point (ns = 16) and 2^28 + 7 points: more threads than a launch takes. Each
+    point's value is its own, so a few thousand of them give the same bits in a plan of their
+    own."""
+    M = 2**28 + 7
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(3)
+    co = torch.rand((3, M), dtype=torch.float32, device="cuda:0", generator=gen).mul_(6.0).sub_(3.0)
+    f = torch.randn((1, 16, 16, 16), dtype=torch.complex64, device="cuda:0", generator=gen)
+    out = torch.full((1, M), float("nan"), dtype=torch.complex64, device="cuda:0")
+    plan = N.NufftPlan(co, [16] * 3, 2, -1, 1, 1e-15)
+    assert plan.info()[1] == 16
+    plan.execute(out, f)
+    plan.close()
+    some = torch.cat([torch.arange(1000), torch.arange(M - 1000, M), torch.randint(0, M, (3000,))]).to("cuda:0")
+    assert torch.equal(out[:, some], N.nufft(co[:, some].contiguous(), f, [16] * 3, 2, -1, 1e-15))
+    assert not bool(torch.isnan(torch.view_as_real(out)).any())
+
+
 @pytest.mark.parametrize("tol,ns", [(1e-6, 7), (1e-12, 13), (1e-15, 16)])
 def test_type2_bins_do_not_grow_with_the_kernel(N, tol, ns):
     """A type-2 plan's bins are an ordering of its points: 8^3 cells or more each at every

@@ -83,6 +83,10 @@ inline void check_launch(const char* what)
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Most workgroups of `threads` threads in one launch: it holds less than 2^32 threads, and what
+// is more is left out without an error.
+inline int64_t max_blocks(int threads) { return ((int64_t(1) << 32) - 1) / threads; }
+
 // Raise a kernel's dynamic-LDS limit before a launch that needs more than 64 KiB
 // (gfx950 has 160 KiB of LDS per CU).
 template <typename K> inline void allow_lds(K kernel, size_t bytes)

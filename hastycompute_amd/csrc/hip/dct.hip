@@ -312,7 +312,7 @@ void run_axis(float2* data, int64_t batch, const int64_t* D, int ax, float thres
     if (ax == 2) {
         if constexpr (MODE != 2) {
             const int64_t nlines = batch * D[0] * D[1], blocks = ceil_div(nlines, kDctCols);
-            HASTY_REQUIRE(blocks < (1ll << 31), "too many DCT lines for one launch");
+            HASTY_REQUIRE(blocks <= max_blocks(kDctThreads), "too many DCT lines for one launch");
             const size_t smem = sizeof(float) * 2 * kDctCols * line_stride(16 * rt);
             auto kern = pw == 1   ? dct_lines_kernel<1, MODE>
                         : pw == 2 ? dct_lines_kernel<2, MODE>
@@ -327,7 +327,7 @@ void run_axis(float2* data, int64_t batch, const int64_t* D, int ax, float thres
     }
     const int64_t inner = ax == 1 ? D[2] : D[1] * D[2], outer = inner * N;
     const int64_t columns = (ax == 1 ? batch * D[0] : batch) * inner, blocks = ceil_div(columns, kDctCols);
-    HASTY_REQUIRE(blocks < (1ll << 31), "too many DCT lines for one launch");
+    HASTY_REQUIRE(blocks <= max_blocks(kDctThreads), "too many DCT lines for one launch");
     const size_t smem = sizeof(float) * 2 * 16 * rt * kColStride;
     auto kern = pw == 1   ? dct_strided_kernel<1, MODE>
                 : pw == 2 ? dct_strided_kernel<2, MODE>

@@ -883,14 +883,13 @@ template <typename R> void run_axis_fft(const AxisFft<R>& a, hipStream_t stream)
     args.stage_tw = lds_bytes(B, true) <= 160 * 1024 ? 1 : 0;
     const size_t smem = lds_bytes(B, args.stage_tw != 0);
     const int64_t blocks = ceil_div(a.nlines, B);
-    HASTY_REQUIRE(blocks < (1ll << 31), "too many FFT lines for one launch");
     const int mode = a.conv_real ? 1 : (a.conv_cplx ? 2 : 0);
     KernelTimer t("fft_axis", stream);
     if constexpr (std::is_same<R, float>::value) {
         const bool reg = a.L == 128 || a.L == 192 || a.L == 256 || a.L == 320;
         if (g_r16.load() && reg && mode == 0 && !a.inmul && !a.outmul && !a.accumulate) {
             const int64_t rblocks = ceil_div(a.nlines, kR16Lines);
-            HASTY_REQUIRE(rblocks < (1ll << 31), "too many FFT lines for one launch");
+            HASTY_REQUIRE(rblocks <= max_blocks(kR16Lines * 20), "too many FFT lines for one launch");
             switch (a.L / 16) {
             case 8: launch_r16<8>(args, rblocks, stream); break;
             case 12: launch_r16<12>(args, rblocks, stream); break;
@@ -903,10 +902,11 @@ template <typename R> void run_axis_fft(const AxisFft<R>& a, hipStream_t stream)
     }
     if constexpr (std::is_same<R, float>::value) {
         if (g_r16.load() && mode <= 1) {
-            HASTY_REQUIRE(ceil_div(a.nlines, kLinesPer) < (1ll << 31), "too many FFT lines for one launch");
-            if (run_line_fft(args, mode, stream)) return;
+            // more lines than a launch of these holds have fewer workgroups on the LDS kernel
+            if (ceil_div(a.nlines, kLinesPer) <= max_blocks(kLineThreads) && run_line_fft(args, mode, stream)) return;
         }
     }
+    HASTY_REQUIRE(blocks <= max_blocks(kFftThreads), "too many FFT lines for one launch");
     if (mode == 0) {
         allow_lds(axis_fft_kernel<R, 0>, smem);
         hipLaunchKernelGGL((axis_fft_kernel<R, 0>), dim3((unsigned)blocks), dim3(kFftThreads), smem, stream, args);

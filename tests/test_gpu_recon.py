@@ -273,6 +273,16 @@ def test_dct_columns_of_several_slices_vs_scipy(shape):
         assert O.rel_l2(native.l1dct_prox_(xt, axis, lam).cpu().numpy(), want) < 2e-6
 
 
+@pytest.mark.parametrize("shape,axis", [((2**29 + 64, 1, 1, 2), (False, False, True)), ((2**29 + 64, 1, 2, 1), (False, True, False))])
+def test_dct_refuses_more_lines_than_a_launch_holds(shape, axis):
+    """2^24 workgroups of 32 lines are 2^32 threads, which a launch leaves out in silence."""
+    from hastycompute_amd import _capi, native
+
+    x = torch.zeros(shape, dtype=torch.complex64, device="cuda:0")
+    with pytest.raises(_capi.HastyError, match="too many DCT lines"):
+        native.dctn_(x, axis)
+
+
 def test_dct_of_narrow_slices_is_no_slower_than_of_wide_ones():
     """The axis before a trailing one of 1, 2 or 4 against the same lines in wide slices: at
     most 2.5 times the time (1.3 measured; 8 to 20 with a workgroup per slice)."""

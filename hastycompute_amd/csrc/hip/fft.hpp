@@ -51,12 +51,12 @@ template <typename R> void run_axis_fft(const AxisFft<R>& a, hipStream_t stream)
 
 bool fft_size_supported(int L);
 // 1 (default): complex64 passes in registers (the 16 x R four-step kernel for plain passes of
-// length 128, 192, 256 or 320, the two-step lines for others of 48 .. 320); 0: the LDS
-// Stockham kernel.
+// length 128, 192, 256 or 320, the two-step lines for others of 48 .. 320 where they are
+// faster); 0: the LDS Stockham kernel.
 void fft_set_r16(int v);
 int fft_get_r16();
-// Lines per workgroup of a pass whose lines are strided (0 = auto, the same as a pass of
-// contiguous lines).
+// Lines per workgroup of an LDS-kernel pass whose lines are strided (0 = auto, the same as a
+// pass of contiguous lines); the register kernels take 16.
 void fft_set_strided_lines(int v);
 int fft_get_strided_lines();
 // Smallest even 2,3,5-smooth integer >= n.

@@ -641,7 +641,8 @@ __global__ void __launch_bounds__(64 * NW) spread_planes_kernel(SpreadArgs<R> a)
 // needed. A crowded core (the k-space centre of a radial trajectory) is split into parts
 // whose sums are added in a fixed order by a second kernel. The crowded cores' parts are
 // listed first, most crowded first, so the long ones start first. Results do not depend
-// on scheduling.
+// on scheduling, for the points as one setpts has listed them (their order inside a core is
+// that of its counting, so another setpts may round the sums differently).
 constexpr int kGC = 16;
 constexpr int kGatherThreads = 256;
 constexpr int kGatherChunk = 64;  // points staged at once
@@ -1255,9 +1256,9 @@ void dispatch_ns(bool spread, int ns, const SpreadArgs<R>& a, int64_t n, size_t 
     check_launch(spread ? "spread_kernel" : "interp_kernel");
 }
 
-// plans the output-driven spreader (variant 6) serves: complex64 type 1 in 3-D with every
-// fine-grid dim a multiple of the core edge and at least three cores long (so the 27
-// neighbours of a core are distinct cores)
+// plans the output-driven spreader (variant 6) serves: type 1 in 3-D with every fine-grid
+// dim a multiple of the core edge and at least three cores long (so the 27 neighbours of a
+// core are distinct cores)
 bool gather_fits(const NufftPlan* p)
 {
     if (p->type != 1 || p->dim != 3) return false;

@@ -55,7 +55,9 @@ struct NufftPlan {
     int* g_pairs = nullptr;     // point of each pair, grouped by core
     int* g_prel = nullptr;      // window corner relative to the core
     int* g_list = nullptr;      // (core, part) entries, then (core, first part, parts) of the crowded cores
-    void* g_partial = nullptr;  // [g_ncrowded][16^3] sums of the crowded cores' parts (plan precision)
+    // [g_ncrowded][16^3] sums of the crowded cores' parts (plan precision): at most 768 parts,
+    // 25 MB complex64 and 50 MB complex128, held for the plan's life like the point lists
+    void* g_partial = nullptr;
     int64_t g_cap_M = 0;
     int64_t g_cap_pairs = 0;
     int64_t g_cap_list = 0;

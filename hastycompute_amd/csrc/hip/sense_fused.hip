@@ -21,7 +21,8 @@
 //              L-point inverse y FFT (cropped to N1 rows) in LDS, a 32-point inverse
 //              wavefront FFT along m, the coset twiddle exp(+2 pi i s n / L), the
 //              conj(S_c) multiply and the coil sum, all accumulated in registers; the
-//              output plane is written once.
+//              output plane is written once. Where few planes x problems leave the GPU
+//              idle, a workgroup takes one coil and coil_sum adds the images.
 // The kernel K is stored in the same permuted (s, ky, m) order as T.
 #include <atomic>
 #include <vector>
@@ -1431,8 +1432,8 @@ __global__ void __launch_bounds__(256) coil_sum_kernel(FusedArgs a, int plane, i
 // per pair and group, so the fewest groups (a power of two, at most the coils) whose last
 // round over the GPU's `slots` is at least 90 % full (a group re-reads the image plane and
 // loses the prefetch across its border). Together with the split inverse: 32^3 x 8 coils
-// 84 -> 49 us per apply, a 64^3 x 8 CG of 10 iterations 2.38 -> 1.26 ms, 160^3 x 20 coils x
-// 2 problems (320 pairs, 1.25 rounds) 8.06 -> 7.56 ms.
+// 84 -> 49 us per apply, a 64^3 x 8 CG of 10 iterations 2.38 -> 1.26 ms, two 160^3 problems
+// of 20 and 14 coils (320 pairs, 1.25 rounds) 8.06 -> 7.56 ms.
 int coil_groups(int64_t wgs, int coils, int64_t slots)
 {
     int g = 1;
@@ -1467,9 +1468,10 @@ bool inverse_split_pays(int NB, int64_t wgs, int coils)
 // One LDS buffer and two barriers per coil: element (k1, n2) has one place, step B writes
 // its results where it read its inputs, and step A of the next coil writes where step A'
 // of this one read, each thread its own places. With separate buffers for the two
-// transposes a 320-point workgroup took 89 KB, one per CU: 3.20 ms per 160^3 x 20 coils x
-// 2 problems, 2.34 ms here (5.2 TB/s of grid and kernel traffic). 256-point lines are at
-// the rate of a 1:1 stream either way (2.15 and 2.07 ms at 128^3 x 16 coils x 5).
+// transposes a 320-point workgroup took 89 KB, one per CU: 3.20 ms for two 160^3 problems
+// of 20 and 14 coils, 2.34 to 2.42 ms here (9.3 GB of grid and kernel traffic, 3.9 TB/s).
+// 256-point lines are at the rate of a 1:1 stream (5.4 TB/s) either way (2.15 and 2.07 ms at
+// 128^3 x 16 coils x 5).
 template <int R1, int R2, int COLS> struct ZConvShape {
     static constexpr int T = R2 * COLS;                      // threads
     // LDS stride of k1 (float2): columns are contiguous, and below 32 columns the next
@@ -1798,7 +1800,8 @@ namespace {
 // variant, so it is set before kernels are prepared.
 std::atomic<int> g_xy_variant{2};
 std::atomic<int> g_zconv_batch{16};  // problems per register z-convolution launch, 1..16
-// z-convolution bundles at N0 = 128 and 160: 0, 2 (default) 16 columns, 1, 3 8 columns
+// z-convolution bundles at N0 = 128 and 160: 0, 2 (default) 16 columns, 1, 3 8 columns, the
+// slower ones, kept because the option accepts their values
 // (half-used 128-byte lines: 3.6 ms where 16 take 1.66 ms, 128^3 x 16 coils x 4 problems)
 std::atomic<int> g_zconv_variant{2};
 

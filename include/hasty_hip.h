@@ -69,8 +69,9 @@ int hasty_toeplitz_build(const void* coords, int coord_fp64, int64_t M, int ndim
                          const float* weights, void* diag_ref, float* kernel, double tol, void* stream);
 
 /* The same with the build's device memory (grids, point lists) given by the caller:
- * workspace of hasty_toeplitz_workspace_size bytes (0 for invalid arguments), or less (the
- * rest is allocated and freed inside). It is free again when the call returns. */
+ * workspace of hasty_toeplitz_workspace_size bytes (0 for arguments the build refuses), or
+ * less, or none (the rest is allocated and freed inside). It may still be in use by what was
+ * queued on `stream` before, and is free again when the call returns, also with an error. */
 size_t hasty_toeplitz_workspace_size(int64_t M, int ndim, const int64_t* nmodes, double tol);
 int hasty_toeplitz_build_ws(const void* coords, int coord_fp64, int64_t M, int ndim, const int64_t* nmodes,
                             const float* weights, void* diag_ref, float* kernel, double tol, void* workspace,
@@ -163,10 +164,10 @@ int hasty_sense_normal_toeplitz_ex(const void* x, void* out, const void* smaps, 
  *     lengths from 48 to 320 as two register steps with the LDS passes' roundings (long
  *     lines from the number of lines on where that is faster); 0 keeps them on the LDS
  *     Stockham passes.
- *   "fft_strided_lines" 0..64 (default 0 = auto): lines per workgroup of the axis FFT
- *     passes whose lines are strided (the NUFFT's outer axes, the Toeplitz kernel build,
- *     the generic normal operator); auto gives every pass 2048 / L (complex64) or
- *     1024 / L (complex128) lines, 1..64, and strided complex128 passes at least 4.
+ *   "fft_strided_lines" 0..64 (default 0 = auto): lines per workgroup of the LDS kernel's
+ *     axis FFT passes whose lines are strided (the Toeplitz kernel build, lengths without a
+ *     register form); auto gives every pass 2048 / L (complex64) or 1024 / L (complex128)
+ *     lines, 1..64, and strided complex128 passes at least 4. Register passes take 16.
  * Returns 0, or 1 for an unknown name or a value out of range. */
 int hasty_set_option(const char* name, int64_t value);
 /* Current value of an option of hasty_set_option (0, or 1 for an unknown name). */

@@ -739,6 +739,36 @@ def test_type2_bins_do_not_grow_with_the_kernel(N, tol, ns):
 
 
 @pytest.mark.parametrize("dims", [(24, 24, 24), (9, 30, 17), (4, 5, 90)])
+@pytest.mark.parametrize("fp64,tol,lanes", [(True, 1e-1, 2), (True, 1e-3, 4), (False, 1e-15, 16), (True, 1e-15, 16)])
+def test_interpolation_lane_groups_at_the_ends(N, dims, fp64, tol, lanes):
+    """The lane-group sizes of each type that the widths below leave out: the narrowest of
+    complex128, the widest (ns = 16) of both. Bound: as below, and for the float32 weights of
+    ns = 16 their exponents, up to beta = 36.8 with a rounding of 2^-24 in each of the three
+    dims."""
+    ct = torch.complex128 if fp64 else torch.complex64
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(sum(dims) + lanes)
+    M = 1237
+    co = (torch.rand((3, M), dtype=torch.float64, device="cuda:0", generator=gen) * 2 - 1) * np.pi
+    co[0, 200:300] = -np.pi
+    co[2, 250:350] = np.pi - 1e-3
+    co = co.to(torch.float64 if fp64 else torch.float32)
+    f = torch.randn((1, *dims), dtype=ct, device="cuda:0", generator=gen)
+    plan = N.NufftPlan(co, dims, 2, -1, 1, tol)
+    ns = plan.info()[1]
+    used = ns if fp64 else (ns + 2) // 2
+    assert lanes / 2 < used <= lanes or (lanes == 2 and used <= 2)
+    got = torch.empty((1, M), dtype=ct, device="cuda:0")
+    plan.execute(got, f)
+    ax = [torch.arange(n, dtype=torch.float64, device="cuda:0") - n // 2 for n in dims]
+    e = [torch.exp(-1j * ax[d][:, None] * co[d].double()[None, :]) for d in range(3)]
+    v = (f[0].to(torch.complex128).reshape(-1, dims[2]) @ e[2]).reshape(dims[0], dims[1], M)
+    ref = ((v * e[1][None]).sum(1) * e[0]).sum(0)
+    err = float(torch.linalg.vector_norm(got[0] - ref) / torch.linalg.vector_norm(ref))
+    assert err < max(10 * tol, 1e-12 if fp64 else 3e-6 + 3 * 36.8 * 2.0**-24), err
+
+
+@pytest.mark.parametrize("dims", [(24, 24, 24), (9, 30, 17), (4, 5, 90)])
 @pytest.mark.parametrize("fp64,tol", [(False, 1e-1), (False, 1e-2), (False, 1e-3), (False, 1e-5), (False, 1e-6),
                                       (False, 1e-8), (True, 1e-6), (True, 1e-9), (True, 1e-14)])
 def test_interpolation_lane_groups(N, dims, fp64, tol):

@@ -33,6 +33,9 @@ KERNEL_NAMES = {"fwd_xy_kernel": "sense_fwd_xy", "inv_xy_kernel": "sense_inv_xy"
                 "gram_kernel": "llr_gram", "gram_small_kernel": "llr_gram",
                 "eig_w_kernel": "llr_eig", "apply_kernel": "llr_apply"}
 
+# kernels launched within the timed step of another one of the same name
+FOLLOW_UPS = {"sum_parts_kernel"}
+
 
 def short_name(full: str) -> str:
     m = re.search(r"(\w+)(?:<[^()]*>)?\(", full.replace("void ", ""))
@@ -112,13 +115,19 @@ def cmd_traffic(a):
     print("| kernel | dispatches | FETCH_SIZE KiB/launch | WRITE_SIZE KiB/launch | HBM read B/launch | "
           "HBM write B/launch | traffic B/launch |")
     print("|---|---:|---:|---:|---:|---:|---:|")
-    js = {}
-    for k in names:
+    js, moved = {}, {}  # moved: name -> [launches of the step, read bytes, written bytes]
+    for k in sorted(names, key=lambda k: k in FOLLOW_UPS):
         f = sum(fetch[k]) / len(fetch[k])
         w = sum(write[k]) / len(write[k])
         rb, wb = f * 1024 / fr, w * 1024 / fw
         print(f"| {k} | {len(fetch[k])} | {f:.1f} | {w:.1f} | {rb:.4g} | {wb:.4g} | {rb + wb:.4g} |")
-        ent = {"kernel_symbol": k, "hbm_read_bytes_per_launch": rb, "hbm_write_bytes_per_launch": wb,
+        m = moved.setdefault(KERNEL_NAMES[k], [0, 0.0, 0.0])
+        m[0] += 0 if k in FOLLOW_UPS else len(fetch[k])
+        m[1] += rb * len(fetch[k])
+        m[2] += wb * len(fetch[k])
+        rb, wb = m[1] / max(m[0], 1), m[2] / max(m[0], 1)
+        ent = {"kernel_symbol": js.get(KERNEL_NAMES[k] + a.key_suffix, {}).get("kernel_symbol", k),
+               "hbm_read_bytes_per_launch": rb, "hbm_write_bytes_per_launch": wb,
                "hbm_bytes_per_launch": rb + wb, "fetch_factor": fr, "write_factor": fw,
                "source_sha256": source_sha256(k)}
         if a.units_per_launch:

@@ -87,6 +87,32 @@ def test_library_allocations_get_what_torch_caches(monkeypatch, name, codes, ret
     assert not left and emptied == ([1] if retried else [])
 
 
+def test_traffic_counts_every_kernel_of_a_step(tmp_path):
+    """The spreader and the sums of its parts are one timed step: its bytes are both kernels',
+    per spreading launch; kernels that serve a step in turn are averaged over its launches."""
+    import json
+
+    from hastycompute_amd import profiling
+
+    def table(name, rows):
+        p = tmp_path / name
+        p.write_text("Kernel_Name,Counter_Value\n" + "".join(f'"void hasty_hip::{k}(Args)",{v}\n' for k, v in rows))
+        return str(p)
+
+    rows = [("sum_parts_kernel<float>", 10), ("gather_spread_kernel<float>", 100), ("sum_parts_kernel<float>", 30),
+            ("gather_spread_kernel<float>", 120), ("axis_fft_r16_kernel<16, 1>", 6), ("line_fft_kernel<A, B, 0, 1>", 2)]
+    copy = [("copy_kernel", 1024)]
+    out = tmp_path / "t.json"
+    profiling.main(["traffic", "--fetch", table("f", rows), "--write", table("w", [(k, 2 * v) for k, v in rows]),
+                    "--copy-fetch", table("cf", copy), "--copy-write", table("cw", copy), "--copy-bytes", str(1 << 20),
+                    "--json", str(out), "--key-suffix", "@t"])
+    js = json.loads(out.read_text())
+    assert js["nufft_spread@t"]["hbm_read_bytes_per_launch"] == pytest.approx(1024 * (220 + 40) / 2)
+    assert js["nufft_spread@t"]["hbm_write_bytes_per_launch"] == pytest.approx(2048 * (220 + 40) / 2)
+    assert js["nufft_spread@t"]["kernel_symbol"] == "gather_spread_kernel"
+    assert js["fft_axis@t"]["hbm_bytes_per_launch"] == pytest.approx(3 * 1024 * (6 + 2) / 2)
+
+
 def test_llr_shifts_host():
     """hasty_llr_shifts is host code: it must reproduce the oracle's restatement."""
     from oracle import oracle as O

@@ -268,12 +268,15 @@ def test_toeplitz_build_without_torch_memory():
     total = torch.cuda.get_device_properties(0).total_memory
     # room for the images, kernels and the operator's grids (some 100 MB), not for 500 MB more
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2**28) / total)
+    held = []
     try:
         with pytest.raises(torch.OutOfMemoryError):
-            torch.empty(2**29 - 2**26, dtype=torch.uint8, device="cuda:0")
+            while len(held) < 64:  # blocks of that size that other tests left inside reserved memory
+                held.append(torch.empty(2**29 - 2**26, dtype=torch.uint8, device="cuda:0"))
         k2, out2 = both()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+        del held
     assert torch.equal(k, k2) and torch.equal(out, out2)
 
 
